@@ -14,7 +14,7 @@ OBJ = os.path.join(HERE, "_build")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-SOURCES = ["kernels.hip", "gemm_lowp.hip", "weights.hip", "backproject.hip", "fourier_map.hip", "reconstruct.hip", "imageprep.hip",
+SOURCES = ["kernels.hip", "gemm_lowp.hip", "weights.hip", "backproject.hip", "fourier_map.hip", "reconstruct.hip", "gridding.hip", "imageprep.hip",
            "proposal.hip", "noalloc.hip",
            "engine.cpp", "sampling.cpp", "mstep.cpp"]
 FLAGS = [

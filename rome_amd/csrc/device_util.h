@@ -137,6 +137,26 @@ DEV double wave_min(double v) {
     return v;
 }
 
+// a0[key] += v, a1[key] += 1 (LDS) for the wave's lanes with key >= 0; equal keys sit in neighbouring lanes and
+// are added up by shuffles first.  Called by all lanes.
+DEV void shell_add(int key, double v, double* a0, double* a1) {
+    const int lane = threadIdx.x & 63;
+    double c = 1.;
+    for (int o = 1; o < 64; o <<= 1) {
+        const double vn = __shfl_down(v, o, 64), cn = __shfl_down(c, o, 64);
+        const int kn = __shfl_down(key, o, 64);
+        if (lane + o < 64 && kn == key) {
+            v += vn;
+            c += cn;
+        }
+    }
+    const int kp = __shfl_up(key, 1, 64);
+    if (key >= 0 && (lane == 0 || kp != key)) {
+        atomicAdd(&a0[key], v);
+        atomicAdd(&a1[key], c);
+    }
+}
+
 // block-wide reduction over blockDim.x threads (multiple of 64), result broadcast
 template <typename T, typename Op>
 DEV T block_reduce(T v, Op op, T* scratch) {

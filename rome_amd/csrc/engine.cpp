@@ -276,6 +276,8 @@ struct rome_ctx {
     DevBuf<double2> rc_data, rc_Fc, rc_Ft;
     DevBuf<double> rc_weight, rc_Fw, rc_Fnw, rc_M, rc_Mout, rc_vol, rc_tab, rc_sums, rc_tau2;
     DevBuf<int> rc_bad;
+    DevBuf<double> dft_cos, dft_sin;  // of the gridding iterations, for dft_P points
+    int dft_P = 0;
     std::vector<double> rc_tab_h;
     // stage timing with HIP events on the engine stream (rome_set_profiling)
     static constexpr int kStages = 13;
@@ -2506,7 +2508,7 @@ int rome_healpix_pix2ang(int order, int pix, double* z, double* phi) {
 }  // extern "C"
 
 int rome_update_model(rome_ctx* ctx, int install, rome_model* out) {
-    if (ctx) ++ctx->state_epoch;  // kernels of captured pools read what this call changes
+    if (ctx && install) ++ctx->state_epoch;  // kernels of captured pools read what an installed model changes
     if (!ctx) return ROME_ERR_ARG;
     if (!ctx->configured || !ctx->have_model) return fail(ctx, ROME_ERR_ARG, "no configured model to update");
     const rome_config& c = ctx->cfg;
@@ -2643,6 +2645,34 @@ static std::vector<double> kaiser_ft_table(double a, double alpha, int nr_elem, 
     return t;
 }
 
+// cos and sin of 2 pi i k / P, 0 <= i, k < H = (P + 1) / 2, in the operand order of the gridding iterations'
+// products (row tile, k step, lane: i = 16 t + lane % 16, k = 4 kk + lane / 16; cos halved at k = 0), kept until P changes
+static int dft_tables(rome_ctx* ctx, int P) {
+    if (ctx->dft_P == P) return ROME_OK;
+    const int H = (P + 1) / 2, nt = (H + 15) / 16, nk = 4 * nt;
+    std::vector<double> c1(P), s1(P), c((size_t)nt * nk * 64, 0.), sn(c.size(), 0.);
+    for (int m = 0; m < P; ++m) {
+        const long double w = 2.0L * 3.14159265358979323846264338327950288L * m / P;
+        c1[m] = (double)cosl(w);
+        s1[m] = (double)sinl(w);
+    }
+    for (int t = 0; t < nt; ++t)
+        for (int kk = 0; kk < nk; ++kk)
+            for (int l = 0; l < 64; ++l) {
+                const int i = 16 * t + l % 16, k = 4 * kk + l / 16;
+                if (i >= H || k >= H) continue;
+                const int m = (int)((long long)i * k % P);
+                c[((size_t)t * nk + kk) * 64 + l] = k ? c1[m] : 0.5;
+                sn[((size_t)t * nk + kk) * 64 + l] = s1[m];
+            }
+    ctx->dft_P = 0;
+    HIPCHK(ctx->dft_cos.upload(c.data(), c.size(), ctx->stream));
+    HIPCHK(ctx->dft_sin.upload(sn.data(), sn.size(), ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    ctx->dft_P = P;
+    return ROME_OK;
+}
+
 int rome_reconstruct(rome_ctx* ctx, int iclass, const rome_recon_params* prm, const double* data_in,
                      const double* weight_in, double* tau2, const double* fsc, double* sigma2,
                      double* data_vs_prior, double* vol_out) {
@@ -2661,19 +2691,22 @@ int rome_reconstruct(rome_ctx* ctx, int iclass, const rome_recon_params* prm, co
     const size_t ng = (size_t)Dz * P * PF, nM = (size_t)Dz * P * P, nFt = (size_t)NZ * N * NF;
     const size_t nMo = (size_t)NZ * N * N, nv = (size_t)OZ * ori * ori;
     const double osc = ctx->is3d ? (double)(pf * pf * pf) : (double)(pf * pf);
-    hipfftHandle planPi, planPf, planNi;
-    int rc = fft_plan(ctx, HIPFFT_Z2D, rank, P, &planPi);
-    if (!rc) rc = fft_plan(ctx, HIPFFT_D2Z, rank, P, &planPf);
-    if (!rc) rc = fft_plan(ctx, HIPFFT_Z2D, rank, N, &planNi);
+    hipfftHandle planNi;
+    int rc = fft_plan(ctx, HIPFFT_Z2D, rank, N, &planNi);
+    if (!rc) rc = dft_tables(ctx, P);
     if (rc) return rc;
+    // the blob table has ended at the grid's last plane: blob(-n) = blob(n) everywhere
+    const double sampling = 0.5 / 10000.;
+    const bool sym = (int)(std::fabs(std::sqrt((double)(P / 2) * (P / 2)) / (double)(ori * pf)) / sampling) >= 10000;
+    const int ldx = (PF + 15) / 16 * 16;
+    const size_t nT = (size_t)(sym ? PF : P) * (ctx->is3d ? P : 1) * ldx;  // of the gridding iterations
     HIPCHK(ctx->rc_data.reserve(ng));
     HIPCHK(ctx->rc_weight.reserve(ng));
     HIPCHK(ctx->rc_Fw.reserve(ng));
     HIPCHK(ctx->rc_Fnw.reserve(ng));
-    // rc_Fc and rc_M also take the transform of the output map (tau2 from the FSC)
-    HIPCHK(ctx->rc_Fc.reserve(std::max(ng, (size_t)OZ * ori * (ori / 2 + 1))));
-    HIPCHK(ctx->rc_M.reserve(std::max(nM, nv)));
-    HIPCHK(ctx->rc_Ft.reserve(nFt));
+    // rc_Fc and rc_Ft hold the gridding iterations' lines; rc_Fc also the output map's transform (tau2 from the FSC)
+    HIPCHK(ctx->rc_Fc.reserve(std::max({ng, nT, (size_t)OZ * ori * (ori / 2 + 1)})));
+    HIPCHK(ctx->rc_Ft.reserve(std::max(nFt, nT)));
     HIPCHK(ctx->rc_Mout.reserve(nMo));
     HIPCHK(ctx->rc_vol.reserve(nv));
     HIPCHK(ctx->rc_sums.reserve(4 * (size_t)std::max(oriF, ori)));
@@ -2737,18 +2770,30 @@ int rome_reconstruct(rome_ctx* ctx, int iclass, const rome_recon_params* prm, co
         ctx->rc_tab_h = kaiser_ft_table(1.9 * pf, 15.0, 10000, &sampling);
         HIPCHK(ctx->rc_tab.upload(ctx->rc_tab_h.data(), ctx->rc_tab_h.size(), s));
     }
-    const double sampling = 0.5 / 10000.;
     HIPCHK(rc_newweight_init(s, ctx->rc_Fnw.p, Dz, P, PF, max_r2));
     auto Z = [](double2* p) { return reinterpret_cast<hipfftDoubleComplex*>(p); };
-    for (int it = 0; it < prm->max_iter_preweight; ++it) {
-        HIPCHK(rc_fconv(s, ctx->rc_Fnw.p, ctx->rc_Fw.p, ctx->rc_Fc.p, ng));
-        if (hipfftExecZ2D(planPi, Z(ctx->rc_Fc.p), ctx->rc_M.p) != HIPFFT_SUCCESS)
-            return fail(ctx, ROME_ERR_HIP, "hipfftExecZ2D failed");
-        HIPCHK(rc_blob(s, ctx->rc_M.p, Dz, P, ori, pf, ctx->rc_tab.p, 10000, sampling, ctx->rc_tab_h[0]));
-        if (hipfftExecD2Z(planPf, ctx->rc_M.p, Z(ctx->rc_Fc.p)) != HIPFFT_SUCCESS)
-            return fail(ctx, ROME_ERR_HIP, "hipfftExecD2Z failed");
-        HIPCHK(rc_newweight(s, ctx->rc_Fc.p, ctx->rc_Fnw.p, Dz, P, PF, max_r2, (double)nM));
-    }
+    GriddingArgs ga{};
+    ga.P = P;
+    ga.H = PF;
+    ga.Py = ctx->is3d ? P : 1;
+    ga.ldx = ldx;
+    ga.nt = (PF + 15) / 16;
+    ga.nk = 4 * ga.nt;
+    ga.max_r2 = max_r2;
+    ga.xlim = pf * r_max - 1;
+    ga.Cf = ctx->dft_cos.p;
+    ga.Sf = ctx->dft_sin.p;
+    ga.Fw = ctx->rc_Fw.p;
+    ga.Fnw = ctx->rc_Fnw.p;
+    ga.T0 = ctx->rc_Fc.p;
+    ga.T1 = ctx->rc_Ft.p;
+    ga.tab = ctx->rc_tab.p;
+    ga.ntab = 10000;
+    ga.npad = ori * pf;
+    ga.sampling = sampling;
+    ga.tab0 = ctx->rc_tab_h[0];
+    ga.size = (double)nM;
+    HIPCHK(gridding_iterations(s, ga, sym, prm->max_iter_preweight));
     // weighted data -> window to 2 ori -> real space -> window to ori, soft mask, gridding correction
     HIPCHK(rc_final_fconv(s, ctx->rc_data.p, ctx->rc_Fnw.p, ctx->rc_Fc.p, Dz, P, PF, max_r2));
     HIPCHK(rc_window_ft(s, ctx->rc_Fc.p, ctx->rc_Ft.p, Dz, P, PF, NZ, N, NF));
@@ -2764,6 +2809,7 @@ int rome_reconstruct(rome_ctx* ctx, int iclass, const rome_recon_params* prm, co
         rc = fft_plan(ctx, HIPFFT_D2Z, rank, ori, &planO);
         if (rc) return rc;
         // the transform input must stay intact (it is the output map): transform a copy
+        HIPCHK(ctx->rc_M.reserve(nv));
         HIPCHK(hipMemcpyAsync(ctx->rc_M.p, ctx->rc_vol.p, nv * sizeof(double), hipMemcpyDeviceToDevice, s));
         if (hipfftExecD2Z(planO, ctx->rc_M.p, Z(ctx->rc_Fc.p)) != HIPFFT_SUCCESS)
             return fail(ctx, ROME_ERR_HIP, "hipfftExecD2Z failed");

@@ -517,11 +517,20 @@ hipError_t rc_map(hipStream_t s, double* Fw, int Dz, int P, int PF, int max_r2, 
                   const double* tau2, int minres, int oriF, double* dvp, double* cnt, int* bad);
 hipError_t rc_normalise(hipStream_t s, double* Fw, double2* data, size_t n, double norm);
 hipError_t rc_newweight_init(hipStream_t s, double* Fnw, int Dz, int P, int PF, int max_r2);
-hipError_t rc_fconv(hipStream_t s, const double* Fnw, const double* Fw, double2* Fc, size_t n);
-hipError_t rc_blob(hipStream_t s, double* M, int Dz, int P, int ori, int pf, const double* tab, int ntab,
-                   double sampling, double norm);
-hipError_t rc_newweight(hipStream_t s, const double2* Fc, double* Fnw, int Dz, int P, int PF, int max_r2,
-                        double size3);
+// Gridding-weight iterations (gridding.hip).  Grids real [Dz][Py][H] in FFT order (Dz = P; 2D: the image's
+// rows are the z axis and Py = 1), H = (P + 1) / 2; T0, T1 complex [H, or P without SYM][Py][ldx].
+struct GriddingArgs {
+    int P, H, Py, ldx, nt, nk;  // nt = ceil(H / 16) row tiles, nk = 4 nt k steps of 4
+    int max_r2, xlim;           // xlim: largest x with x^2 < max_r2
+    const double *Cf, *Sf;      // cos (halved at k = 0) / sin of 2 pi i k / P as operands [nt][nk][64], zero past H
+    const double* Fw;
+    double* Fnw;
+    double2 *T0, *T1;
+    const double* tab;          // blob transform, ntab samples `sampling` apart in units of 1 / npad
+    int ntab, npad;
+    double sampling, tab0, size;
+};
+hipError_t gridding_iterations(hipStream_t s, const GriddingArgs& a, bool sym, int iters);
 hipError_t rc_final_fconv(hipStream_t s, const double2* data, const double* Fnw, double2* Fc, int Dz, int P, int PF,
                           int max_r2);
 hipError_t rc_window_ft(hipStream_t s, const double2* Fc, double2* Ft, int Dz, int P, int PF, int NZ, int N, int NF);
