@@ -260,6 +260,12 @@ struct rome_ctx {
     DevBuf<double> slice_w;
     DevBuf<unsigned> bp_count, bp_off, bp_coff, bp_cursor;
     DevBuf<unsigned long long> bp_rec;
+    // whole images at given poses (rome_backproject_images), at most 1024 at a time
+    DevBuf<double> bi_in, bi_one, bi_acc;
+    DevBuf<float2> bi_val;
+    DevBuf<float> bi_wgt;
+    DevBuf<int> bi_task;
+    DevBuf<unsigned long long> bi_rec;
     // hipFFT plans by (type, rank, size), kept for the context's lifetime
     struct FftPlan {
         int type, rank, n, batch;
@@ -3313,42 +3319,107 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
     if (n == 0) return ROME_OK;
     HIPCHK(hipSetDevice(ctx->device));
     hipStream_t s = ctx->stream;
-    const int F2 = ctx->F2f, Pf = ctx->Pf;
-    const int chunk = 2048;
-    DevBuf<float2> X, S;
-    DevBuf<float> C;
-    DevBuf<double> Ai, sx, sy;
-    std::vector<float2> hx((size_t)std::min(n, chunk) * F2);
-    std::vector<float> hc((size_t)std::min(n, chunk) * F2);
-    std::vector<double> ha(6 * (size_t)std::min(n, chunk)), hsx(std::min(n, chunk)), hsy(std::min(n, chunk));
+    const int F2 = ctx->F2f, Pf = ctx->Pf, chunk = std::min(n, 1024);
+    const bool use_ctf = fctf && ctx->cfg.do_ctf_correction;
+    const size_t gn = ctx->grid_n;
+    // FP64 as the caller holds them: re, im, CTF, then matrices and offsets (8 per image)
+    const size_t per = (size_t)F2 * (use_ctf ? 3 : 2);
+    HIPCHK(ctx->bi_in.reserve(chunk * (per + 8)));
+    std::vector<double> hs(8 * (size_t)chunk);
+    BpImageArgs ia{};
+    ia.F2 = F2;
+    ia.Pf = Pf;
+    ia.ori = ctx->cfg.ori_size;
+    ia.f_nfine = ctx->f_nfine.p;
+    ia.f_xy = ctx->f_xy.p;
+    ia.sintab = ctx->sintab.p;
+    ia.costab = ctx->costab.p;
+    ia.pad = ctx->pad;
+    ia.padF = ctx->padF;
+    ia.c = ctx->cgrid;
+    ia.r_max = ctx->r_max;
+    float *gd = ctx->bp_data.p + 2 * gn * iclass, *gw = ctx->bp_weight.p + gn * iclass;
+    BpArgs ba{};
+    if (ctx->is3d) {
+        HIPCHK(ctx->bi_val.reserve((size_t)chunk * Pf));
+        HIPCHK(ctx->bi_wgt.reserve((size_t)chunk * Pf));
+        HIPCHK(ctx->bi_rec.reserve((size_t)chunk * Pf));
+        HIPCHK(ctx->bi_task.reserve(2 * (size_t)chunk));
+        HIPCHK(ctx->bi_one.reserve(chunk));
+        ba.K = 1;
+        ba.Pf = Pf;
+        ba.NOR = 1;
+        ba.R = chunk;  // slice = image: its "rotation" is its own index
+        ba.pad = ctx->pad;
+        ba.padF = ctx->padF;
+        ba.c = ctx->cgrid;
+        ba.r_max = ctx->r_max;
+        ba.grid_stride = gn;
+        ba.nbx = (ctx->padF + 7) / 8;
+        ba.nby = ba.nbz = (ctx->pad + 7) / 8;
+        ba.nb_class = ba.nbx * ba.nby * ba.nbz;
+        HIPCHK(ctx->bp_count.reserve(ba.nb_class));
+        HIPCHK(ctx->bp_off.reserve(ba.nb_class + 1));
+        HIPCHK(ctx->bp_coff.reserve(ba.nb_class + 1));
+        HIPCHK(ctx->bp_cursor.reserve(ba.nb_class));
+        ia.val = ctx->bi_val.p;
+        ia.wgt = ctx->bi_wgt.p;
+        ia.task_img = ctx->bi_task.p;
+        ia.task_m = ctx->bi_task.p + chunk;
+        ia.slice_w = ctx->bi_one.p;
+        ba.task_img = ia.task_img;
+        ba.task_m = ia.task_m;
+        ba.f_xy = ctx->f_xy.p;
+        ba.MC2bp = ctx->bi_wgt.p;
+        ba.slice_w = ctx->bi_one.p;
+        ba.slice_val = ctx->bi_val.p;
+        ba.count = ctx->bp_count.p;
+        ba.off = ctx->bp_off.p;
+        ba.coff = ctx->bp_coff.p;
+        ba.cursor = ctx->bp_cursor.p;
+        ba.rec = ctx->bi_rec.p;
+        ba.bp_data = gd;
+        ba.bp_weight = gw;
+    } else {
+        HIPCHK(ctx->bi_acc.reserve(3 * gn * kBpCopies));
+        HIPCHK(launch_fill32(s, ctx->bi_acc.p, 0u, 2 * 3 * gn * kBpCopies));
+        ia.acc = ctx->bi_acc.p;
+    }
     for (int i0 = 0; i0 < n; i0 += chunk) {
         const int m = std::min(chunk, n - i0);
-        for (size_t q = 0; q < (size_t)m * F2; ++q) {
-            hx[q] = make_float2((float)fre[(size_t)i0 * F2 + q], (float)fim[(size_t)i0 * F2 + q]);
-            hc[q] = fctf && ctx->cfg.do_ctf_correction ? (float)fctf[(size_t)i0 * F2 + q] : 1.f;
-        }
+        const size_t px = (size_t)m * F2, o = (size_t)i0 * F2;
+        double* d = ctx->bi_in.p;
+        HIPCHK(hipMemcpyAsync(d, fre + o, px * sizeof(double), hipMemcpyHostToDevice, s));
+        HIPCHK(hipMemcpyAsync(d + px, fim + o, px * sizeof(double), hipMemcpyHostToDevice, s));
+        if (use_ctf) HIPCHK(hipMemcpyAsync(d + 2 * px, fctf + o, px * sizeof(double), hipMemcpyHostToDevice, s));
         for (int i = 0; i < m; ++i) {
             double A[9];
             const double* e = euler + 3 * (size_t)(i0 + i);
             if (ctx->is3d) euler_matrix(e[0], e[1], e[2], A);
             else euler_matrix(0, 0, e[2], A);
-            rot6(A, &ha[6 * (size_t)i]);
-            hsx[i] = shift[2 * (size_t)(i0 + i)];
-            hsy[i] = shift[2 * (size_t)(i0 + i) + 1];
+            rot6(A, &hs[6 * (size_t)i]);
+            hs[6 * (size_t)m + i] = shift[2 * (size_t)(i0 + i)];
+            hs[7 * (size_t)m + i] = shift[2 * (size_t)(i0 + i) + 1];
         }
-        HIPCHK(X.upload(hx.data(), (size_t)m * F2, s));
-        HIPCHK(C.upload(hc.data(), (size_t)m * F2, s));
-        HIPCHK(Ai.upload(ha.data(), 6 * (size_t)m, s));
-        HIPCHK(sx.upload(hsx.data(), m, s));
-        HIPCHK(sy.upload(hsy.data(), m, s));
-        HIPCHK(S.reserve((size_t)m * Pf));
-        HIPCHK(launch_phase_table(s, sx.p, sy.p, m, ctx->f_xy.p, Pf, ctx->cfg.ori_size, ctx->sintab.p, ctx->costab.p,
-                                  S.p));
-        BpImageArgs ba{X.p,     C.p,       S.p,     Ai.p,       F2,        Pf,      ctx->f_nfine.p,
-                       ctx->f_xy.p, ctx->is3d, ctx->pad, ctx->padF, ctx->cgrid, ctx->r_max,
-                       ctx->bp_data.p + 2 * ctx->grid_n * iclass, ctx->bp_weight.p + ctx->grid_n * iclass};
-        HIPCHK(launch_bp_images(s, m, ba));
-        HIPCHK(hipStreamSynchronize(s));  // the host staging is reused by the next chunk
+        double* dm = d + m * per;
+        HIPCHK(hipMemcpyAsync(dm, hs.data(), 8 * (size_t)m * sizeof(double), hipMemcpyHostToDevice, s));
+        ia.fre = d;
+        ia.fim = d + px;
+        ia.ctf = use_ctf ? d + 2 * px : nullptr;
+        ia.Ai = ba.Ai_fine = dm;
+        ia.sx = dm + 6 * (size_t)m;
+        ia.sy = dm + 7 * (size_t)m;
+        if (ctx->is3d) {
+            HIPCHK(launch_bp_image_values(s, m, ia));
+            HIPCHK(launch_backproject_binned(s, m, ba));
+        } else {
+            HIPCHK(launch_bp_images2d(s, m, ia));
+        }
+        HIPCHK(hipStreamSynchronize(s));  // the staging buffers are reused by the next chunk
+    }
+    if (!ctx->is3d) {
+        HIPCHK(launch_bp_add2d(s, ctx->bi_acc.p, gn, gd, gw));
+        HIPCHK(hipStreamSynchronize(s));
     }
     return ROME_OK;
 }

@@ -490,20 +490,29 @@ struct MetaArgs {
     int* argmax;               // [n][6]
 };
 hipError_t launch_meta(hipStream_t s, const MetaArgs& a);
-// Whole images scattered into one class grid at their own poses (the offline reconstruction).
+// Whole images at their own poses into one class grid (the offline reconstruction): the pixel values and
+// weights as slices for the binned scatter (3D), or scattered (2D).
 struct BpImageArgs {
-    const float2* X;      // [n][F2] transforms (current_size half-plane)
-    const float* ctf;     // [n][F2]
-    const float2* phase;  // [n][Pf] tabulated shift phase of each image's offset
-    const double* Ai;     // [n][6] 2 A^T restricted to (x, y)
-    int F2, Pf;
+    const double *fre, *fim;  // [n][F2] transforms (current_size half-plane)
+    const double* ctf;        // [n][F2], or null: ones
+    const double *sx, *sy;    // [n] offsets (pixels)
+    const double* Ai;         // [n][6] 2 A^T restricted to (x, y)
+    int F2, Pf, ori;
     const int* f_nfine;
     const int* f_xy;
-    int is3d, pad, padF, c, r_max;
-    float* bp_data;       // the class's grid [pad][pad][padF] float2 (interleaved)
-    float* bp_weight;
+    const double *sintab, *costab;
+    int pad, padF, c, r_max;
+    float2* val;              // [n][Pf] shifted transform times the CTF
+    float* wgt;               // [n][Pf] CTF^2
+    int *task_img, *task_m;   // [n] 0, 1, ..: every image its own slice (binned scatter)
+    double* slice_w;          // [n] 1
+    double* acc;              // 2D: [kBpCopies][3][pad * padF] sums (re, im, weight), zero at the start
 };
-hipError_t launch_bp_images(hipStream_t s, int n, const BpImageArgs& a);
+constexpr int kBpCopies = 8;
+hipError_t launch_bp_image_values(hipStream_t s, int n, const BpImageArgs& a);
+hipError_t launch_bp_images2d(hipStream_t s, int n, const BpImageArgs& a);
+// 2D sums added to the class grid (n = pad * padF elements)
+hipError_t launch_bp_add2d(hipStream_t s, const double* acc, size_t n, float* bp_data, float* bp_weight);
 hipError_t launch_store_sums(hipStream_t s, const StoreArgs& a);
 // With a.ntask_dev (device-driven pools) S is read on the device and persist_blocks blocks stride over
 // the slices (one pixel block per grid row) and over the brick chunks.

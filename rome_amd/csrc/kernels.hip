@@ -24,29 +24,29 @@ namespace rome {
 // ------------------------------------------------------------------ phase tables
 // Tabulated shift phase of shiftImageInFourierTransform (src/image.h:1478-1574):
 // index = (int)(|2 pi (x xs + y ys)| / (2 pi / 5000)) % 5000, xs = shift_x / (-ori).
+DEV float2 tab_phase(double sx, double sy, int xy, int ori, const double* __restrict__ sintab,
+                     const double* __restrict__ costab) {
+#pragma clang fp contract(off)
+    const double xs = __ddiv_rn(sx, (double)(-ori));
+    const double ys = __ddiv_rn(sy, (double)(-ori));
+    if (fabs(xs) < 1e-6 && fabs(ys) < 1e-6) return make_float2(1.f, 0.f);
+    const double twopi = 2.0 * 3.14159265358979323846;
+    const double sampling = twopi / 5000.0;
+    const double x = (double)px_x(xy), y = (double)px_y(xy);
+    const double dotp = dmul(twopi, dadd(dmul(x, xs), dmul(y, ys)));
+    const int it = ((int)__ddiv_rn(fabs(dotp), sampling)) % 5000;
+    double a = costab[it], b = sintab[it];
+    if (dotp < 0) b = -b;
+    return make_float2((float)a, (float)b);
+}
+
 __global__ void k_phase_table(const double* __restrict__ sx, const double* __restrict__ sy, int nshift,
                               const int* __restrict__ xy, int P, int ori, const double* __restrict__ sintab,
                               const double* __restrict__ costab, float2* __restrict__ out) {
-#pragma clang fp contract(off)
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (size_t)nshift * P) return;
     const int s = (int)(idx / P), p = (int)(idx % P);
-    const double xs = __ddiv_rn(sx[s], (double)(-ori));
-    const double ys = __ddiv_rn(sy[s], (double)(-ori));
-    float2 r;
-    if (fabs(xs) < 1e-6 && fabs(ys) < 1e-6) {
-        r = make_float2(1.f, 0.f);
-    } else {
-        const double twopi = 2.0 * 3.14159265358979323846;
-        const double sampling = twopi / 5000.0;
-        const double x = (double)px_x(xy[p]), y = (double)px_y(xy[p]);
-        const double dotp = dmul(twopi, dadd(dmul(x, xs), dmul(y, ys)));
-        const int it = ((int)__ddiv_rn(fabs(dotp), sampling)) % 5000;
-        double a = costab[it], b = sintab[it];
-        if (dotp < 0) b = -b;
-        r = make_float2((float)a, (float)b);
-    }
-    out[idx] = r;
+    out[idx] = tab_phase(sx[s], sy[s], xy[p], ori, sintab, costab);
 }
 
 // ------------------------------------------------------------------ projections
@@ -1343,53 +1343,74 @@ __global__ void k_meta(MetaArgs a) {
 }
 
 // ------------------------------------------------------------------ backprojection of whole images
-// MyBackProjector::backproject of one image per block at its own pose (apps/rome_reconstruct.cpp:104-330):
-// the transform X (current_size half-plane) shifted by the image's tabulated phase, times the CTF, and the
-// weight CTF^2, scattered trilinearly (bilinearly in 2D) into one class grid; the pixel set is the fine
-// one (x = 0 column for y >= 0 only, as the reference's first_x rule), radius r_max.
-__global__ __launch_bounds__(256) void k_bp_images(BpImageArgs a) {
+// MyBackProjector::backproject of images at their own poses (apps/rome_reconstruct.cpp:104-330): the transform
+// (current_size half-plane) shifted by the image's tabulated phase, times the CTF, and the weight CTF^2; the
+// pixel set is the fine one (x = 0 column for y >= 0 only, as the reference's first_x rule), radius r_max.
+// 3D: these values are the slices of the binned scatter (backproject.hip), one slice per image; a direct
+// scatter's 24 float atomics a pixel took 1.82 ms for 400 images of 100^2, this pass and the binned one 0.2.
+DEV void bp_image_value(const BpImageArgs& a, int img, int p, float2& v, float& w) {
+    const size_t nf = (size_t)img * a.F2 + a.f_nfine[p];
+    const float cv = a.ctf ? (float)a.ctf[nf] : 1.f;
+    const float2 t = cmul(make_float2((float)a.fre[nf], (float)a.fim[nf]),
+                          tab_phase(a.sx[img], a.sy[img], a.f_xy[p], a.ori, a.sintab, a.costab));
+    v = make_float2(t.x * cv, t.y * cv);
+    w = cv * cv;
+}
+
+__global__ __launch_bounds__(256) void k_bp_image_values(BpImageArgs a) {
+    const int img = blockIdx.y, p = blockIdx.x * 256 + threadIdx.x;
+    if (p == 0) {
+        a.task_img[img] = a.task_m[img] = img;
+        a.slice_w[img] = 1.;
+    }
+    if (p >= a.Pf) return;
+    float2 v;
+    float w;
+    bp_image_value(a, img, p, v, w);
+    a.val[(size_t)img * a.Pf + p] = v;
+    a.wgt[(size_t)img * a.Pf + p] = w;
+}
+
+// 2D: direct scatter into FP64 sums, a copy per XCD (blocks reach the XCDs round-robin) so that the images'
+// few thousand shared grid points are contended an eighth as much; the sums do not depend on the order to
+// FP32 rounding.
+__global__ __launch_bounds__(256) void k_bp_images2d(BpImageArgs a) {
     const int img = blockIdx.x;
-    const float2* X = a.X + (size_t)img * a.F2;
-    const float* ctf = a.ctf + (size_t)img * a.F2;
-    const float2* S = a.phase + (size_t)img * a.Pf;
-    const double* A6 = a.Ai + 6 * (size_t)img;
-    float* gd = a.bp_data;
-    float* gw = a.bp_weight;
+    const size_t gn = (size_t)a.pad * a.padF;
+    double* acc = a.acc + 3 * gn * (blockIdx.x % kBpCopies);
     for (int p = threadIdx.x; p < a.Pf; p += blockDim.x) {
         const int xy = a.f_xy[p];
         const int x = px_x(xy), y = px_y(xy);
         if (x * x + y * y > a.r_max * a.r_max) continue;
-        const int nf = a.f_nfine[p];
-        const float cv = ctf[nf];
-        const float wgt = cv * cv;
+        float2 v;
+        float wgt;
+        bp_image_value(a, img, p, v, wgt);
         if (!(wgt > 0.f)) continue;
-        const float2 v = cmul(X[nf], S[p]);
-        const Coords c = map_coords(A6, x, y, a.c, a.is3d != 0);
-        const float vr = v.x * cv, vi = (c.neg ? -v.y : v.y) * cv;
-        const float mfx = 1.f - c.fx, mfy = 1.f - c.fy, mfz = 1.f - c.fz;
-        if (a.is3d) {
-            const float dd[8] = {mfz * mfy * mfx, mfz * mfy * c.fx, mfz * c.fy * mfx, mfz * c.fy * c.fx,
-                                 c.fz * mfy * mfx, c.fz * mfy * c.fx, c.fz * c.fy * mfx, c.fz * c.fy * c.fx};
+        const Coords c = map_coords(a.Ai + 6 * (size_t)img, x, y, a.c, false);
+        const float vr = v.x, vi = c.neg ? -v.y : v.y;
+        const float mfx = 1.f - c.fx, mfy = 1.f - c.fy;
+        const float dd[4] = {mfy * mfx, mfy * c.fx, c.fy * mfx, c.fy * c.fx};
 #pragma unroll
-            for (int cc = 0; cc < 8; ++cc) {
-                const int dz = cc >> 2, dy = (cc >> 1) & 1, dx = cc & 1;
-                const size_t idx = ((size_t)(c.z0 + dz) * a.pad + (c.y0 + dy)) * a.padF + (c.x0 + dx);
-                atomicAdd(&gd[2 * idx], dd[cc] * vr);
-                atomicAdd(&gd[2 * idx + 1], dd[cc] * vi);
-                atomicAdd(&gw[idx], dd[cc] * wgt);
-            }
-        } else {
-            const float dd[4] = {mfy * mfx, mfy * c.fx, c.fy * mfx, c.fy * c.fx};
-#pragma unroll
-            for (int cc = 0; cc < 4; ++cc) {
-                const int dy = cc >> 1, dx = cc & 1;
-                const size_t idx = (size_t)(c.y0 + dy) * a.padF + (c.x0 + dx);
-                atomicAdd(&gd[2 * idx], dd[cc] * vr);
-                atomicAdd(&gd[2 * idx + 1], dd[cc] * vi);
-                atomicAdd(&gw[idx], dd[cc] * wgt);
-            }
+        for (int cc = 0; cc < 4; ++cc) {
+            const size_t idx = (size_t)(c.y0 + (cc >> 1)) * a.padF + (c.x0 + (cc & 1));
+            atomicAdd(&acc[idx], (double)(dd[cc] * vr));
+            atomicAdd(&acc[gn + idx], (double)(dd[cc] * vi));
+            atomicAdd(&acc[2 * gn + idx], (double)(dd[cc] * wgt));
         }
     }
+}
+
+__global__ __launch_bounds__(256) void k_bp_add2d(const double* __restrict__ acc, size_t n, float* __restrict__ bp_data,
+                                                  float* __restrict__ bp_weight) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    double s[3] = {0., 0., 0.};
+    for (int k = 0; k < kBpCopies; ++k)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) s[q] += acc[(3 * (size_t)k + q) * n + i];
+    bp_data[2 * i] = (float)((double)bp_data[2 * i] + s[0]);
+    bp_data[2 * i + 1] = (float)((double)bp_data[2 * i + 1] + s[1]);
+    bp_weight[i] = (float)((double)bp_weight[i] + s[2]);
 }
 
 // ------------------------------------------------------------------ launch wrappers
@@ -1751,9 +1772,22 @@ hipError_t launch_store_sums(hipStream_t s, const StoreArgs& a) {
     return hipSuccess;
 }
 
-hipError_t launch_bp_images(hipStream_t s, int n, const BpImageArgs& a) {
+hipError_t launch_bp_image_values(hipStream_t s, int n, const BpImageArgs& a) {
     if (n <= 0) return hipSuccess;
-    k_bp_images<<<n, 256, 0, s>>>(a);
+    k_bp_image_values<<<dim3((a.Pf + 255) / 256, n), 256, 0, s>>>(a);
+    LAUNCH_CHECK();
+    return hipSuccess;
+}
+
+hipError_t launch_bp_images2d(hipStream_t s, int n, const BpImageArgs& a) {
+    if (n <= 0) return hipSuccess;
+    k_bp_images2d<<<n, 256, 0, s>>>(a);
+    LAUNCH_CHECK();
+    return hipSuccess;
+}
+
+hipError_t launch_bp_add2d(hipStream_t s, const double* acc, size_t n, float* bp_data, float* bp_weight) {
+    k_bp_add2d<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(acc, n, bp_data, bp_weight);
     LAUNCH_CHECK();
     return hipSuccess;
 }
