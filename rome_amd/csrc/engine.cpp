@@ -189,7 +189,7 @@ struct rome_ctx {
     DevBuf<float4> cube;  // 3D: 2x2x2 neighbourhood records of grids, rebuilt when a grid changes
     DevBuf<double> Ai_c, Ai_f, sintab, costab, d_sxc, d_syc, d_sxf, d_syf, d_tx, d_ty, d_pose_c, d_pose_f;
     DevBuf<int> c_nfine, c_ires, c_xy, f_nfine, f_ires, f_xy;
-    DevBuf<float2> Sc, Sf;
+    DevBuf<float2> Sc, ScT, Sf;
     DevBuf<double> sigma2, pdf_dir, lpdf_dir, prior_x, prior_y, logsigma2, pdf_m, lpdf_m;
     DevBuf<int> k_m;
     DevBuf<float2> mrow;
@@ -480,6 +480,9 @@ int build_phase_tables(rome_ctx* ctx) {
     HIPCHK(ctx->Sc.reserve((size_t)ctx->T * ctx->Pc));
     HIPCHK(launch_phase_table(ctx->stream, ctx->d_sxc.p, ctx->d_syc.p, ctx->T, ctx->c_xy.p, ctx->Pc, c.ori_size,
                               ctx->sintab.p, ctx->costab.p, ctx->Sc.p));
+    HIPCHK(ctx->ScT.reserve((size_t)ctx->T * ctx->Pc));
+    HIPCHK(launch_phase_table(ctx->stream, ctx->d_sxc.p, ctx->d_syc.p, ctx->T, ctx->c_xy.p, ctx->Pc, c.ori_size,
+                              ctx->sintab.p, ctx->costab.p, ctx->ScT.p, true));
     const int nsf = ctx->T * ctx->NOTf;
     HIPCHK(ctx->Sf.reserve((size_t)nsf * ctx->Pf));
     const double* sx = ctx->two_pass ? ctx->d_sxf.p : ctx->d_sxc.p;
@@ -846,7 +849,6 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
     // ---- image preparation
     if (prec == ROME_PREC_FP32) {
         HIPCHK(ctx->WcT.reserve((size_t)Kdim * Npad));
-        HIPCHK(launch_fill32(s, ctx->WcT.p, 0u, (size_t)Kdim * Npad));
     } else {
         // 256 rows of slack: the audit slice of a learned-proposal pool reads whole 256-row tiles from its start
         HIPCHK(ctx->W16.reserve((size_t)(Npad + 256) * K16));
@@ -857,7 +859,6 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
     }
     const int ldn = (n + 127) / 128 * 128;  // images of the A-term operand, padded with zero columns
     HIPCHK(ctx->MC2c.reserve((size_t)ctx->Kq * ldn));
-    HIPCHK(launch_fill32(s, ctx->MC2c.p, 0u, (size_t)ctx->Kq * ldn));
     HIPCHK(ctx->C2c.reserve(n));
     HIPCHK(ctx->C2f.reserve(n));
     const size_t nPf = (size_t)n * ctx->Pf;
@@ -886,13 +887,15 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
     pa.Npad = Npad;
     pa.c_nfine = ctx->c_nfine.p;
     pa.c_ires = ctx->c_ires.p;
-    pa.Sc = ctx->Sc.p;
+    pa.ScT = ctx->ScT.p;
     pa.Pf = ctx->Pf;
     pa.f_nfine = ctx->f_nfine.p;
     pa.f_ires = ctx->f_ires.p;
     pa.WcT = prec == ROME_PREC_FP32 ? ctx->WcT.p : nullptr;
     pa.MC2c = ctx->MC2c.p;
     pa.mc2_ld = ldn;
+    pa.Kq = ctx->Kq;
+    pa.n = n;
     pa.C2c = ctx->C2c.p;
     pa.Xf = ctx->Xf.p;
     pa.Minvf = ctx->Minvf.p;

@@ -27,15 +27,15 @@ struct PrepArgs {
     int Pc, Pc_pad, T, Npad;
     const int* c_nfine;
     const int* c_ires;
-    const float2* Sc;       // [T][Pc]
+    const float2* ScT;      // [Pc][T]
     // fine pixel set
     int Pf;
     const int* f_nfine;
     const int* f_ires;
     // outputs
-    float* WcT;             // [2*Pc_pad][Npad]
+    float* WcT;             // [2*Pc_pad][Npad], null in the mixed arms
     float* MC2c;            // [Kq][mc2_ld] (transposed: A-term operand; rows >= Pc, columns >= n zero)
-    int mc2_ld;
+    int mc2_ld, Kq, n;
     double* C2c;            // [n]  1/2 (sum Minv|X|^2 + hxi2), coarse
     float2* Xf;             // [n][Pf]
     float* Minvf;           // [n][Pf]
@@ -352,7 +352,7 @@ struct StoreArgs {
 };
 
 hipError_t launch_phase_table(hipStream_t s, const double* sx, const double* sy, int nshift, const int* xy, int P, int ori,
-                              const double* sintab, const double* costab, float2* out);
+                              const double* sintab, const double* costab, float2* out, bool by_pixel = false);
 hipError_t launch_project_coarse(hipStream_t s, const float2* grids, size_t grid_stride, int pad, int padF, int c, int is3d,
                                  const double* Ai, int R, int Mtot, const int* xy, int Pc, int Pc_pad, int my_r_max,
                                  int Mpad, float* FcT);

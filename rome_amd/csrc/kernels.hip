@@ -42,11 +42,11 @@ DEV float2 tab_phase(double sx, double sy, int xy, int ori, const double* __rest
 
 __global__ void k_phase_table(const double* __restrict__ sx, const double* __restrict__ sy, int nshift,
                               const int* __restrict__ xy, int P, int ori, const double* __restrict__ sintab,
-                              const double* __restrict__ costab, float2* __restrict__ out) {
+                              const double* __restrict__ costab, float2* __restrict__ out, int by_pixel) {
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (size_t)nshift * P) return;
     const int s = (int)(idx / P), p = (int)(idx % P);
-    out[idx] = tab_phase(sx[s], sy[s], xy[p], ori, sintab, costab);
+    out[by_pixel ? (size_t)p * nshift + s : idx] = tab_phase(sx[s], sy[s], xy[p], ori, sintab, costab);
 }
 
 // ------------------------------------------------------------------ projections
@@ -201,10 +201,8 @@ __global__ void k_project_plane(const float2* __restrict__ grid, int pad, int pa
 }
 
 // ------------------------------------------------------------------ image preparation (K6)
-// One block per image.  Windows the masked image to the coarse size, builds the
-// CTF-Minv weighted shifted images (GEMM operand), the coarse norm weights and the
-// FP64 image norm; gathers the fine pixel set (masked, unmasked*Minv*CTF for the
-// backprojector).  src/exp_model.cpp:935-1103, src/map3d_optimizer.cpp:2246-2308.
+// One block per image: the FP64 image norm over the coarse pixels, then the fine pixel set (masked,
+// unmasked*Minv*CTF for the backprojector).  src/exp_model.cpp:935-1103, src/map3d_optimizer.cpp:2246-2308.
 __global__ void k_prep_images(PrepArgs a) {
     const int img = blockIdx.x;
     const int g = a.group[img];
@@ -216,21 +214,9 @@ __global__ void k_prep_images(PrepArgs a) {
     // coarse
     double x2 = 0.0;
     for (int p = threadIdx.x; p < a.Pc; p += blockDim.x) {
-        const int nf = a.c_nfine[p];
-        const float2 X = fm[nf];
+        const float2 X = fm[a.c_nfine[p]];
         const double minv = 1.0 / (a.sigma2_fudge * s2[a.c_ires[p]]);
-        const float ctf = a.ctf_in_diff ? fc[nf] : 1.f;
-        const float mc = (float)minv * ctf;
-        a.MC2c[(size_t)p * a.mc2_ld + img] = mc * ctf;
         x2 += minv * ((double)X.x * X.x + (double)X.y * X.y);
-        if (!a.WcT) continue;  // the mixed-precision arm writes its own operand
-        for (int t = 0; t < a.T; ++t) {
-            const float2 S = a.Sc[(size_t)t * a.Pc + p];
-            const float2 XS = cmul(X, S);
-            const size_t col = (size_t)img * a.T + t;
-            a.WcT[(size_t)p * a.Npad + col] = mc * XS.x;
-            a.WcT[(size_t)(a.Pc_pad + p) * a.Npad + col] = mc * XS.y;
-        }
     }
     double s = block_reduce(x2, [](double u, double v) { return u + v; }, red);
     if (threadIdx.x == 0) a.C2c[img] = 0.5 * (s + a.hxi2[img]);
@@ -259,6 +245,58 @@ __global__ void k_prep_images(PrepArgs a) {
     }
     s = block_reduce(x2f, [](double u, double v) { return u + v; }, red);
     if (threadIdx.x == 0) a.C2f[img] = 0.5 * (s + a.hxi2[img]);
+}
+
+// Coarse operands of 8 images and 32 pixels: the A-term's weights Minv CTF^2 and (WCT) the GEMM operand
+// Minv CTF X S_t, both pixel-major, so consecutive lanes take consecutive (image, translation) columns of one
+// pixel; every row and column of the padding is written as zero.  (A block per image with a pixel per lane
+// wrote 4 bytes a line: 1.25 ms for 1000 images of 1651 pixels x 29 translations, this and the rest of the preparation 0.13.)
+constexpr int kPcImg = 8, kPcPix = 32;
+template <bool WCT>
+__global__ __launch_bounds__(256) void k_prep_coarse(PrepArgs a) {
+    __shared__ float2 sX[kPcPix][kPcImg];
+    __shared__ float smc[kPcPix][kPcImg];
+    const int tid = threadIdx.x, i0 = blockIdx.x * kPcImg, p0 = blockIdx.y * kPcPix;
+    {
+        const int tp = tid / kPcImg, ti = tid % kPcImg, p = p0 + tp, img = i0 + ti;
+        float2 X = make_float2(0.f, 0.f);
+        float mc = 0.f, mc2 = 0.f;
+        if (p < a.Pc && img < a.n) {
+            const size_t o = (size_t)img * a.F2f + a.c_nfine[p];
+            const double minv = 1.0 / (a.sigma2_fudge * a.sigma2[(size_t)a.group[img] * a.ori_Fsize + a.c_ires[p]]);
+            const float ctf = a.ctf_in_diff ? a.fctf[o] : 1.f;
+            X = a.fmask[o];
+            mc = (float)minv * ctf;
+            mc2 = mc * ctf;
+        }
+        sX[tp][ti] = X;
+        smc[tp][ti] = mc;
+        if (p < a.Kq) a.MC2c[(size_t)p * a.mc2_ld + img] = mc2;  // img < mc2_ld: the grid covers the padding
+    }
+    if constexpr (WCT) {
+        if (i0 >= a.n) return;
+        __syncthreads();
+        const int lane = tid & 63, col0 = i0 * a.T;
+        const int ncol = (i0 + kPcImg >= a.n ? a.Npad : (i0 + kPcImg) * a.T) - col0;  // the last group: padding too
+        for (int tp = tid >> 6; tp < kPcPix && p0 + tp < a.Pc_pad; tp += 4) {
+            const int p = p0 + tp;
+            float* wr = a.WcT + (size_t)p * a.Npad + col0;
+            float* wi = wr + (size_t)a.Pc_pad * a.Npad;
+            const float2* S = a.ScT + (size_t)p * a.T;
+            for (int c = lane; c < ncol; c += 64) {
+                const int ti = (int)((unsigned)c / (unsigned)a.T), t = c - ti * a.T;
+                float re = 0.f, im = 0.f;
+                if (ti < kPcImg && p < a.Pc) {
+                    const float2 XS = cmul(sX[tp][ti], S[t]);
+                    const float mc = smc[tp][ti];
+                    re = mc * XS.x;
+                    im = mc * XS.y;
+                }
+                wr[c] = re;
+                wi[c] = im;
+            }
+        }
+    }
 }
 
 // Squared magnitudes of the coarse projections, the A-term's K-major operand: Qc[p][m] = Re^2 + Im^2 of
@@ -1421,10 +1459,10 @@ __global__ __launch_bounds__(256) void k_bp_add2d(const double* __restrict__ acc
     } while (0)
 
 hipError_t launch_phase_table(hipStream_t s, const double* sx, const double* sy, int nshift, const int* xy, int P, int ori,
-                              const double* sintab, const double* costab, float2* out) {
+                              const double* sintab, const double* costab, float2* out, bool by_pixel) {
     const size_t tot = (size_t)nshift * P;
     if (tot == 0) return hipSuccess;
-    k_phase_table<<<(unsigned)((tot + 255) / 256), 256, 0, s>>>(sx, sy, nshift, xy, P, ori, sintab, costab, out);
+    k_phase_table<<<(unsigned)((tot + 255) / 256), 256, 0, s>>>(sx, sy, nshift, xy, P, ori, sintab, costab, out, by_pixel ? 1 : 0);
     LAUNCH_CHECK();
     return hipSuccess;
 }
@@ -1504,7 +1542,12 @@ hipError_t launch_project_plane(hipStream_t s, const float2* grid, int pad, int 
 }
 
 hipError_t launch_prep_images(hipStream_t s, int n, const PrepArgs& a) {
+    if (a.mc2_ld % kPcImg || a.mc2_ld < n || a.n != n || a.Kq < a.Pc || a.Pc_pad > (a.Kq + kPcPix - 1) / kPcPix * kPcPix)
+        return hipErrorInvalidValue;
     k_prep_images<<<n, 256, 0, s>>>(a);
+    const dim3 g(a.mc2_ld / kPcImg, (a.Kq + kPcPix - 1) / kPcPix);
+    if (a.WcT) k_prep_coarse<true><<<g, 256, 0, s>>>(a);
+    else k_prep_coarse<false><<<g, 256, 0, s>>>(a);
     LAUNCH_CHECK();
     return hipSuccess;
 }
