@@ -1303,8 +1303,7 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
         HIPCHK(launch_recompute_split(s, prec, n, ra));
         stage_end(ctx, 11);
         HIPCHK(hipMemcpyAsync(ctx->c_dmin1.p, ctx->c_dmin.p, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-        const bool dense =
-            !dd && (ctx->sig_cap == 0 || ctx->sig_dense_left > 0 || (long long)M * T > 0x7fffffffLL);
+        const bool dense = !dd && sig_dense;  // the form the marked samples were kept in
         rc = significance(nullptr, dense, true);
         if (rc) return rc;
         // The significant samples are drawn from the marked ones, whose keys fit the cap when this pass
