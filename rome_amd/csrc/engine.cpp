@@ -201,6 +201,10 @@ struct rome_ctx {
     DevBuf<float> lpd_row, reach, list_val;  // lpd_row [Mpad]: ln pdf_direction per rotation (-inf: none)
     DevBuf<int> vbound, list_cnt;
     DevBuf<unsigned> list_ent;
+    DevBuf<double> ls_hsum, ls_part;  // scan of long lists
+    DevBuf<unsigned> ls_hcnt;
+    DevBuf<long long> ls_key;
+    ListScanArgs list_scan() const { return ListScanArgs{ls_hsum.p, ls_hcnt.p, ls_part.p, ls_key.p}; }
     long long last_list_max = 0, last_list_total = 0;
     int last_coarse_full = 0;  // last batch: 0 list, 1 full pose term, 2 list overflowed -> full
     DevBuf<double> cand_w, cand_du;
@@ -938,7 +942,11 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
     if (!given) HIPCHK(launch_coarse_aterm(s, n, ctx->Qc.p, ctx->Kq, M, ctx->Mpad, ctx->MC2c.p, ldn, ctx->At.p));
     if (!given && ctx->coarse_mode == ROME_COARSE_LIST && ctx->two_pass) {
         HIPCHK(ctx->reach.reserve(n));
-        HIPCHK(launch_list_reach(s, n, wp, ctx->reach.p));
+        HIPCHK(ctx->ls_hsum.reserve((size_t)n * kBinCount));
+        HIPCHK(ctx->ls_hcnt.reserve((size_t)n * kBinCount));
+        HIPCHK(ctx->ls_part.reserve((size_t)n * kListParts * 3));
+        HIPCHK(ctx->ls_key.reserve((size_t)n * kListParts));
+        HIPCHK(launch_list_reach(s, n, wp, ctx->reach.p, ctx->list_scan()));
     }
     stage_end(ctx, 1);
     for (auto* b : {&ctx->c_dmin, &ctx->c_sumw, &ctx->c_maxw, &ctx->c_thr, &ctx->c_tail, &ctx->f_dmin, &ctx->f_sumw,
@@ -1009,7 +1017,7 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
             HIPCHK(launch_weights_fine(s, n, wp_exact, ctx->D2c.p, ctx->blk_task.p, ctx->blk_t.p, ctx->task_m.p,
                                        ctx->blk_off.p, 1, wc_exact, cand, TailArgs{ctx->c_tail.p, ctx->c_dmin1.p}, sg));
         else if (L)
-            HIPCHK(launch_weights_list(s, n, wp, *L, ctx->C2c.p, ctx->emin_key.p, wc, sg, cand));
+            HIPCHK(launch_weights_list(s, n, wp, *L, ctx->C2c.p, ctx->emin_key.p, wc, sg, cand, ctx->list_scan()));
         else
             HIPCHK(launch_weights_coarse(s, n, wp, ctx->E.p, ctx->C2c.p, ctx->emin_key.p, wc, sg, cand));
         stage_end(ctx, 3);

@@ -411,12 +411,21 @@ hipError_t launch_weights_coarse(hipStream_t s, int n, const WeightParams& wp, c
                                  const CandArgs& cand);
 // The same weights and significance from the coarse list (ListArgs); an image whose list
 // overflowed gets status 8 and nothing else.
+// Scan of long coarse lists over several blocks: per image a histogram (zeroed by launch_list_reach) and per part
+// the sum, the maximum with its key and the minimum of u.
+constexpr int kListParts = 8;
+struct ListScanArgs {
+    double* hsum;    // [n][kBinCount]
+    unsigned* hcnt;  // [n][kBinCount]
+    double* part;    // [n][kListParts][3] sum, maximum, minimum of u
+    long long* key;  // [n][kListParts]
+};
 hipError_t launch_weights_list(hipStream_t s, int n, const WeightParams& wp, const ListArgs& list, const double* C2c,
                                const int* emin_key, const WeightOutArgs& wo, const SigArgs& sig,
-                               const CandArgs& cand);
+                               const CandArgs& cand, const ListScanArgs& scan);
 // reach[img] = kWeightWindow + (max - min of ln pdf_offset over (class, translation)) + slack,
-// +inf when a pdf_offset is zero
-hipError_t launch_list_reach(hipStream_t s, int n, const WeightParams& wp, float* reach);
+// +inf when a pdf_offset is zero; clears the images' histograms of the list scan
+hipError_t launch_list_reach(hipStream_t s, int n, const WeightParams& wp, float* reach, const ListScanArgs& scan);
 hipError_t launch_weights_fine(hipStream_t s, int n, const WeightParams& wp, const double* D2, const int* blk_task,
                                const int* blk_t, const int* task_m, const long long* img_blk, int NE,
                                const WeightOutArgs& wo, const CandArgs& cand, TailArgs tail = TailArgs{nullptr, nullptr},

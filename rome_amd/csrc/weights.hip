@@ -2,7 +2,7 @@
 //   convertSquaredDifferencesToWeights  src/map3d_optimizer.cpp:1610-1810 (2D :1077-1224)
 //   findAllSignificantPoints            src/map3d_optimizer.cpp:1812-1931 (2D :1226-1311)
 //
-// One 1024-thread block per image.  With u = d - ln(pdf_direction * pdf_offset) the weight of
+// One block per image.  With u = d - ln(pdf_direction * pdf_offset) the weight of
 // an entry is w = exp(dmin - u); wherever a weight is used this kernel evaluates the reference's
 // own expression pdf_direction * pdf_offset * exp(-(diff2 - min_diff2)) (0 beyond 700).
 //
@@ -17,8 +17,16 @@
 //            -> threshold and NR_SIGN.
 //   mark   : (coarse) the samples with w >= threshold: their keys m*T + t per image, or bits of
 //            the significance mask.
-// When an image has more candidates than the list holds, select / mark rescan the entries.
+// When an image has more candidates than the list holds, the entries down to the crossing bucket (and the mark
+// margin) are collected in one more pass; if those do not fit either, select / mark rescan the entries.
+//
+// A coarse list longer than kSplitList is scanned by kListParts blocks (k_list_scan) ahead of its image's
+// block: a broad posterior leaves hundreds of thousands of entries inside the window, each an FP64 exponential.
+// Measured: 333 images of 13824 rotations x 29 shifts, lists of 50 thousand entries on average and up to 302
+// thousand, one block an image with three exact passes 938 us, now 136 (scan) + 243; 2000 images of 18432 x 81,
+// 10 thousand on average, 547 us, now 132 + 192.
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <stdint.h>
 
 #include "device_util.h"
@@ -49,10 +57,15 @@ struct Cand {
     int cap;
 };
 
+// K * T tables of the image's ln pdf_offset, in dynamic LDS
+struct OffTables {
+    double *poff, *lpoff;
+    float* lpoff_f;
+    DEV OffTables(double* lds, int kt) : poff(lds), lpoff(lds + kt), lpoff_f(reinterpret_cast<float*>(lds + 2 * kt)) {}
+};
+inline size_t off_bytes(const WeightParams& wp) { return (size_t)wp.K * wp.T * 20; }
+
 struct WShared {
-    double poff[kMaxKT];
-    double lpoff[kMaxKT];
-    float lpoff_f[kMaxKT];
     double hsum[kBinCount];
     unsigned int hcnt[kBinCount];
     double cw[kSortCap];
@@ -63,22 +76,26 @@ struct WShared {
     int ncand;
     int nmark;
     int done;
+    int bstar, blast;
     double lo, width, mbefore;
     long long cbefore;
     double thr;
     long long nsig;
 };
 
-// Pre(e0, bound, lpoff_f) -> bit mask over the Pre::VW entries e0 .. e0 + VW - 1 (those < count): a
+// Pre(e0, bound, lpmax, lpoff_f) -> bit mask over the Pre::VW entries e0 .. e0 + VW - 1 (those < count): a
 // cheap FP32 test whose bit is clear only for entries whose exact FP64 du = u - u0 is >= kWin when
 // bound = (float)(u0 + kWin) + margin (the margin covers the FP32 rounding).
 // Key(e, m, t): the entry's position in the reference's loop order; the max-posterior entry is the
 // first maximum in that order (ties between equal weights).
-template <typename Get, typename Pre, typename Key>
+template <int NT, typename Get, typename Pre, typename Key>
 __device__ void weight_pass(int img, size_t count, double cimg, const WeightParams& wp, Get get, Pre pre, Key key,
                             WeightOut wo, WShared& sh, SigArgs sig, Cand cand, const int* emin_key,
-                            TailArgs tail = TailArgs{nullptr, nullptr}) {
-    constexpr int NT = 1024;
+                            TailArgs tail = TailArgs{nullptr, nullptr},
+                            ListScanArgs scan = ListScanArgs{nullptr, nullptr, nullptr, nullptr}) {
+    static_assert(kBinCount % NT == 0, "whole buckets per thread");
+    extern __shared__ double off_lds[];
+    const OffTables tb(off_lds, wp.K * wp.T);
     const int tid = threadIdx.x;
     const int T = wp.T;
     double lpo_max = -INFINITY;
@@ -86,16 +103,16 @@ __device__ void weight_pass(int img, size_t count, double cimg, const WeightPara
         const int k = q / T, t = q % T;
         const double po = pdf_offset(wp.trans_x[t], wp.trans_y[t], wp.old_offx[img], wp.old_offy[img], wp.prior_x[k],
                                      wp.prior_y[k], wp.sigma2_offset);
-        sh.poff[q] = po;
-        sh.lpoff[q] = po > 0 ? log(po) : -INFINITY;
-        sh.lpoff_f[q] = (float)sh.lpoff[q];
-        lpo_max = fmax(lpo_max, sh.lpoff[q]);
+        tb.poff[q] = po;
+        tb.lpoff[q] = po > 0 ? log(po) : -INFINITY;
+        tb.lpoff_f[q] = (float)tb.lpoff[q];
+        lpo_max = fmax(lpo_max, tb.lpoff[q]);
     }
     lpo_max = block_reduce(lpo_max, [](double a, double b) { return fmax(a, b); }, sh.red_d);
-    auto u_of = [&](double d, int m, int t) { return d - (wp.lpdf_m[m] + sh.lpoff[wp.k_m[m] * T + t]); };
+    auto u_of = [&](double d, int m, int t) { return d - (wp.lpdf_m[m] + tb.lpoff[wp.k_m[m] * T + t]); };
     auto w_of = [&](double d, int m, int t, double dmin) {
         const double dd = (d + cimg) - dmin;
-        const double w = wp.pdf_m[m] * sh.poff[wp.k_m[m] * T + t];
+        const double w = wp.pdf_m[m] * tb.poff[wp.k_m[m] * T + t];
         return dd > 700. ? 0. : w * exp(-dd);
     };
     // ---- minimum of d (the coarse pass gets it from the cross-term epilogue)
@@ -115,10 +132,11 @@ __device__ void weight_pass(int img, size_t count, double cimg, const WeightPara
     double u0 = mn - (wp.lpdf_max + lpo_max);
     // FP32 pre-test bound: rounding of d - lpdf - lpoff and of u0 + kWin stays far below the margin
     // (relative 2^-22 of magnitudes that the 1e-4 term covers; log priors are > -746)
-    auto pre_bound = [&](double a0) {
-        return (float)(a0 + kWin) + 1.0f + 1e-4f * (float)(fabs(a0) + fabs(mn) + kWin + fabs(wp.lpdf_max) + fabs(lpo_max));
+    auto pre_bound = [&](double a0, double win) {
+        return (float)(a0 + win) + 1.0f + 1e-4f * (float)(fabs(a0) + fabs(mn) + kWin + fabs(wp.lpdf_max) + fabs(lpo_max));
     };
-    float bound = pre_bound(u0);
+    float bound = pre_bound(u0, kWin);
+    const float lpmax = (float)(wp.lpdf_max + lpo_max);
     // every entry that may lie inside the window, each thread in increasing e (four groups of VW in
     // flight per step): fn(e)
     auto for_window = [&](float bnd, auto&& fn) {
@@ -126,7 +144,7 @@ __device__ void weight_pass(int img, size_t count, double cimg, const WeightPara
         for (size_t e0 = (size_t)tid * VW; e0 < count; e0 += 4 * STEP) {
             unsigned m[4];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) m[g] = pre(e0 + g * STEP, bnd, sh.lpoff_f);
+            for (int g = 0; g < 4; ++g) m[g] = pre(e0 + g * STEP, bnd, lpmax, tb.lpoff_f);
 #pragma unroll
             for (int g = 0; g < 4; ++g)
                 while (m[g]) {
@@ -139,7 +157,27 @@ __device__ void weight_pass(int img, size_t count, double cimg, const WeightPara
     // ---- scan
     double sum = 0., mx = -1.;
     long long am = -1;
-    for (int attempt = 0; attempt < 2; ++attempt) {
+    bool scanned = false;
+    if (scan.part) {  // by k_list_scan, anchored at the same u0; usable unless the window has to move
+        double umin = INFINITY;
+        for (int q = 0; q < kListParts; ++q) umin = fmin(umin, scan.part[((size_t)img * kListParts + q) * 3 + 2]);
+        scanned = !(umin - u0 > kAnchorSlack);
+    }
+    if (scanned) {
+        for (int b = tid; b < kBinCount; b += NT) {
+            sh.hsum[b] = scan.hsum[(size_t)img * kBinCount + b];
+            sh.hcnt[b] = scan.hcnt[(size_t)img * kBinCount + b];
+        }
+        if (tid == 0) sh.ncand = INT_MAX;
+        if (tid < kListParts) {  // block reductions below
+            const size_t q = (size_t)img * kListParts + tid;
+            sum = scan.part[3 * q];
+            mx = scan.part[3 * q + 1];
+            am = scan.key[q];
+        }
+        __syncthreads();
+    }
+    for (int attempt = 0; attempt < 2 && !scanned; ++attempt) {
         for (int b = tid; b < kBinCount; b += NT) {
             sh.hsum[b] = 0.;
             sh.hcnt[b] = 0;
@@ -192,7 +230,7 @@ __device__ void weight_pass(int img, size_t count, double cimg, const WeightPara
             umin = block_reduce(umin, [](double a, double b) { return fmin(a, b); }, sh.red_d);
         }
         u0 = umin;  // priors spread u widely: anchor the window at the true minimum and rescan
-        bound = pre_bound(u0);
+        bound = pre_bound(u0, kWin);
     }
     sum = block_reduce(sum, [](double a, double b) { return a + b; }, sh.red_d);
     // mass of the previous pass's unmarked entries, re-anchored from its minimum to this one:
@@ -205,8 +243,9 @@ __device__ void weight_pass(int img, size_t count, double cimg, const WeightPara
         mx = m2;
     }
     const double target = wp.adaptive_fraction * sum;
-    const int ncand = sh.ncand;
-    const bool listed = ncand <= cand.cap;
+    int ncand = sh.ncand;
+    bool listed = ncand <= cand.cap;
+    const bool overflow = !listed;
     // visit(lo, hi, fn): every entry with weight > 0 and lo <= du < hi, as (w, du, e)
     auto visit = [&](double lo, double hi, auto&& fn) {
         if (listed) {
@@ -238,35 +277,83 @@ __device__ void weight_pass(int img, size_t count, double cimg, const WeightPara
     __syncthreads();
     int status = 0;
     for (int level = 0;; ++level) {
-        if (tid == 0) {
-            double cum = sh.mbefore;
-            long long cnt = sh.cbefore;
-            int bstar = -1, last = -1;
-            for (int b = 0; b < kBinCount; ++b) {
-                if (sh.hcnt[b] == 0) continue;
-                last = b;
-                if (cum + sh.hsum[b] > target) {
-                    bstar = b;
-                    break;
+        // the first bucket where the cumulative mass crosses the target, from block-wide prefix sums (a single
+        // thread walking the buckets took a quarter of a small image's pass)
+        {
+            constexpr int PT = kBinCount / NT;
+            const int lane = tid & 63, wid = tid >> 6, b0 = PT * tid;
+            double p = 0.;
+            long long pc = 0;
+            for (int q = 0; q < PT; ++q) {
+                p += sh.hsum[b0 + q];
+                pc += sh.hcnt[b0 + q];
+            }
+            double ex = 0.;  // mass and count before the thread's buckets
+            long long exc = 0;
+            {
+                double v = p;
+                long long vc = pc;
+                for (int o = 1; o < 64; o <<= 1) {
+                    const double u = __shfl_up(v, o, 64);
+                    const long long uc = __shfl_up(vc, o, 64);
+                    if (lane >= o) {
+                        v += u;
+                        vc += uc;
+                    }
                 }
-                cum += sh.hsum[b];
-                cnt += sh.hcnt[b];
+                if (lane == 63) {
+                    sh.red_d[wid] = v;
+                    sh.red_l[wid] = vc;
+                }
+                const double u = __shfl_up(v, 1, 64);
+                const long long uc = __shfl_up(vc, 1, 64);
+                if (lane) {
+                    ex = u;
+                    exc = uc;
+                }
             }
-            if (bstar < 0 && last >= 0) {  // rounding left the crossing unreached: last bucket
-                bstar = last;
-                cum -= sh.hsum[last];
-                cnt -= sh.hcnt[last];
+            if (tid == 0) {
+                sh.bstar = kBinCount;
+                sh.blast = -1;
+                sh.ncand_sort = 0;
             }
-            if (bstar < 0) {
-                sh.done = 2;
-            } else {
-                sh.mbefore = cum;
-                sh.cbefore = cnt;
-                sh.lo = sh.lo + bstar * sh.width;
-                sh.done = (sh.hcnt[bstar] <= (unsigned)kSortCap || level >= 2) ? 1 : 0;
+            __syncthreads();
+            double off = sh.mbefore;
+            long long offc = sh.cbefore;
+            for (int w = 0; w < wid; ++w) {
+                off += sh.red_d[w];
+                offc += sh.red_l[w];
+            }
+            double cum = off + ex;
+            int cross = -1, last = -1;
+            if (pc) {
+                for (int q = 0; q < PT; ++q) {
+                    if (!sh.hcnt[b0 + q]) continue;
+                    last = b0 + q;
+                    cum += sh.hsum[b0 + q];
+                    if (cross < 0 && cum > target) cross = b0 + q;
+                }
+                if (cross >= 0) atomicMin(&sh.bstar, cross);
+                atomicMax(&sh.blast, last);
+            }
+            __syncthreads();
+            // rounding left the crossing unreached: the last bucket
+            const int bs = sh.bstar < kBinCount ? sh.bstar : sh.blast;
+            if (bs < 0) {
+                if (tid == 0) sh.done = 2;
+            } else if (bs / PT == tid) {
+                double m = off + ex;
+                long long c = offc + exc;
+                for (int q = b0; q < bs; ++q) {
+                    m += sh.hsum[q];
+                    c += sh.hcnt[q];
+                }
+                sh.mbefore = m;
+                sh.cbefore = c;
+                sh.lo = sh.lo + bs * sh.width;
+                sh.done = (sh.hcnt[bs] <= (unsigned)kSortCap || level >= 2) ? 1 : 0;
                 sh.width = sh.width / (double)kBinCount;
             }
-            sh.ncand_sort = 0;
         }
         __syncthreads();
         if (sh.done == 2) {
@@ -274,6 +361,33 @@ __device__ void weight_pass(int img, size_t count, double cimg, const WeightPara
             break;
         }
         const double lo = sh.lo, hi = lo + sh.width * kBinCount;
+        if (!listed && level == 0) {
+            // everything select and mark can still ask for: w >= thr_mark >= the bucket's least weight exp(-margin)
+            const double need = hi + wp.mark_margin + 1e-6;
+            __syncthreads();
+            if (tid == 0) sh.ncand = 0;
+            __syncthreads();
+            if (need < kWin)
+                for_window(pre_bound(u0, need), [&](size_t e) {
+                    double d;
+                    int m, t;
+                    if (!get(e, d, m, t)) return;
+                    const double du = u_of(d, m, t) - u0;
+                    if (!(du < need)) return;
+                    const double w = w_of(d, m, t, dmin);
+                    if (!(w > 0.)) return;
+                    const int slot = atomicAdd(&sh.ncand, 1);
+                    if (slot < cand.cap) {
+                        const size_t o = (size_t)img * cand.cap + slot;
+                        cand.w[o] = w;
+                        cand.du[o] = du;
+                        cand.e[o] = (long long)e;
+                    }
+                });
+            __syncthreads();
+            ncand = sh.ncand;
+            listed = need < kWin && ncand <= cand.cap;
+        }
         if (sh.done == 1) {
             visit(lo, hi, [&](double w, double, long long e) {
                 const int slot = atomicAdd(&sh.ncand_sort, 1);
@@ -349,7 +463,7 @@ __device__ void weight_pass(int img, size_t count, double cimg, const WeightPara
         wo.amax[img] = am;
         wo.thr[img] = thr;
         if (wo.nsig) wo.nsig[img] = status == 1 ? 0 : (int)sh.nsig;
-        wo.status[img] = status | (listed ? 0 : 4);
+        wo.status[img] = status | (overflow ? 4 : 0);
     }
     // ---- mark: w >= threshold, with the weight the reference compares (or the superset within
     // mark_margin nats of it); the mass left unmarked goes to wo.tail
@@ -407,7 +521,7 @@ struct CoarsePre {
     int Mtot;
     const float2* mrow;
     bool vec;
-    DEV unsigned operator()(size_t e0, float bound, const float* lpoff_f) const {
+    DEV unsigned operator()(size_t e0, float bound, float, const float* lpoff_f) const {
         if (e0 >= count) return 0u;
         unsigned msk = 0u;
         if (vec) {
@@ -436,11 +550,31 @@ struct CoarsePre {
     }
 };
 
+// List pre-test: d - lpdf_m - lpoff in FP32, as CoarsePre (most of a list lies outside the window: it was kept
+// against bounds that only fell later).
+struct ListPre {
+    static constexpr int VW = 1;
+    const unsigned* ent;
+    const float* val;
+    size_t count;
+    unsigned long long magic;
+    int Mtot;
+    const float2* mrow;
+    // lpmax: the largest ln prior; an entry that fails with it needs no look at its own
+    DEV unsigned operator()(size_t e, float bound, float lpmax, const float* lpoff_f) const {
+        if (e >= count || !(val[e] - lpmax < bound)) return 0u;
+        int m, t;
+        coarse_mt(ent[e], magic, Mtot, m, t);
+        const float2 mr = mrow[m];
+        return val[e] - mr.x - lpoff_f[__float_as_int(mr.y) + t] < bound ? 1u : 0u;
+    }
+};
+
 // Fine pass: every entry goes to the exact test.
 struct AllPre {
     static constexpr int VW = 1;
     size_t count;
-    DEV unsigned operator()(size_t e0, float, const float*) const { return e0 < count ? 1u : 0u; }
+    DEV unsigned operator()(size_t e0, float, float, const float*) const { return e0 < count ? 1u : 0u; }
 };
 
 __global__ __launch_bounds__(1024) void k_weights_coarse(WeightParams wp, const float* __restrict__ E,
@@ -461,16 +595,108 @@ __global__ __launch_bounds__(1024) void k_weights_coarse(WeightParams wp, const 
     };
     const CoarsePre pre{Ei, (size_t)Mtot * T, magic, Mtot, wp.mrow, (Mtot & 3) == 0};
     auto key = [&](size_t, int m, int t) { return (long long)m * T + t; };  // (class, dir, psi, t) order
-    weight_pass(img, (size_t)Mtot * T, C2c[img], wp, get, pre, key, wo, sh, sig, cand, emin_key);
+    weight_pass<1024>(img, (size_t)Mtot * T, C2c[img], wp, get, pre, key, wo, sh, sig, cand, emin_key);
+}
+
+// The scan of weight_pass (the same expressions and anchor) over part blockIdx.y of a list longer than
+// kSplitList, runs of 1024 entries dealt out round-robin.  8192: below it the image's own block is as fast.
+constexpr int kSplitList = 8192;
+__global__ __launch_bounds__(256) void k_list_scan(WeightParams wp, ListArgs L, const double* __restrict__ C2c,
+                                                   const int* __restrict__ emin_key, ListScanArgs out) {
+    __shared__ double hsum[kBinCount];
+    __shared__ unsigned hcnt[kBinCount];
+    __shared__ double red_d[16];
+    __shared__ long long red_l[16];
+    extern __shared__ double off_lds[];
+    const int img = blockIdx.x, part = blockIdx.y, tid = threadIdx.x, T = wp.T;
+    const int cnt = L.count[img];
+    if (cnt <= kSplitList || cnt > L.cap) return;
+    const OffTables tb(off_lds, wp.K * T);
+    double lpo_max = -INFINITY;
+    for (int q = tid; q < wp.K * T; q += 256) {
+        const int k = q / T, t = q % T;
+        const double po = pdf_offset(wp.trans_x[t], wp.trans_y[t], wp.old_offx[img], wp.old_offy[img], wp.prior_x[k],
+                                     wp.prior_y[k], wp.sigma2_offset);
+        tb.poff[q] = po;
+        tb.lpoff[q] = po > 0 ? log(po) : -INFINITY;
+        lpo_max = fmax(lpo_max, tb.lpoff[q]);
+    }
+    for (int b = tid; b < kBinCount; b += 256) {
+        hsum[b] = 0.;
+        hcnt[b] = 0u;
+    }
+    lpo_max = block_reduce(lpo_max, [](double a, double b) { return fmax(a, b); }, red_d);
+    const double mn = (double)float_from_order_key(emin_key[img]), cimg = C2c[img], dmin = mn + cimg;
+    const double u0 = mn - (wp.lpdf_max + lpo_max);
+    const unsigned* ent = L.ent + (size_t)img * L.cap;
+    const float* val = L.val + (size_t)img * L.cap;
+    double sum = 0., mx = -1., umin = INFINITY;
+    long long am = -1;
+    for (int i0 = part * 1024 + tid; i0 < cnt; i0 += kListParts * 1024) {
+        unsigned e[4];
+        float v[4], lp[4];
+        int m[4], t[4], kT[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int i = min(i0 + 256 * g, cnt - 1);
+            e[g] = ent[i];
+            v[g] = val[i];
+        }
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            coarse_mt(e[g], wp.magicM, wp.Mtot, m[g], t[g]);
+            const float2 mr = wp.mrow[m[g]];
+            lp[g] = mr.x;
+            kT[g] = __float_as_int(mr.y);
+        }
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if (i0 + 256 * g >= cnt || !(lp[g] > -INFINITY)) continue;
+            const double d = (double)v[g], u = d - (wp.lpdf_m[m[g]] + tb.lpoff[kT[g] + t[g]]);
+            umin = fmin(umin, u);
+            const double du = u - u0;
+            if (!(du < kWin)) continue;
+            const double dd = (d + cimg) - dmin;
+            const double w = dd > 700. ? 0. : wp.pdf_m[m[g]] * tb.poff[kT[g] + t[g]] * exp(-dd);
+            sum += w;
+            const long long ke = (long long)m[g] * T + t[g];
+            if (w > mx || (w == mx && ke < am)) {
+                mx = w;
+                am = ke;
+            }
+            if (w > 0.) {
+                const int b = du > 0. ? (int)(du * kBinScale) : 0;
+                atomicAdd(&hsum[b], w);
+                atomicAdd(&hcnt[b], 1u);
+            }
+        }
+    }
+    sum = block_reduce(sum, [](double a, double b) { return a + b; }, red_d);
+    umin = block_reduce(umin, [](double a, double b) { return fmin(a, b); }, red_d);
+    const double m2 = block_reduce(mx, [](double a, double b) { return fmax(a, b); }, red_d);
+    am = block_reduce((mx == m2 && am >= 0) ? am : (long long)0x7fffffffffffffffLL,
+                      [](long long a, long long b) { return a < b ? a : b; }, red_l);
+    if (tid == 0) {
+        const size_t q = (size_t)img * kListParts + part;
+        out.part[3 * q] = sum;
+        out.part[3 * q + 1] = m2;
+        out.part[3 * q + 2] = umin;
+        out.key[q] = am == 0x7fffffffffffffffLL ? -1 : am;
+    }
+    for (int b = tid; b < kBinCount; b += 256)
+        if (hcnt[b]) {
+            atomicAdd(&out.hsum[(size_t)img * kBinCount + b], hsum[b]);
+            atomicAdd(&out.hcnt[(size_t)img * kBinCount + b], hcnt[b]);
+        }
 }
 
 // Coarse weights from the list the cross-term GEMM kept (every entry within kWin of the minimum
 // u, and more): entries i = 0 .. count-1 of the image's list, argmax keys in the reference's order.
-// 8 waves per SIMD: two 1024-thread blocks per CU (64 VGPRs; the few spills cost less than the
-// second block gains on this latency-bound pass)
-__global__ __launch_bounds__(1024, 8) void k_weights_list(WeightParams wp, ListArgs L, const double* __restrict__ C2c,
-                                                       const int* __restrict__ emin_key, WeightOut wo,
-                                                       SigArgs sig, Cand cand) {
+// 512 threads, two blocks per CU without spills (1024 at 64 VGPRs spilled 44 registers).
+constexpr int kListThreads = 512;
+__global__ __launch_bounds__(kListThreads, 4) void k_weights_list(WeightParams wp, ListArgs L, const double* __restrict__ C2c,
+                                                               const int* __restrict__ emin_key, WeightOut wo,
+                                                               SigArgs sig, Cand cand, ListScanArgs scan) {
     __shared__ WShared sh;
     const int img = blockIdx.x;
     const int cnt = L.count[img];
@@ -492,16 +718,28 @@ __global__ __launch_bounds__(1024, 8) void k_weights_list(WeightParams wp, ListA
         d = (double)val[i];
         return true;
     };
-    const AllPre pre{(size_t)cnt};
+    const ListPre pre{ent, val, (size_t)cnt, magic, Mtot, wp.mrow};
     auto key = [&](size_t, int m, int t) { return (long long)m * T + t; };
-    weight_pass(img, (size_t)cnt, C2c[img], wp, get, pre, key, wo, sh, sig, cand, emin_key);
+    const bool split = cnt > kSplitList;
+    if (!split) scan.part = nullptr;
+    weight_pass<kListThreads>(img, (size_t)cnt, C2c[img], wp, get, pre, key, wo, sh, sig, cand, emin_key,
+                              TailArgs{nullptr, nullptr}, scan);
+    if (split)  // the scan of a rerun of this pool's weights starts from zero again
+        for (int b = threadIdx.x; b < kBinCount; b += kListThreads) {
+            scan.hsum[(size_t)img * kBinCount + b] = 0.;
+            scan.hcnt[(size_t)img * kBinCount + b] = 0u;
+        }
 }
 
 // reach[img] = kWin + (max - min of ln pdf_offset over the image's (class, translation) pairs) + 1
 // nat of slack (+inf when a pdf_offset is zero: the list then takes every entry and overflows).
-__global__ void k_list_reach(WeightParams wp, float* __restrict__ reach) {
+__global__ void k_list_reach(WeightParams wp, float* __restrict__ reach, ListScanArgs scan) {
     __shared__ double red[16];
     const int img = blockIdx.x;
+    for (int b = threadIdx.x; b < kBinCount; b += blockDim.x) {
+        scan.hsum[(size_t)img * kBinCount + b] = 0.;
+        scan.hcnt[(size_t)img * kBinCount + b] = 0u;
+    }
     double lo = INFINITY, hi = -INFINITY;
     for (int q = threadIdx.x; q < wp.K * wp.T; q += blockDim.x) {
         const int k = q / wp.T, t = q - k * wp.T;
@@ -516,8 +754,9 @@ __global__ void k_list_reach(WeightParams wp, float* __restrict__ reach) {
     if (threadIdx.x == 0) reach[img] = lo > -INFINITY ? (float)(kWin + (hi - lo) + 1.0) : INFINITY;
 }
 
-// two blocks per CU, as k_weights_list
-__global__ __launch_bounds__(1024, 8) void k_weights_fine(WeightParams wp, const double* __restrict__ D2,
+// An image has some hundreds of fine samples: 256 threads, more images in flight per CU and cheaper barriers.
+constexpr int kFineThreads = 256;
+__global__ __launch_bounds__(kFineThreads, 3) void k_weights_fine(WeightParams wp, const double* __restrict__ D2,
                                                        const int* __restrict__ blk_task, const int* __restrict__ blk_t,
                                                        const int* __restrict__ task_m,
                                                        const long long* __restrict__ img_blk, int log2NE, WeightOut wo,
@@ -536,7 +775,7 @@ __global__ __launch_bounds__(1024, 8) void k_weights_fine(WeightParams wp, const
     };
     const AllPre pre{count};
     auto key = [](size_t e, int, int) { return (long long)e; };
-    weight_pass(img, count, 0.0, wp, get, pre, key, wo, sh, sig, cand, nullptr, tail);
+    weight_pass<kFineThreads>(img, count, 0.0, wp, get, pre, key, wo, sh, sig, cand, nullptr, tail);
 }
 
 }  // namespace
@@ -546,23 +785,25 @@ hipError_t launch_weights_coarse(hipStream_t s, int n, const WeightParams& wp, c
                                  const CandArgs& c) {
     if (sig.keys && ((long long)wp.Mtot * wp.T > 0x7fffffffLL || sig.cap > kSigCap)) return hipErrorInvalidValue;
     WeightOut o{wo.dmin, wo.sumw, wo.maxw, wo.amax, wo.thr, wo.nsig, wo.status, wo.tail};
-    k_weights_coarse<<<n, 1024, 0, s>>>(wp, E, C2c, emin_key, o, sig, Cand{c.w, c.du, c.e, c.cap});
+    k_weights_coarse<<<n, 1024, off_bytes(wp), s>>>(wp, E, C2c, emin_key, o, sig, Cand{c.w, c.du, c.e, c.cap});
     return hipGetLastError();
 }
 
 hipError_t launch_weights_list(hipStream_t s, int n, const WeightParams& wp, const ListArgs& list, const double* C2c,
                                const int* emin_key, const WeightOutArgs& wo, const SigArgs& sig,
-                               const CandArgs& c) {
+                               const CandArgs& c, const ListScanArgs& scan) {
     if (wp.K * wp.T > kMaxKT) return hipErrorInvalidValue;
     if (sig.keys && ((long long)wp.Mtot * wp.T > 0x7fffffffLL || sig.cap > kSigCap)) return hipErrorInvalidValue;
     WeightOut o{wo.dmin, wo.sumw, wo.maxw, wo.amax, wo.thr, wo.nsig, wo.status, wo.tail};
-    k_weights_list<<<n, 1024, 0, s>>>(wp, list, C2c, emin_key, o, sig, Cand{c.w, c.du, c.e, c.cap});
+    if (list.cap > kSplitList)
+        k_list_scan<<<dim3(n, kListParts), 256, off_bytes(wp), s>>>(wp, list, C2c, emin_key, scan);
+    k_weights_list<<<n, kListThreads, off_bytes(wp), s>>>(wp, list, C2c, emin_key, o, sig, Cand{c.w, c.du, c.e, c.cap}, scan);
     return hipGetLastError();
 }
 
-hipError_t launch_list_reach(hipStream_t s, int n, const WeightParams& wp, float* reach) {
+hipError_t launch_list_reach(hipStream_t s, int n, const WeightParams& wp, float* reach, const ListScanArgs& scan) {
     if (n == 0) return hipSuccess;
-    k_list_reach<<<n, 256, 0, s>>>(wp, reach);
+    k_list_reach<<<n, 256, 0, s>>>(wp, reach, scan);
     return hipGetLastError();
 }
 
@@ -575,7 +816,7 @@ hipError_t launch_weights_fine(hipStream_t s, int n, const WeightParams& wp, con
     if ((sig.keys || sig.mask) && NE != 1) return hipErrorInvalidValue;  // marking keys m*T + t: one entry per block
     if (sig.keys && ((long long)wp.Mtot * wp.T > 0x7fffffffLL || sig.cap > kSigCap)) return hipErrorInvalidValue;
     WeightOut o{wo.dmin, wo.sumw, wo.maxw, wo.amax, wo.thr, wo.nsig, wo.status, wo.tail};
-    k_weights_fine<<<n, 1024, 0, s>>>(wp, D2, blk_task, blk_t, task_m, img_blk, log2NE, o, Cand{c.w, c.du, c.e, c.cap},
+    k_weights_fine<<<n, kFineThreads, off_bytes(wp), s>>>(wp, D2, blk_task, blk_t, task_m, img_blk, log2NE, o, Cand{c.w, c.du, c.e, c.cap},
                                       tail, sig);
     return hipGetLastError();
 }
