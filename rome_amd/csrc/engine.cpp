@@ -2607,17 +2607,15 @@ int rome_fourier_map(rome_ctx* ctx, int iclass, const double* vol, int do_griddi
     HIPCHK(ctx->fm_F.reserve(nF));
     const hipfftResult fr = hipfftExecD2Z(plan, ctx->fm_Mc.p, reinterpret_cast<hipfftDoubleComplex*>(ctx->fm_F.p));
     if (fr != HIPFFT_SUCCESS) return fail(ctx, ROME_ERR_HIP, "hipfftExecD2Z failed: %d", (int)fr);
-    HIPCHK(ctx->fm_grid64.reserve(ctx->grid_n));
-    HIPCHK(hipMemsetAsync(ctx->fm_grid64.p, 0, ctx->grid_n * sizeof(double2), s));
+    if (grid_out) HIPCHK(ctx->fm_grid64.reserve(ctx->grid_n));
     float2* g32 = ctx->grids.p + ctx->grid_n * iclass;
-    HIPCHK(hipMemsetAsync(g32, 0, ctx->grid_n * sizeof(float2), s));
     HIPCHK(ctx->fm_pw.reserve(oriF));
     HIPCHK(ctx->fm_cnt.reserve(oriF));
     HIPCHK(hipMemsetAsync(ctx->fm_pw.p, 0, oriF * sizeof(double), s));
     HIPCHK(hipMemsetAsync(ctx->fm_cnt.p, 0, oriF * sizeof(double), s));
     const double normfft = dim3 ? (double)(pf * pf * pf * ori) : (double)(pf * pf);
-    HIPCHK(launch_fm_window(s, ctx->fm_F.p, padori, dim3, pf, ctx->r_max, ctx->pad, oriF, normfft, ctx->fm_grid64.p,
-                            g32, ctx->fm_pw.p, ctx->fm_cnt.p));
+    HIPCHK(launch_fm_window(s, ctx->fm_F.p, padori, dim3, pf, ctx->r_max, ctx->pad, oriF, normfft,
+                            grid_out ? ctx->fm_grid64.p : nullptr, g32, ctx->fm_pw.p, ctx->fm_cnt.p));
     std::vector<double> pw(oriF), cnt(oriF);
     HIPCHK(hipMemcpyAsync(pw.data(), ctx->fm_pw.p, oriF * sizeof(double), hipMemcpyDeviceToHost, s));
     HIPCHK(hipMemcpyAsync(cnt.data(), ctx->fm_cnt.p, oriF * sizeof(double), hipMemcpyDeviceToHost, s));
