@@ -10,13 +10,17 @@
 #include <atomic>
 #include <chrono>
 #include <cmath>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <limits>
+#include <mutex>
 #include <numeric>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/rome_gpu.h"
@@ -106,6 +110,112 @@ struct DevBuf {
     }
 };
 
+// Large results for a caller's pageable arrays.  The runtime stages such a copy through its own buffer with one
+// thread, which on the freshly allocated pages callers usually pass ran at 10 GB/s; here the pieces land in a ring
+// of pinned slots at the link's rate while up to six threads, alive for the call only, copy the ones before out.
+struct CopyOut {
+    static constexpr size_t kPiece = (size_t)1 << 20, kSmall = (size_t)4 << 20;
+    static constexpr int kSlots = 8, kThreads = 6;
+    struct Part {
+        void* dst;
+        const void* src;  // device
+        size_t bytes;
+    };
+    PinnedBuf ring;
+    hipEvent_t ev[kSlots] = {};
+    ~CopyOut() {
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
+    }
+    // every part on the host when it returns; parts without a destination are skipped
+    hipError_t run(hipStream_t s, const std::vector<Part>& parts) {
+        size_t total = 0;
+        for (const Part& p : parts) total += p.dst ? p.bytes : 0;
+        hipError_t e = hipSuccess;
+        if (total < kSmall || (e = ready()) != hipSuccess) {  // (no pinned memory to be had: the plain copy)
+            (void)hipGetLastError();
+            e = hipSuccess;
+            for (const Part& p : parts)
+                if (p.dst && p.bytes && e == hipSuccess) e = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s);
+            const hipError_t w = hipStreamSynchronize(s);
+            return e != hipSuccess ? e : w;
+        }
+        std::vector<Part> pieces;
+        for (const Part& p : parts)
+            for (size_t o = 0; p.dst && o < p.bytes; o += kPiece)
+                pieces.push_back({static_cast<char*>(p.dst) + o, static_cast<const char*>(p.src) + o,
+                                  std::min(kPiece, p.bytes - o)});
+        const int n = (int)pieces.size();
+        char* base = static_cast<char*>(ring.p);
+        auto slot = [&](int i) { return base + (size_t)(i % kSlots) * kPiece; };
+        std::mutex m;
+        std::condition_variable cv;
+        int landed = 0, next = 0;       // pieces in their slots; the next one to copy out
+        std::vector<char> out(n, 0);    // copied out
+        bool stop = false;
+        auto drain_one = [&](std::unique_lock<std::mutex>& lk) {  // one landed piece to its place, if there is one
+            if (next >= landed) return false;
+            const int i = next++;
+            lk.unlock();
+            std::memcpy(pieces[i].dst, slot(i), pieces[i].bytes);
+            lk.lock();
+            out[i] = 1;
+            cv.notify_all();
+            return true;
+        };
+        std::vector<std::thread> th;
+        try {
+            for (int t = 0; t < std::min(kThreads, n / 2); ++t)
+                th.emplace_back([&] {
+                    std::unique_lock<std::mutex> lk(m);
+                    for (;;) {
+                        cv.wait(lk, [&] { return stop || next < landed; });
+                        if (!drain_one(lk) && stop) return;
+                    }
+                });
+        } catch (const std::system_error&) {  // fewer helpers, or none: this thread copies too
+        }
+        int issued = 0;
+        for (int i = 0; i < n && e == hipSuccess; ++i) {
+            for (; issued < n && issued < i + kSlots && e == hipSuccess; ++issued) {
+                if (issued >= kSlots) {  // the slot's piece before has to be out
+                    std::unique_lock<std::mutex> lk(m);
+                    const int before = issued - kSlots;
+                    if (issued > i && !out[before]) break;
+                    while (!out[before])
+                        if (!drain_one(lk)) cv.wait(lk, [&] { return out[before] || next < landed; });
+                }
+                e = hipMemcpyAsync(slot(issued), pieces[issued].src, pieces[issued].bytes, hipMemcpyDeviceToHost, s);
+                if (e == hipSuccess) e = hipEventRecord(ev[issued % kSlots], s);
+            }
+            if (e == hipSuccess) e = hipEventSynchronize(ev[i % kSlots]);
+            if (e == hipSuccess) {
+                std::lock_guard<std::mutex> lk(m);
+                landed = i + 1;
+                cv.notify_all();
+            }
+        }
+        if (e != hipSuccess) (void)hipStreamSynchronize(s);  // nothing writes the ring any more
+        {
+            std::unique_lock<std::mutex> lk(m);
+            while (drain_one(lk)) {
+            }
+            stop = true;
+            cv.notify_all();
+        }
+        for (auto& t : th) t.join();
+        return e;
+    }
+
+private:
+    hipError_t ready() {
+        hipError_t e = ring.reserve(kSlots * kPiece);
+        for (int i = 0; i < kSlots && e == hipSuccess; ++i)
+            if (!ev[i]) e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);
+        return e;
+    }
+};
+
 struct Error {
     int code;
 };
@@ -144,6 +254,7 @@ struct ProposalState {
     DevBuf<float> tprob, tshift;
     DevBuf<uint16_t> x, h[3], xT, hT[3], dzq, dzqT, daq, daqT;
     DevBuf<float> a[3], z, dz, dh;
+    DevBuf<float> pack;  // W1 without its padding columns
     DevBuf<int> bidx, bcell, bcnt;
     DevBuf<float> bprob, bshift, loss;
     DevBuf<unsigned> gmask;
@@ -277,7 +388,8 @@ struct rome_ctx {
     };
     // image preparation (rome_prepare_images)
     DevBuf<double> ip_img, ip_timg, ip_cbuf, ip_noise, ip_scal, ip_ctf, ip_fctf, ip_power;
-    DevBuf<double2> ip_F1, ip_F2, ip_fn, ip_fm;
+    DevBuf<double2> ip_F1, ip_F2;
+    DevBuf<double> ip_ft;
     std::vector<FftPlan> fft_plans;
     // projector grids built on the device (rome_fourier_map)
     DevBuf<double> fm_vol, fm_Mc, fm_corr, fm_pw, fm_cnt;
@@ -302,6 +414,7 @@ struct rome_ctx {
     // batched read-backs / uploads (pack kernel + pinned staging)
     DevBuf<unsigned char> rb_dev;
     PinnedBuf rb_host, up_host;
+    CopyOut copy_out;
     // last batch bookkeeping (parity hooks)
     int last_n = 0;
     long long last_blocks = 0, last_tasks = 0;
@@ -2619,11 +2732,8 @@ int rome_fourier_map(rome_ctx* ctx, int iclass, const double* vol, int do_griddi
     std::vector<double> pw(oriF), cnt(oriF);
     HIPCHK(hipMemcpyAsync(pw.data(), ctx->fm_pw.p, oriF * sizeof(double), hipMemcpyDeviceToHost, s));
     HIPCHK(hipMemcpyAsync(cnt.data(), ctx->fm_cnt.p, oriF * sizeof(double), hipMemcpyDeviceToHost, s));
-    if (corrected_map)
-        HIPCHK(hipMemcpyAsync(corrected_map, ctx->fm_corr.p, nvol * sizeof(double), hipMemcpyDeviceToHost, s));
-    if (grid_out)
-        HIPCHK(hipMemcpyAsync(grid_out, ctx->fm_grid64.p, ctx->grid_n * sizeof(double2), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    HIPCHK(ctx->copy_out.run(s, {{corrected_map, ctx->fm_corr.p, nvol * sizeof(double)},
+                                 {grid_out, ctx->fm_grid64.p, ctx->grid_n * sizeof(double2)}}));
     if (power_spectrum)  // radial average (src/reconstruct.cpp:213-221)
         for (int i = 0; i < oriF; ++i) power_spectrum[i] = cnt[i] < 1. ? 0. : pw[i] / cnt[i];
     ctx->have_ref[iclass] = 1;
@@ -2835,8 +2945,7 @@ int rome_reconstruct(rome_ctx* ctx, int iclass, const rome_recon_params* prm, co
         const double nf = ctx->is3d ? (double)ori * ori : 1.;
         for (int i = 0; i < oriF; ++i) tau2[i] = prm->tau2_fudge * (sp[i] / sp[ori + i] * nf / 2.);
     }
-    HIPCHK(hipMemcpyAsync(vol_out, ctx->rc_vol.p, nv * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    HIPCHK(ctx->copy_out.run(s, {{vol_out, ctx->rc_vol.p, nv * sizeof(double)}}));
     return ROME_OK;
 }
 
@@ -2871,8 +2980,9 @@ int rome_prepare_images(rome_ctx* ctx, const rome_raw_images* in, const rome_pre
         HIPCHK(ctx->ip_cbuf.reserve((size_t)n * n2));
         HIPCHK(ctx->ip_F1.reserve((size_t)n * nF));
         HIPCHK(ctx->ip_F2.reserve((size_t)n * nF));
-        HIPCHK(ctx->ip_fn.reserve((size_t)n * cF));
-        HIPCHK(ctx->ip_fm.reserve((size_t)n * cF));
+        // FP64 transforms as the host takes them: real and imaginary parts apart
+        const bool want64 = ho && (ho->fmask_re || ho->fmask_im || ho->fnomask_re || ho->fnomask_im);
+        if (want64) HIPCHK(ctx->ip_ft.reserve((size_t)4 * n * cF));
         HIPCHK(ctx->ip_fctf.reserve((size_t)n * cF));
         HIPCHK(ctx->ip_power.reserve((size_t)n * oriF));
         ImagePrepArgs a{};
@@ -2893,8 +3003,12 @@ int rome_prepare_images(rome_ctx* ctx, const rome_raw_images* in, const rome_pre
         a.cosine_width = p->width_mask_edge;
         a.F1 = ctx->ip_F1.p;
         a.F2 = ctx->ip_F2.p;
-        a.fnomask = ctx->ip_fn.p;
-        a.fmask = ctx->ip_fm.p;
+        if (want64) {
+            a.fmask_re = ctx->ip_ft.p;
+            a.fmask_im = a.fmask_re + (size_t)n * cF;
+            a.fnomask_re = a.fmask_im + (size_t)n * cF;
+            a.fnomask_im = a.fnomask_re + (size_t)n * cF;
+        }
         a.fnomask32 = dout && dout->fnomask ? (float2*)dout->fnomask + (size_t)i0 * cF : nullptr;
         a.fmask32 = dout && dout->fmask ? (float2*)dout->fmask + (size_t)i0 * cF : nullptr;
         a.power = ctx->ip_power.p;
@@ -2932,34 +3046,14 @@ int rome_prepare_images(rome_ctx* ctx, const rome_raw_images* in, const rome_pre
             HIPCHK(d2d(dout->old_offy, a.old_offy, n));
         }
         if (ho) {
-            std::vector<double2> fn, fm;
-            if (ho->fnomask_re || ho->fnomask_im) {
-                fn.resize((size_t)n * cF);
-                HIPCHK(hipMemcpyAsync(fn.data(), a.fnomask, fn.size() * sizeof(double2), hipMemcpyDeviceToHost, s));
-            }
-            if (ho->fmask_re || ho->fmask_im) {
-                fm.resize((size_t)n * cF);
-                HIPCHK(hipMemcpyAsync(fm.data(), a.fmask, fm.size() * sizeof(double2), hipMemcpyDeviceToHost, s));
-            }
-            auto d2h = [&](double* dst, const double* src, size_t cnt) -> hipError_t {
-                return dst ? hipMemcpyAsync(dst + (size_t)i0 * (cnt / n), src, cnt * sizeof(double),
-                                            hipMemcpyDeviceToHost, s)
-                           : hipSuccess;
+            auto part = [&](double* dst, const double* src, size_t per) {
+                return CopyOut::Part{dst ? dst + (size_t)i0 * per : nullptr, src, n * per * sizeof(double)};
             };
-            HIPCHK(d2h(ho->fctf, a.fctf, (size_t)n * cF));
-            HIPCHK(d2h(ho->highres_Xi2, a.hxi2, n));
-            HIPCHK(d2h(ho->power_img, a.power, (size_t)n * oriF));
-            HIPCHK(d2h(ho->old_offx, a.old_offx, n));
-            HIPCHK(d2h(ho->old_offy, a.old_offy, n));
-            HIPCHK(hipStreamSynchronize(s));
-            for (size_t q = 0; q < fn.size(); ++q) {
-                if (ho->fnomask_re) ho->fnomask_re[(size_t)i0 * cF + q] = fn[q].x;
-                if (ho->fnomask_im) ho->fnomask_im[(size_t)i0 * cF + q] = fn[q].y;
-            }
-            for (size_t q = 0; q < fm.size(); ++q) {
-                if (ho->fmask_re) ho->fmask_re[(size_t)i0 * cF + q] = fm[q].x;
-                if (ho->fmask_im) ho->fmask_im[(size_t)i0 * cF + q] = fm[q].y;
-            }
+            HIPCHK(ctx->copy_out.run(s, {part(ho->fmask_re, a.fmask_re, cF), part(ho->fmask_im, a.fmask_im, cF),
+                                         part(ho->fnomask_re, a.fnomask_re, cF), part(ho->fnomask_im, a.fnomask_im, cF),
+                                         part(ho->fctf, a.fctf, cF), part(ho->power_img, a.power, oriF),
+                                         part(ho->highres_Xi2, a.hxi2, 1), part(ho->old_offx, a.old_offx, 1),
+                                         part(ho->old_offy, a.old_offy, 1)}));
         }
         HIPCHK(hipStreamSynchronize(s));  // the staging buffers are reused by the next chunk
     }
@@ -3165,18 +3259,22 @@ int rome_proposal_get_params(rome_ctx* ctx, rome_proposal_params* o) {
     if (!P.ready) return fail(ctx, ROME_ERR_ARG, "rome_proposal_configure has not been called");
     HIPCHK(hipSetDevice(ctx->device));
     float* dst[8] = {o->W1, o->b1, o->W2, o->b2, o->W3, o->b3, o->W4, o->b4};
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    std::vector<CopyOut::Part> parts;
     for (int q = 0; q < 8; ++q) {
         if (!dst[q]) continue;
         const int l = q / 2;
         if (q & 1) {
-            HIPCHK(hipMemcpy(dst[q], P.w[q].p, (size_t)P.rows[l] * sizeof(float), hipMemcpyDeviceToHost));
+            parts.push_back({dst[q], P.w[q].p, (size_t)P.rows[l] * sizeof(float)});
+        } else if (l == 0) {  // without its padding columns, packed on the device (row by row over the link: 60 ms)
+            HIPCHK(P.pack.reserve((size_t)P.rows[0] * P.Fin));
+            HIPCHK(hipMemcpy2DAsync(P.pack.p, P.Fin * sizeof(float), P.w[q].p, P.cols[0] * sizeof(float),
+                                    P.Fin * sizeof(float), P.rows[0], hipMemcpyDeviceToDevice, ctx->stream));
+            parts.push_back({dst[q], P.pack.p, (size_t)P.rows[0] * P.Fin * sizeof(float)});
         } else {
-            const int c = l == 0 ? P.Fin : P.cols[l];
-            HIPCHK(hipMemcpy2D(dst[q], c * sizeof(float), P.w[q].p, P.cols[l] * sizeof(float), c * sizeof(float),
-                               P.rows[l], hipMemcpyDeviceToHost));
+            parts.push_back({dst[q], P.w[q].p, (size_t)P.rows[l] * P.cols[l] * sizeof(float)});
         }
     }
+    HIPCHK(ctx->copy_out.run(ctx->stream, parts));
     return ROME_OK;
 }
 

@@ -121,8 +121,12 @@ __global__ void k_ip_window(ImagePrepArgs a) {
     vm.x *= inv;
     vm.y *= inv;
     const size_t o = (size_t)img * cur * curF + q;
-    if (a.fnomask) a.fnomask[o] = vn;
-    if (a.fmask) a.fmask[o] = vm;
+    if (a.fmask_re) {
+        a.fnomask_re[o] = vn.x;
+        a.fnomask_im[o] = vn.y;
+        a.fmask_re[o] = vm.x;
+        a.fmask_im[o] = vm.y;
+    }
     if (a.fnomask32) a.fnomask32[o] = make_float2((float)vn.x, (float)vn.y);
     if (a.fmask32) a.fmask32[o] = make_float2((float)vm.x, (float)vm.y);
 }

@@ -318,8 +318,8 @@ struct ImagePrepArgs {
     double radius, cosine_width;     // mask: particle_diameter / (2 pixel_size), width_mask_edge
     const double2* F1;               // [n][ori][ori/2+1] unnormalised transform of the unmasked image
     const double2* F2;               // same, masked image
-    double2* fnomask;                // [n][cur][cur/2+1]
-    double2* fmask;
+    double *fmask_re, *fmask_im;     // [n][cur][cur/2+1], all four or none
+    double *fnomask_re, *fnomask_im;
     float2* fnomask32;
     float2* fmask32;
     double* power;                   // [n][ori/2+1]
