@@ -15,11 +15,11 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <limits>
 #include <mutex>
 #include <numeric>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -164,6 +164,7 @@ struct CopyOut {
             return true;
         };
         std::vector<std::thread> th;
+        th.reserve(kThreads);
         try {
             for (int t = 0; t < std::min(kThreads, n / 2); ++t)
                 th.emplace_back([&] {
@@ -173,7 +174,7 @@ struct CopyOut {
                         if (!drain_one(lk) && stop) return;
                     }
                 });
-        } catch (const std::system_error&) {  // fewer helpers, or none: this thread copies too
+        } catch (const std::exception&) {  // fewer helpers, or none: this thread copies too
         }
         int issued = 0;
         for (int i = 0; i < n && e == hipSuccess; ++i) {
@@ -372,6 +373,7 @@ struct rome_ctx {
     // binned backprojection
     static constexpr size_t kBinnedBytes = (size_t)40 << 30;  // slice values + records per batch
     DevBuf<float2> slice_val;
+    DevBuf<float> bp_work;  // partial bands of 2D grids
     DevBuf<double> slice_w;
     DevBuf<unsigned> bp_count, bp_off, bp_coff, bp_cursor;
     DevBuf<unsigned long long> bp_rec;
@@ -482,8 +484,12 @@ struct rome_ctx {
         const long long by_mem = (long long)(kPfineBytes / ((size_t)NORf * Pf * sizeof(float2)));
         return (int)std::max<long long>(1, std::min<long long>({(long long)Mtot, (long long)n * sig_cap, by_mem}));
     }
-    // slices of the binned backprojection a device-driven pool can hold
+    // slices of the binned / banded backprojection a device-driven pool can hold.  2D classes have few samples
+    // an image: 32 tasks each, or 512 MB, and the direct scatter for more
     long long dd_slice_cap(int n) const {
+        if (!is3d)
+            return std::min((long long)n * sig_cap * NORf,
+                            std::max<long long>(((long long)512 << 20) / (8 * Pf), (long long)n * 32 * NORf));
         const long long by_mem = (long long)(kBinnedBytes / ((size_t)Pf * 16));
         const long long by_index = (long long)(((1ULL << 32) - 1) / (unsigned long long)Pf);
         return std::max<long long>(1, std::min<long long>({(long long)n * sig_cap * NORf, by_mem, by_index}));
@@ -1562,13 +1568,14 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
         pp.wsum_prior_y = ctx->wsum_prior_y.p;
         pp.wsum_scalars = ctx->wsum_scalars.p;
         pp.wnorm = ctx->wnorm.p;
-        // 3D: slices to HBM, then the binned scatter (bounded by a slice buffer of kBinnedBytes).
-        // Device-driven pools: the slice buffer has a fixed capacity; the per-slice kernel and the binned
-        // scatter take a pool whose slices fit it, the direct scatter (k_post) one whose slices do not.
+        // Slices to HBM, then the binned scatter (3D; bounded by a slice buffer of kBinnedBytes) or the banded one (2D).
+        // Device-driven pools: the slice buffer has a fixed capacity; the binned and banded forms take a pool
+        // whose slices fit it, the direct scatter (k_post) one whose slices do not.
         long long S = ntasks * NOR;
         const long long slice_cap = ctx->dd_slice_cap(n);
-        if (dd) S = post_slices_supported(NOR, NOT, ctx->Pf, ctx->is3d) ? slice_cap : 0;
-        const bool binned = ctx->is3d && S > 0 && (unsigned long long)S * ctx->Pf < (1ULL << 32) &&
+        const bool by_slice = post_slices_supported(NOR, NOT, ctx->Pf, ctx->is3d);
+        if (dd) S = by_slice || !ctx->is3d ? slice_cap : 0;
+        const bool binned = S > 0 && (!ctx->is3d || (unsigned long long)S * ctx->Pf < (1ULL << 32)) &&
                             (size_t)S * ctx->Pf * 16 <= rome_ctx::kBinnedBytes;
         if (dd) {
             pp.ntask_dev = ctx->task_off.p + n;
@@ -1588,8 +1595,10 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
         hipError_t pe = hipErrorNotSupported;
         if (dd) {
             HIPCHK(launch_fill32(s, ctx->wnorm.p, 0u, 2 * (size_t)n));
-            if (binned)
+            if (binned && by_slice)
                 HIPCHK(launch_post_slices(s, ntasks, NOR, NOT, pp, ctx->persist_blocks(2), ctx->guess_tasks(n, ntasks)));
+            else if (binned)
+                HIPCHK(launch_post(s, n, NOR, NOT, pp));
             PostArgs pd = pp;  // the direct scatter of pools past the slice buffer
             pd.slice_val = nullptr;
             pd.slice_w = nullptr;
@@ -1614,16 +1623,18 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
             ba.c = ctx->cgrid;
             ba.r_max = ctx->r_max;
             ba.grid_stride = ctx->grid_n;
-            ba.nbx = (ctx->padF + 7) / 8;
-            ba.nby = (ctx->pad + 7) / 8;
-            ba.nbz = (ctx->pad + 7) / 8;
-            ba.nb_class = ba.nbx * ba.nby * ba.nbz;
-            const size_t nb = (size_t)ba.nb_class * ctx->K;
-            HIPCHK(ctx->bp_count.reserve(nb));
-            HIPCHK(ctx->bp_off.reserve(nb + 1));
-            HIPCHK(ctx->bp_coff.reserve(nb + 1));
-            HIPCHK(ctx->bp_cursor.reserve(nb));
-            HIPCHK(sized(ctx->bp_rec, (size_t)S * ctx->Pf));
+            if (ctx->is3d) {
+                ba.nbx = (ctx->padF + 7) / 8;
+                ba.nby = (ctx->pad + 7) / 8;
+                ba.nbz = (ctx->pad + 7) / 8;
+                ba.nb_class = ba.nbx * ba.nby * ba.nbz;
+                const size_t nb = (size_t)ba.nb_class * ctx->K;
+                HIPCHK(ctx->bp_count.reserve(nb));
+                HIPCHK(ctx->bp_off.reserve(nb + 1));
+                HIPCHK(ctx->bp_coff.reserve(nb + 1));
+                HIPCHK(ctx->bp_cursor.reserve(nb));
+                HIPCHK(sized(ctx->bp_rec, (size_t)S * ctx->Pf));
+            }
             ba.task_img = ctx->task_img.p;
             ba.task_m = ctx->task_m.p;
             ba.Ai_fine = ctx->Ai_f.p;
@@ -1644,7 +1655,13 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
                 ba.abort = ctx->pool_flags.p;
             }
             stage_begin(ctx, 10);
-            HIPCHK(launch_backproject_binned(s, S, ba, ctx->persist_blocks(3)));
+            if (ctx->is3d) {
+                HIPCHK(launch_backproject_binned(s, S, ba, ctx->persist_blocks(3)));
+            } else {
+                const BandPlan plan = bp_band_plan(n, ctx->K, ctx->pad, ctx->padF, ctx->n_cu);
+                HIPCHK(ctx->bp_work.reserve(plan.work));
+                HIPCHK(launch_backproject_bands(s, S, ba, plan, ctx->bp_work.p));
+            }
             stage_end(ctx, 10);
         }
     } else {

@@ -264,7 +264,7 @@ struct PostArgs {
     double* wsum_prior_y;
     double* wsum_scalars;       // [4]
     double* wnorm;              // [n]
-    // binned 3D backprojection: slices go to HBM instead of the grids (null: direct scatter)
+    // binned / banded backprojection: slices go to HBM instead of the grids (null: direct scatter)
     float2* slice_val;          // [ntask * NOR][Pf]
     double* slice_w;            // [ntask * NOR]
     // device-driven pools (null otherwise): the task total on the device, the slice buffer's capacity
@@ -526,6 +526,13 @@ hipError_t launch_store_sums(hipStream_t s, const StoreArgs& a);
 // With a.ntask_dev (device-driven pools) S is read on the device and persist_blocks blocks stride over
 // the slices (one pixel block per grid row) and over the brick chunks.
 hipError_t launch_backproject_binned(hipStream_t s, long long S, const BpArgs& a, int persist_blocks = 0);
+// 2D: bands of grid rows accumulated in LDS, the slices of a class split over parts blocks per band
+struct BandPlan {
+    int rows, bands, parts;
+    size_t work;  // floats of partial sums (0: one part, added to the grids directly)
+};
+BandPlan bp_band_plan(int n, int K, int pad, int padF, int n_cu);
+hipError_t launch_backproject_bands(hipStream_t s, long long S, const BpArgs& a, const BandPlan& plan, float* work);
 // M-step reconstruction (reconstruct.hip)
 hipError_t rc_fold(hipStream_t s, double2* data, double* weight, int Dz, int P, int PF);
 hipError_t rc_decenter_real(hipStream_t s, const double* cen, double* out, int Dz, int P, int PF, int max_r2);
