@@ -1207,7 +1207,7 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
         stage_begin(ctx, 2);
         if (prec == ROME_PREC_FP32) {
             // an L2-resident slice of the rotation operand per XCD: about 2.5 MB of its 4 MB L2
-            const int nbm = ctx->Mpad / 128;
+            const int nbm = (M + 127) / 128;
             GemmArgs ga{ctx->FcT.p, ctx->WcT.p, ctx->At.p, Ep, ctx->valid.p, ctx->emin_key.p, Kdim, ctx->Mpad, Npad, M,
                         Ncols, T, gemm_sub_band(nbm, (size_t)128 * Kdim * 4, (size_t)5 << 19), L};
             HIPCHK(launch_coarse_gemm(s, ga));

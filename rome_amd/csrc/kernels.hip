@@ -314,6 +314,91 @@ __global__ void k_fct_norm(const float* __restrict__ FcT, int Pc, int Pc_pad, in
     Qc[i] = q;
 }
 
+// 128 x 128 tile of C = A^T B (A: rows k of lda floats, B of ldb) over nk chunks of 16 k: 4 waves (2 x 2), each 2 x 2
+// blocks of v_mfma_f32_32x32x2f32.  Two LDS stages filled from registers; the fragments of a step of two k are read
+// while the step before multiplies, the next chunk is written to LDS among the MFMAs of the last steps but one, and the
+// barrier and the next chunk's first fragments stand inside the last step's, so that the matrix cores do not wait
+// for LDS.  (Reading each step's fragments right before its MFMAs, two waves a SIMD left the matrix cores idle a third of the time: with three waves (128^2 x 250 images,
+// 18432 rotations x 81 shifts) 3460 -> 3207-3319 us at 2.1 GHz under this load; 976 -> 700 us for 360 x 29000 x 3304,
+// most of that from the padding rows no longer multiplied.)
+// smem: 4 * 16 * 128 floats, 16-byte aligned; every thread of the 256 calls it, Ag / Bg already offset to its
+// float4 of the chunk's rows tid / 32 and 8 further.
+DEV void mma_tile_f32(const float* __restrict__ Ag, const float* __restrict__ Bg, size_t lda, size_t ldb, int nk,
+                      float* smem, int tid, f16v (&acc)[2][2]) {
+    constexpr int BM = 128, BK = 16;
+    typedef float Stage[BK][BM];
+    Stage* As = reinterpret_cast<Stage*>(smem);
+    Stage* Bs = reinterpret_cast<Stage*>(smem + 2 * BK * BM);
+    const int lane = tid & 63, wave = tid >> 6;
+    const int lr = tid >> 5, lc = (tid & 31) * 4;
+    const int fk = lane >> 5, fa = (wave >> 1) * 64 + (lane & 31), fb = (wave & 1) * 64 + (lane & 31);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    const size_t a8 = 8 * lda, b8 = 8 * ldb, astep = BK * lda, bstep = BK * ldb;
+    // staging in named registers (arrays of them end up in scratch)
+    float4 ra0 = *reinterpret_cast<const float4*>(Ag), ra1 = *reinterpret_cast<const float4*>(Ag + a8);
+    float4 rb0 = *reinterpret_cast<const float4*>(Bg), rb1 = *reinterpret_cast<const float4*>(Bg + b8);
+    auto stage = [&](int b) {
+        *reinterpret_cast<float4*>(&As[b][lr][lc]) = ra0;
+        *reinterpret_cast<float4*>(&As[b][lr + 8][lc]) = ra1;
+        *reinterpret_cast<float4*>(&Bs[b][lr][lc]) = rb0;
+        *reinterpret_cast<float4*>(&Bs[b][lr + 8][lc]) = rb1;
+    };
+    float av[2][2], bv[2][2];  // fragments of two steps
+    auto frag = [&](int f, int b, int kk) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) av[f][i] = As[b][kk + fk][fa + i * 32];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) bv[f][j] = Bs[b][kk + fk][fb + j * 32];
+    };
+    auto mma = [&](int f, int i) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[f][i], bv[f][j], acc[i][j], 0, 0, 0);
+    };
+    stage(0);
+    __syncthreads();
+    frag(0, 0, 0);
+    for (int kc = 0; kc < nk; ++kc) {
+        const int cur = kc & 1;
+        const bool more = kc + 1 < nk;
+        if (more) {
+            Ag += astep;
+            Bg += bstep;
+            ra0 = *reinterpret_cast<const float4*>(Ag);
+            ra1 = *reinterpret_cast<const float4*>(Ag + a8);
+            rb0 = *reinterpret_cast<const float4*>(Bg);
+            rb1 = *reinterpret_cast<const float4*>(Bg + b8);
+        }
+#pragma unroll
+        for (int st = 0; st < BK / 2; ++st) {
+            const int f = st & 1;
+            if (st < BK / 2 - 1) {
+                frag(f ^ 1, cur, 2 * st + 2);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            mma(f, 0);
+            if (st == BK / 2 - 2 && more) {
+                __builtin_amdgcn_sched_barrier(0);
+                stage(cur ^ 1);  // last read before the barrier of the chunk before
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (st == BK / 2 - 1 && more) {
+                __builtin_amdgcn_sched_barrier(0);
+                __syncthreads();
+                frag(f ^ 1, cur ^ 1, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            mma(f, 1);
+        }
+    }
+    __syncthreads();  // the stages may be reused
+}
+
 // A-term as an FP32 MFMA GEMM: At[img][m] = 0.5 * sum_p Qc[p][m] * MC2cT[p][img] (rows padded to Mpad,
 // zero beyond Mtot).  128 rotations x 128 images per block of 4 waves (2 x 2, each 2 x 2 blocks of
 // v_mfma_f32_32x32x2f32), BK = 16, two LDS stages: the rotation table is read once per 128 images.
@@ -321,60 +406,14 @@ __global__ __launch_bounds__(256) void k_coarse_aterm(const float* __restrict__ 
                                                       const float* __restrict__ MC2cT, int ldn, int n,
                                                       float* __restrict__ At) {
     constexpr int BM = 128, BN = 128, BK = 16;
-    __shared__ __attribute__((aligned(16))) float As[2][BK][BM];
-    __shared__ __attribute__((aligned(16))) float Bs[2][BK][BN];
+    __shared__ __attribute__((aligned(16))) float smem[4 * BK * BM];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
     const int lr = tid >> 5, lc = (tid & 31) * 4;  // rows lr and lr + 8 of a 16 x 128 chunk
     f16v acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    const float* Ag = Qc + (size_t)lr * Mpad + m0 + lc;
-    const float* Bg = MC2cT + (size_t)lr * ldn + n0 + lc;
-    const size_t a8 = (size_t)8 * Mpad, b8 = (size_t)8 * ldn;
-    float4 ra0 = *reinterpret_cast<const float4*>(Ag), ra1 = *reinterpret_cast<const float4*>(Ag + a8);
-    float4 rb0 = *reinterpret_cast<const float4*>(Bg), rb1 = *reinterpret_cast<const float4*>(Bg + b8);
-    *reinterpret_cast<float4*>(&As[0][lr][lc]) = ra0;
-    *reinterpret_cast<float4*>(&As[0][lr + 8][lc]) = ra1;
-    *reinterpret_cast<float4*>(&Bs[0][lr][lc]) = rb0;
-    *reinterpret_cast<float4*>(&Bs[0][lr + 8][lc]) = rb1;
-    __syncthreads();
-    const int nk = Kq / BK;
-    for (int kc = 0; kc < nk; ++kc) {
-        const int cur = kc & 1;
-        if (kc + 1 < nk) {
-            const float* an = Ag + (size_t)(kc + 1) * BK * Mpad;
-            const float* bn = Bg + (size_t)(kc + 1) * BK * ldn;
-            ra0 = *reinterpret_cast<const float4*>(an);
-            ra1 = *reinterpret_cast<const float4*>(an + a8);
-            rb0 = *reinterpret_cast<const float4*>(bn);
-            rb1 = *reinterpret_cast<const float4*>(bn + b8);
-        }
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 2) {
-            float av[2], bv[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) av[i] = As[cur][kk + (lane >> 5)][wm * 64 + i * 32 + (lane & 31)];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) bv[j] = Bs[cur][kk + (lane >> 5)][wn * 64 + j * 32 + (lane & 31)];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i][j], 0, 0, 0);
-        }
-        if (kc + 1 < nk) {
-            *reinterpret_cast<float4*>(&As[cur ^ 1][lr][lc]) = ra0;
-            *reinterpret_cast<float4*>(&As[cur ^ 1][lr + 8][lc]) = ra1;
-            *reinterpret_cast<float4*>(&Bs[cur ^ 1][lr][lc]) = rb0;
-            *reinterpret_cast<float4*>(&Bs[cur ^ 1][lr + 8][lc]) = rb1;
-        }
-        __syncthreads();
-    }
+    mma_tile_f32(Qc + (size_t)lr * Mpad + m0 + lc, MC2cT + (size_t)lr * ldn + n0 + lc, Mpad, ldn,
+                 m0 < Mtot ? Kq / BK : 0 /* a tile of padding rows: zeros */, smem, tid, acc);
     // lane: column img = n0 + wn*64 + j*32 + lane%32, rows m0 + wm*64 + i*32 + 8q + 4(lane/32) + u
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -395,17 +434,62 @@ __global__ __launch_bounds__(256) void k_coarse_aterm(const float* __restrict__ 
     }
 }
 
+// The same product (same MFMA, same ascending k per element: the same values) by one wave per 32 x 32 tile straight from
+// L2, the next 16 k in flight: for pools and tables of fewer 128 x 128 tiles than CUs, whose blocks would be alone on
+// theirs with a round trip per 16 k (360 rotations x 1000 images x 1664 k: 124 -> 66 us).
+__global__ __launch_bounds__(64) void k_coarse_aterm_wave(const float* __restrict__ Qc, int Kq, int Mtot, int Mpad,
+                                                          const float* __restrict__ MC2cT, int ldn, int n,
+                                                          float* __restrict__ At) {
+    constexpr int U = 8;  // steps of two k in flight
+    const int lane = threadIdx.x, m0 = blockIdx.x * 32, n0 = blockIdx.y * 32;
+    const float* A = Qc + (size_t)(lane >> 5) * Mpad + m0 + (lane & 31);
+    const float* B = MC2cT + (size_t)(lane >> 5) * ldn + n0 + (lane & 31);
+    f16v acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    if (m0 < Mtot) {
+        float av[U], bv[U], an[U], bn[U];
+        auto load = [&](float(&x)[U], float(&y)[U], int k) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                x[u] = A[(size_t)(k + 2 * u) * Mpad];
+                y[u] = B[(size_t)(k + 2 * u) * ldn];
+            }
+        };
+        auto mul = [&](const float(&x)[U], const float(&y)[U]) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[u], y[u], acc, 0, 0, 0);
+        };
+        load(av, bv, 0);
+        for (int k = 0; k < Kq; k += 4 * U) {  // Kq is a multiple of 16 = 2 U
+            if (k + 2 * U < Kq) load(an, bn, k + 2 * U);
+            mul(av, bv);
+            if (k + 2 * U >= Kq) break;
+            if (k + 4 * U < Kq) load(av, bv, k + 4 * U);
+            mul(an, bn);
+        }
+    }
+    const int img = n0 + (lane & 31);
+    if (img >= n) return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int m = m0 + 8 * q + 4 * (lane >> 5);
+        float4 v;
+        v.x = m < Mtot ? 0.5f * acc[4 * q] : 0.f;
+        v.y = m + 1 < Mtot ? 0.5f * acc[4 * q + 1] : 0.f;
+        v.z = m + 2 < Mtot ? 0.5f * acc[4 * q + 2] : 0.f;
+        v.w = m + 3 < Mtot ? 0.5f * acc[4 * q + 3] : 0.f;
+        *reinterpret_cast<float4*>(&At[(size_t)img * Mpad + m]) = v;
+    }
+}
+
 // ------------------------------------------------------------------ coarse cross term (K2), FP32 MFMA
 // C[m][j] = sum_kk FcT[kk][m] * WcT[kk][j];  E[img][m][t] = At[img][m] - C[m][img*T+t].
 // 256 threads, 128x128 tile, BK = 16, v_mfma_f32_32x32x2f32, LDS double buffer.
 template <bool LIST>
-__global__ __launch_bounds__(256) void k_coarse_gemm(GemmArgs a) {
+__global__ __launch_bounds__(256, LIST ? 3 : 2) void k_coarse_gemm(GemmArgs a) {
     constexpr int BM = 128, BN = 128, BK = 16;
-    constexpr int kOps = 2 * 2 * BK * BM;  // operand stages
-    __shared__ __attribute__((aligned(16))) float smem[kOps];
-    typedef float Stage[BK][BM];
-    Stage* As = reinterpret_cast<Stage*>(smem);
-    Stage* Bs = reinterpret_cast<Stage*>(smem + 2 * BK * BM);
+    __shared__ __attribute__((aligned(16))) float smem[4 * BK * BM];  // operand stages
     __shared__ int slot_min[epi_slots<BN>()];
     __shared__ int slot_vb[LIST ? epi_slots<BN>() : 1];
     __shared__ float slot_lim[LIST ? epi_slots<BN>() : 1];
@@ -413,62 +497,14 @@ __global__ __launch_bounds__(256) void k_coarse_gemm(GemmArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     int bm, bn;
-    gemm_tile(blockIdx.x, a.Mpad / BM, a.Npad / BN, a.sband, bm, bn);
+    gemm_tile(blockIdx.x, (a.Mtot + BM - 1) / BM, a.Npad / BN, a.sband, bm, bn);
     const int m0 = bm * BM, n0 = bn * BN;
     if (n0 >= a.Ncols) return;  // a tile of padding columns only (block-uniform, before any barrier)
     // global load mapping: 16 rows x 128 cols = 2048 floats = 512 float4 -> 2 per thread per operand
     const int lr = tid >> 5, lc = (tid & 31) * 4;  // rows lr and lr+8
     f16v acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-    const int nk = a.K / BK;
-    // staging in named registers (arrays of them end up in scratch)
-    const float* Ag = a.A + (size_t)lr * a.Mpad + m0 + lc;
-    const float* Bg = a.B + (size_t)lr * a.Npad + n0 + lc;
-    const size_t a8 = (size_t)8 * a.Mpad, b8 = (size_t)8 * a.Npad;
-    const size_t astep = (size_t)BK * a.Mpad, bstep = (size_t)BK * a.Npad;
-    float4 ra0 = *reinterpret_cast<const float4*>(Ag), ra1 = *reinterpret_cast<const float4*>(Ag + a8);
-    float4 rb0 = *reinterpret_cast<const float4*>(Bg), rb1 = *reinterpret_cast<const float4*>(Bg + b8);
-    *reinterpret_cast<float4*>(&As[0][lr][lc]) = ra0;
-    *reinterpret_cast<float4*>(&As[0][lr + 8][lc]) = ra1;
-    *reinterpret_cast<float4*>(&Bs[0][lr][lc]) = rb0;
-    *reinterpret_cast<float4*>(&Bs[0][lr + 8][lc]) = rb1;
-    __syncthreads();
-    for (int kc = 0; kc < nk; ++kc) {
-        const int cur = kc & 1;
-        if (kc + 1 < nk) {
-            const float* an = Ag + (size_t)(kc + 1) * astep;
-            const float* bnp = Bg + (size_t)(kc + 1) * bstep;
-            ra0 = *reinterpret_cast<const float4*>(an);
-            ra1 = *reinterpret_cast<const float4*>(an + a8);
-            rb0 = *reinterpret_cast<const float4*>(bnp);
-            rb1 = *reinterpret_cast<const float4*>(bnp + b8);
-        }
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 2) {
-            float av[2], bv[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) av[i] = As[cur][kk + (lane >> 5)][wm * 64 + i * 32 + (lane & 31)];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) bv[j] = Bs[cur][kk + (lane >> 5)][wn * 64 + j * 32 + (lane & 31)];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i][j], 0, 0, 0);
-        }
-        if (kc + 1 < nk) {
-            *reinterpret_cast<float4*>(&As[cur ^ 1][lr][lc]) = ra0;
-            *reinterpret_cast<float4*>(&As[cur ^ 1][lr + 8][lc]) = ra1;
-            *reinterpret_cast<float4*>(&Bs[cur ^ 1][lr][lc]) = rb0;
-            *reinterpret_cast<float4*>(&Bs[cur ^ 1][lr + 8][lc]) = rb1;
-        }
-        __syncthreads();
-    }
+    mma_tile_f32(a.A + (size_t)lr * a.Mpad + m0 + lc, a.B + (size_t)lr * a.Npad + n0 + lc, a.Mpad, a.Npad, a.K / BK, smem,
+                 tid, acc);
     if constexpr (LIST)
         gemm_epilogue_list<false, 2, 2, BN>(acc, ContigRows{m0 + wm * 64, lane >> 5}, n0 + wn * 64, n0, lane, tid, a.At, nullptr,
                                             a.emin_key, a.Mtot, a.Mpad, a.Ncols, a.T, a.list, slot_min, slot_vb,
@@ -1587,14 +1623,17 @@ hipError_t launch_coarse_aterm(hipStream_t s, int n, const float* Qc, int Kq, in
                                int ldn, float* At) {
     if (n <= 0) return hipSuccess;
     if (Kq % 16 || Mpad % 128 || ldn % 128 || ldn < n) return hipErrorInvalidValue;
-    dim3 grid(Mpad / 128, ldn / 128);
-    k_coarse_aterm<<<grid, 256, 0, s>>>(Qc, Kq, Mtot, Mpad, MC2cT, ldn, n, At);
+    const dim3 grid(Mpad / 128, ldn / 128);
+    if (grid.x * grid.y < 256)
+        k_coarse_aterm_wave<<<dim3(Mpad / 32, (n + 31) / 32), 64, 0, s>>>(Qc, Kq, Mtot, Mpad, MC2cT, ldn, n, At);
+    else
+        k_coarse_aterm<<<grid, 256, 0, s>>>(Qc, Kq, Mtot, Mpad, MC2cT, ldn, n, At);
     LAUNCH_CHECK();
     return hipSuccess;
 }
 
 hipError_t launch_coarse_gemm(hipStream_t s, const GemmArgs& a) {
-    const int tiles = (a.Mpad / 128) * (a.Npad / 128);
+    const int tiles = ((a.Mtot + 127) / 128) * (a.Npad / 128);  // (Mpad is whole 256-row tiles)
     if (a.list.count) k_coarse_gemm<true><<<tiles, 256, 0, s>>>(a);
     else if (a.E) k_coarse_gemm<false><<<tiles, 256, 0, s>>>(a);
     else return hipErrorInvalidValue;
