@@ -6,14 +6,15 @@
 //             V_s(p) = sum_t w_t/sumw * Minv CTF X_nomask(p) S_t(p) (float2 [S][Pf]) and
 //             W_s = sum_t w_t/sumw (double [S]; 0: the slice has no significant sample).
 //   count   : every (slice, pixel) with a positive weight, inside r_max -> trilinear base voxel ->
-//             brick (8x8x8 base voxels of one class grid); counts per brick, first gathered per
+//             brick (16x8x4 base voxels of one class grid); counts per brick, first gathered per
 //             block in an LDS hash table (one global atomic per distinct brick of the block).
-//   scan    : exclusive prefix sums of the counts and of the chunks (kChunk records) per brick.
+//   scan    : exclusive prefix sums of the counts and of the chunks (kChunk records) per brick, the brick of
+//             every chunk.
 //   fill    : records (slice << 32 | pixel) grouped by brick; ranges reserved per distinct brick
 //             of the block as in count.
 //   brick   : one block per chunk of a brick's records (bricks near the origin, crossed by nearly
 //             every slice, hold hundreds of thousands): the records' 8 corners accumulate in a
-//             9x9x9 LDS box (base voxels plus the +1 corner halo), then each non-zero voxel goes to
+//             17x9x5 LDS box (base voxels plus the +1 corner halo), then each non-zero voxel goes to
 //             the grids with one atomic per component.  Corner weights and values are computed
 //             exactly as the direct scatter computes them; only the order of the FP32 additions
 //             differs.
@@ -32,8 +33,8 @@ namespace rome {
 
 namespace {
 
-constexpr int kBrick = 8, kBox = kBrick + 1, kBox3 = kBox * kBox * kBox;
-constexpr unsigned kChunk = 1024;  // records per brick block (41 KB of LDS: three blocks per CU)
+constexpr int kBoxX = kBrickX + 1, kBoxY = kBrickY + 1, kBoxZ = kBrickZ + 1, kBox3 = kBoxX * kBoxY * kBoxZ;
+constexpr unsigned kChunk = 1024;  // records per brick block
 constexpr int kHash = 512;         // LDS hash slots for the <= 256 bricks of one count / fill block
 
 // Slot of brick b in the block's hash table (keys b + 1, 0 = empty; linear probing).  At most 256
@@ -61,8 +62,8 @@ struct Sample {
 DEV bool bp_sample(const BpArgs& a, long long s, int p, Sample& out) {
     const double wsl = a.slice_w[s];
     if (!(wsl > 0.)) return false;
-    const long long q = s / a.NOR;
-    const int o = (int)(s - q * a.NOR);
+    const unsigned q = (unsigned)s / (unsigned)a.NOR;  // slices are counted in 32 bits (records hold them so)
+    const int o = (int)((unsigned)s - q * (unsigned)a.NOR);
     const int img = a.task_img[q], m = a.task_m[q];
     const int xy = a.f_xy[p];
     const int x = px_x(xy), y = px_y(xy);
@@ -78,7 +79,7 @@ DEV bool bp_sample(const BpArgs& a, long long s, int p, Sample& out) {
 
 // brick of the base voxel: class-major, then z, y, x in bricks of 8 (grid coordinates are >= 0)
 DEV int brick_of(const BpArgs& a, const Sample& sm) {
-    const int bx = sm.c.x0 / kBrick, by = sm.c.y0 / kBrick, bz = sm.c.z0 / kBrick;
+    const int bx = sm.c.x0 / kBrickX, by = sm.c.y0 / kBrickY, bz = sm.c.z0 / kBrickZ;
     return sm.k * a.nb_class + (bz * a.nby + by) * a.nbx + bx;
 }
 
@@ -123,65 +124,65 @@ __global__ __launch_bounds__(256) void k_bp_count(BpArgs a, long long S_host) {
     }
 }
 
-// Exclusive scans of count[0..nb) into off[0..nb] and of the chunks per brick into coff[0..nb];
-// cursor cleared.  One block of 1024 threads over tiles of 4096 bricks: four consecutive bricks per
-// thread, wave scans by shuffles, the 16 wave totals through LDS, a running carry between tiles.
-__global__ __launch_bounds__(1024) void k_bp_scan(const unsigned* __restrict__ count, int nb,
-                                                  unsigned* __restrict__ off, unsigned* __restrict__ coff,
-                                                  unsigned* __restrict__ cursor) {
-    __shared__ unsigned wa[16], wc[16];
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    unsigned carry = 0u, ccarry = 0u;
-    for (int t0 = 0; t0 < nb; t0 += 4096) {
-        const int b = t0 + 4 * tid;
-        unsigned c[4], cc[4], loc = 0u, cloc = 0u;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            c[j] = b + j < nb ? count[b + j] : 0u;
-            cc[j] = (c[j] + kChunk - 1) / kChunk;
-            loc += c[j];
-            cloc += cc[j];
-        }
-        unsigned in = loc, cin = cloc;
-        for (int o = 1; o < 64; o <<= 1) {
-            const unsigned v = __shfl_up(in, o, 64), cv = __shfl_up(cin, o, 64);
-            if (lane >= o) {
-                in += v;
-                cin += cv;
-            }
-        }
-        if (lane == 63) {
-            wa[wid] = in;
-            wc[wid] = cin;
-        }
-        __syncthreads();
-        unsigned pre = 0u, cpre = 0u, tot = 0u, ctot = 0u;
-        for (int w = 0; w < 16; ++w) {
-            if (w < wid) {
-                pre += wa[w];
-                cpre += wc[w];
-            }
-            tot += wa[w];
-            ctot += wc[w];
-        }
-        unsigned run = carry + pre + in - loc, crun = ccarry + cpre + cin - cloc;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (b + j < nb) {
-                off[b + j] = run;
-                coff[b + j] = crun;
-                cursor[b + j] = 0u;
-            }
-            run += c[j];
-            crun += cc[j];
-        }
-        carry += tot;
-        ccarry += ctot;
-        __syncthreads();  // the wave totals are rewritten by the next tile
+// Exclusive scans of count[0..nb) into off[0..nb] and of the chunks per brick into coff[0..nb], the brick of every
+// chunk into ck_brick, cursor cleared: k_bp_sums leaves the totals of blocks of 1024 bricks, each block of k_bp_scan adds
+// up the totals before its own and scans its bricks.  (One block over all bricks, tile by tile: 78 us for 74 k bricks,
+// 10 us now.)
+constexpr int kScanBlock = 1024;  // bricks and threads per block
+__global__ __launch_bounds__(kScanBlock) void k_bp_sums(const unsigned* __restrict__ count, int nb,
+                                                        unsigned* __restrict__ sums) {
+    __shared__ unsigned red[kScanBlock / 64];
+    const int b = blockIdx.x * kScanBlock + threadIdx.x;
+    const unsigned c = b < nb ? count[b] : 0u;
+    const unsigned t = block_reduce(c, [](unsigned x, unsigned y) { return x + y; }, red);
+    const unsigned ct = block_reduce((c + kChunk - 1) / kChunk, [](unsigned x, unsigned y) { return x + y; }, red);
+    if (threadIdx.x == 0) {
+        sums[2 * blockIdx.x] = t;
+        sums[2 * blockIdx.x + 1] = ct;
     }
-    if (tid == 0) {
-        off[nb] = carry;
-        coff[nb] = ccarry;
+}
+
+__global__ __launch_bounds__(kScanBlock) void k_bp_scan(const unsigned* __restrict__ count, int nb,
+                                                        const unsigned* __restrict__ sums, unsigned* __restrict__ off,
+                                                        unsigned* __restrict__ coff, unsigned* __restrict__ cursor,
+                                                        unsigned* __restrict__ ck_brick) {
+    constexpr int NW = kScanBlock / 64;
+    __shared__ unsigned wa[NW], wc[NW], red[NW];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, b = blockIdx.x * kScanBlock + tid;
+    unsigned pre = 0u, cpre = 0u;  // of the blocks before
+    for (int q = tid; q < (int)blockIdx.x; q += kScanBlock) {
+        pre += sums[2 * q];
+        cpre += sums[2 * q + 1];
+    }
+    const unsigned c = b < nb ? count[b] : 0u, cc = (c + kChunk - 1) / kChunk;
+    pre = block_reduce(pre, [](unsigned x, unsigned y) { return x + y; }, red);
+    cpre = block_reduce(cpre, [](unsigned x, unsigned y) { return x + y; }, red);
+    unsigned in = c, cin = cc;
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned v = __shfl_up(in, o, 64), cv = __shfl_up(cin, o, 64);
+        if (lane >= o) {
+            in += v;
+            cin += cv;
+        }
+    }
+    if (lane == 63) {
+        wa[wid] = in;
+        wc[wid] = cin;
+    }
+    __syncthreads();
+    for (int w = 0; w < wid; ++w) {
+        pre += wa[w];
+        cpre += wc[w];
+    }
+    if (b >= nb) return;
+    const unsigned o0 = pre + in - c, c0 = cpre + cin - cc;
+    off[b] = o0;
+    coff[b] = c0;
+    cursor[b] = 0u;
+    for (unsigned q = 0; q < cc; ++q) ck_brick[c0 + q] = (unsigned)b;
+    if (b == nb - 1) {
+        off[nb] = o0 + c;
+        coff[nb] = c0 + cc;
     }
 }
 
@@ -225,28 +226,25 @@ __global__ __launch_bounds__(256) void k_bp_fill(BpArgs a, long long S_host) {
 // base voxel in LDS, each thread sums the 8 corner contributions of the records of its base voxels in
 // registers, then the corners are added to the box in 8 passes, one corner offset per pass, in which
 // distinct base voxels reach distinct box voxels.
-DEV void bp_brick_one(const BpArgs& a, int nb, unsigned ck) {
-    constexpr int kVox = kBrick * kBrick * kBrick;  // base voxels of a brick
-    __shared__ float box[3][kBox3];
-    __shared__ unsigned vcnt[kVox], voff[kVox + 1];
+DEV void bp_brick_one(const BpArgs& a, unsigned ck) {
+    constexpr int kVox = kBrickX * kBrickY * kBrickZ;  // base voxels of a brick
+    static_assert(kVox == 512, "two base voxels a thread, eight a lane of the scan");
+    // exactly 32 KB: five blocks per CU.  The records' fx, fy, fz, value re, value im (mirror applied) and weight; the
+    // box once they are summed.
+    __shared__ float rec_f[6][kChunk];
+    __shared__ unsigned vcnt[kVox], voff[kVox];
     __shared__ unsigned short order[kChunk], vox[kChunk];
-    __shared__ float rec_f[6][kChunk];  // fx, fy, fz, value re, value im (mirror applied), weight
+    typedef float Box[kBox3];
+    Box* box = reinterpret_cast<Box*>(&rec_f[0][0]);
+    static_assert(3 * kBox3 <= 6 * kChunk, "the box takes the records' place");
     const int tid = threadIdx.x;
-    // brick b with coff[b] <= ck < coff[b + 1] (bricks without records hold no chunk)
-    int lo = 0, hi = nb - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (a.coff[mid] <= ck) lo = mid;
-        else hi = mid - 1;
-    }
-    const int b = lo;
+    const int b = (int)a.ck_brick[ck];
     const unsigned r0 = a.off[b] + (ck - a.coff[b]) * kChunk, r1 = min(a.off[b + 1], r0 + kChunk);
     if (r0 >= r1) return;
     const int n = (int)(r1 - r0);
     const int k = b / a.nb_class;
     const int rem = b - k * a.nb_class;
     const int bx = rem % a.nbx, by = (rem / a.nbx) % a.nby, bz = rem / (a.nbx * a.nby);
-    for (int v = tid; v < 3 * kBox3; v += blockDim.x) (&box[0][0])[v] = 0.f;
     for (int v = tid; v < kVox; v += blockDim.x) vcnt[v] = 0u;
     __syncthreads();
     // records -> LDS (geometry and values), base voxel histogram
@@ -258,8 +256,8 @@ DEV void bp_brick_one(const BpArgs& a, int nb, unsigned ck) {
         bp_sample(a, s, p, sm);  // true: the record was made from the same test
         const Coords& c = sm.c;
         const float2 v = a.slice_val[(size_t)s * a.Pf + p];
-        const int lx = c.x0 - bx * kBrick, ly = c.y0 - by * kBrick, lz = c.z0 - bz * kBrick;
-        const int lv = (lz * kBrick + ly) * kBrick + lx;
+        const int lx = c.x0 - bx * kBrickX, ly = c.y0 - by * kBrickY, lz = c.z0 - bz * kBrickZ;
+        const int lv = (lz * kBrickY + ly) * kBrickX + lx;
         vox[i] = (unsigned short)lv;
         rec_f[0][i] = c.fx;
         rec_f[1][i] = c.fy;
@@ -290,7 +288,6 @@ DEV void bp_brick_one(const BpArgs& a, int nb, unsigned ck) {
             vcnt[tid * 8 + q] = run;  // becomes the scatter cursor
             run += loc[q];
         }
-        if (tid == 63) voff[kVox] = run;
     }
     __syncthreads();
     for (int i = tid; i < n; i += blockDim.x) order[atomicAdd(&vcnt[vox[i]], 1u)] = (unsigned short)i;
@@ -302,7 +299,8 @@ DEV void bp_brick_one(const BpArgs& a, int nb, unsigned ck) {
         const int lv = tid + 256 * h;
 #pragma unroll
         for (int cc = 0; cc < 8; ++cc) acc[h][cc][0] = acc[h][cc][1] = acc[h][cc][2] = 0.f;
-        for (unsigned j = voff[lv]; j < voff[lv + 1]; ++j) {
+        const unsigned je = lv + 1 < kVox ? voff[lv + 1] : (unsigned)n;
+        for (unsigned j = voff[lv]; j < je; ++j) {
             const int i = order[j];
             const float fx = rec_f[0][i], fy = rec_f[1][i], fz = rec_f[2][i];
             const float vr = rec_f[3][i], vi = rec_f[4][i], w = rec_f[5][i];
@@ -317,14 +315,17 @@ DEV void bp_brick_one(const BpArgs& a, int nb, unsigned ck) {
             }
         }
     }
+    __syncthreads();
+    for (int v = tid; v < 3 * kBox3; v += blockDim.x) (&box[0][0])[v] = 0.f;
+    __syncthreads();
 #pragma unroll
     for (int cc = 0; cc < 8; ++cc) {
         const int dz = cc >> 2, dy = (cc >> 1) & 1, dx = cc & 1;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int lv = tid + 256 * h;
-            const int lx = lv & 7, ly = (lv >> 3) & 7, lz = lv >> 6;
-            const int idx = ((lz + dz) * kBox + (ly + dy)) * kBox + (lx + dx);
+            const int lx = lv % kBrickX, ly = lv / kBrickX % kBrickY, lz = lv / (kBrickX * kBrickY);
+            const int idx = ((lz + dz) * kBoxY + (ly + dy)) * kBoxX + (lx + dx);
             box[0][idx] += acc[h][cc][0];
             box[1][idx] += acc[h][cc][1];
             box[2][idx] += acc[h][cc][2];
@@ -333,31 +334,42 @@ DEV void bp_brick_one(const BpArgs& a, int nb, unsigned ck) {
     }
     float* gd = a.bp_data + a.grid_stride * 2 * k;
     float* gw = a.bp_weight + a.grid_stride * k;
+    // to the grids: re and im in neighbouring lanes, as they lie there, so that one instruction's atomics fill their lines
+    auto voxel = [&](int v, size_t& idx) {
+        const int lx = v % kBoxX, ly = v / kBoxX % kBoxY, lz = v / (kBoxX * kBoxY);
+        const int gx = bx * kBrickX + lx, gy = by * kBrickY + ly, gz = bz * kBrickZ + lz;
+        idx = ((size_t)gz * a.pad + gy) * a.padF + gx;
+        return gx < a.padF && gy < a.pad && gz < a.pad;  // else nothing lands there (zero)
+    };
+    size_t idx;
+    for (int u = tid; u < 2 * kBox3; u += blockDim.x) {
+        const float d = box[u & 1][u >> 1];
+        if (d != 0.f && voxel(u >> 1, idx)) atomicAdd(&gd[2 * idx + (u & 1)], d);
+    }
     for (int v = tid; v < kBox3; v += blockDim.x) {
-        const float d0 = box[0][v], d1 = box[1][v], w = box[2][v];
-        if (d0 == 0.f && d1 == 0.f && w == 0.f) continue;
-        const int lx = v % kBox, ly = (v / kBox) % kBox, lz = v / (kBox * kBox);
-        const int gx = bx * kBrick + lx, gy = by * kBrick + ly, gz = bz * kBrick + lz;
-        if (gx >= a.padF || gy >= a.pad || gz >= a.pad) continue;  // nothing lands there (zero)
-        const size_t idx = ((size_t)gz * a.pad + gy) * a.padF + gx;
-        if (d0 != 0.f) atomicAdd(&gd[2 * idx], d0);
-        if (d1 != 0.f) atomicAdd(&gd[2 * idx + 1], d1);
-        if (w != 0.f) atomicAdd(&gw[idx], w);
+        const float w = box[2][v];
+        if (w != 0.f && voxel(v, idx)) atomicAdd(&gw[idx], w);
     }
 }
 
-// One block per chunk (the grid sized for the most chunks there can be), or (device-driven pools) a
-// fixed grid striding over the chunks, up to the total the scan left in coff[nb].
+// One block per chunk (the grid sized for the most chunks there can be), or (device-driven pools) a fixed grid whose
+// blocks stride over the chunks, up to the total the scan left in coff[nb]; blocks reach the 8 XCDs round-robin, and
+// each XCD strides over one contiguous eighth, so that neighbouring bricks share the lines of its L2 (259 x 259 x 130
+// voxels a class, 4 classes, 250 images: 440 -> 396 us).
+// What bounds it is the atomics' traffic past L2: bricks 16 voxels long (8 x 8 x 8: 703 us, 32 x 4 x 4: 669), re and
+// im added by neighbouring lanes (954 us with an instruction each), chunks of 1024 records (512: + 10 %, 4096: tails);
+// 2000 images of 128^2 in 4 classes: 995 -> 647 us.  Plain read-modify-writes of the voxels only one brick
+// reaches were slower (1192 us).
 template <bool Q>
-__global__ __launch_bounds__(256) void k_bp_brick(BpArgs a, int nb) {
+__global__ __launch_bounds__(256, 5) void k_bp_brick(BpArgs a, int nb) {
     if constexpr (!Q) {
-        if (blockIdx.x < a.coff[nb]) bp_brick_one(a, nb, blockIdx.x);
+        if (blockIdx.x < a.coff[nb]) bp_brick_one(a, blockIdx.x);
         return;
     }
     if (*a.abort) return;
-    const unsigned nck = a.coff[nb];
-    for (unsigned ck = blockIdx.x; ck < nck; ck += gridDim.x) {  // chunks strided over the grid
-        bp_brick_one(a, nb, ck);
+    const unsigned nck = a.coff[nb], per = (nck + 7) / 8, c0 = (blockIdx.x & 7) * per, c1 = min(c0 + per, nck);
+    for (unsigned ck = c0 + (blockIdx.x >> 3); ck < c1; ck += gridDim.x >> 3) {
+        bp_brick_one(a, ck);
         __syncthreads();  // the box of the next chunk
     }
 }
@@ -479,6 +491,12 @@ __global__ __launch_bounds__(256) void k_bp_band_add(BpArgs a, long long S_host,
     a.bp_weight[gn * k + i] += s[2];
 }
 
+void bp_scan(hipStream_t s, const BpArgs& a, int nb) {
+    const unsigned blocks = (unsigned)((nb + kScanBlock - 1) / kScanBlock);
+    k_bp_sums<<<blocks, kScanBlock, 0, s>>>(a.count, nb, a.sums);
+    k_bp_scan<<<blocks, kScanBlock, 0, s>>>(a.count, nb, a.sums, a.off, a.coff, a.cursor, a.ck_brick);
+}
+
 }  // namespace
 
 BandPlan bp_band_plan(int n, int K, int pad, int padF, int n_cu) {
@@ -507,6 +525,9 @@ hipError_t launch_backproject_bands(hipStream_t s, long long S, const BpArgs& a,
     return hipGetLastError();
 }
 
+// at most one chunk per brick plus one per kChunk records
+size_t bp_chunks_max(size_t nb, long long S, int Pf) { return nb + ((size_t)S * Pf + kChunk - 1) / kChunk; }
+
 hipError_t launch_backproject_binned(hipStream_t s, long long S, const BpArgs& a, int persist_blocks) {
     const int nb = a.nb_class * a.K;
     hipError_t e;
@@ -517,9 +538,9 @@ hipError_t launch_backproject_binned(hipStream_t s, long long S, const BpArgs& a
         const int nPB = (a.Pf + 255) / 256;
         const dim3 g2((unsigned)std::max(1, persist_blocks / nPB), (unsigned)nPB);
         k_bp_count<true><<<g2, 256, 0, s>>>(a, 0);
-        k_bp_scan<<<1, 1024, 0, s>>>(a.count, nb, a.off, a.coff, a.cursor);
+        bp_scan(s, a, nb);
         k_bp_fill<true><<<g2, 256, 0, s>>>(a, 0);
-        k_bp_brick<true><<<persist_blocks, 256, 0, s>>>(a, nb);
+        k_bp_brick<true><<<std::max(1, persist_blocks / 8) * 8, 256, 0, s>>>(a, nb);
         return hipGetLastError();
     }
     if (S <= 0) return hipSuccess;
@@ -527,10 +548,9 @@ hipError_t launch_backproject_binned(hipStream_t s, long long S, const BpArgs& a
     if ((e = launch_fill32(s, a.count, 0u, (size_t)nb)) != hipSuccess) return e;
     const dim3 grid((unsigned)S, (a.Pf + 255) / 256);
     k_bp_count<false><<<grid, 256, 0, s>>>(a, S);
-    k_bp_scan<<<1, 1024, 0, s>>>(a.count, nb, a.off, a.coff, a.cursor);
+    bp_scan(s, a, nb);
     k_bp_fill<false><<<grid, 256, 0, s>>>(a, S);
-    // at most one chunk per brick plus one per kChunk records
-    const unsigned long long chunks = (unsigned long long)nb + ((unsigned long long)S * a.Pf + kChunk - 1) / kChunk;
+    const unsigned long long chunks = bp_chunks_max(nb, S, a.Pf);
     k_bp_brick<false><<<(unsigned)chunks, 256, 0, s>>>(a, nb);
     return hipGetLastError();
 }

@@ -375,7 +375,7 @@ struct rome_ctx {
     DevBuf<float2> slice_val;
     DevBuf<float> bp_work;  // partial bands of 2D grids
     DevBuf<double> slice_w;
-    DevBuf<unsigned> bp_count, bp_off, bp_coff, bp_cursor;
+    DevBuf<unsigned> bp_count, bp_off, bp_coff, bp_cursor, bp_ck, bp_sums;
     DevBuf<unsigned long long> bp_rec;
     // whole images at given poses (rome_backproject_images), at most 1024 at a time
     DevBuf<double> bi_in, bi_one, bi_acc;
@@ -1624,15 +1624,17 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
             ba.r_max = ctx->r_max;
             ba.grid_stride = ctx->grid_n;
             if (ctx->is3d) {
-                ba.nbx = (ctx->padF + 7) / 8;
-                ba.nby = (ctx->pad + 7) / 8;
-                ba.nbz = (ctx->pad + 7) / 8;
+                ba.nbx = (ctx->padF + kBrickX - 1) / kBrickX;
+                ba.nby = (ctx->pad + kBrickY - 1) / kBrickY;
+                ba.nbz = (ctx->pad + kBrickZ - 1) / kBrickZ;
                 ba.nb_class = ba.nbx * ba.nby * ba.nbz;
                 const size_t nb = (size_t)ba.nb_class * ctx->K;
                 HIPCHK(ctx->bp_count.reserve(nb));
                 HIPCHK(ctx->bp_off.reserve(nb + 1));
                 HIPCHK(ctx->bp_coff.reserve(nb + 1));
                 HIPCHK(ctx->bp_cursor.reserve(nb));
+                HIPCHK(ctx->bp_sums.reserve(bp_scan_sums(nb)));
+                HIPCHK(sized(ctx->bp_ck, bp_chunks_max(nb, S, ctx->Pf)));
                 HIPCHK(sized(ctx->bp_rec, (size_t)S * ctx->Pf));
             }
             ba.task_img = ctx->task_img.p;
@@ -1646,6 +1648,8 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
             ba.off = ctx->bp_off.p;
             ba.coff = ctx->bp_coff.p;
             ba.cursor = ctx->bp_cursor.p;
+            ba.ck_brick = ctx->bp_ck.p;
+            ba.sums = ctx->bp_sums.p;
             ba.rec = ctx->bp_rec.p;
             ba.bp_data = ctx->bp_data.p;
             ba.bp_weight = ctx->bp_weight.p;
@@ -3478,13 +3482,15 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
         ba.c = ctx->cgrid;
         ba.r_max = ctx->r_max;
         ba.grid_stride = gn;
-        ba.nbx = (ctx->padF + 7) / 8;
-        ba.nby = ba.nbz = (ctx->pad + 7) / 8;
+        ba.nbx = (ctx->padF + kBrickX - 1) / kBrickX;
+        ba.nby = ba.nbz = (ctx->pad + kBrickZ - 1) / kBrickZ;
         ba.nb_class = ba.nbx * ba.nby * ba.nbz;
         HIPCHK(ctx->bp_count.reserve(ba.nb_class));
         HIPCHK(ctx->bp_off.reserve(ba.nb_class + 1));
         HIPCHK(ctx->bp_coff.reserve(ba.nb_class + 1));
         HIPCHK(ctx->bp_cursor.reserve(ba.nb_class));
+        HIPCHK(ctx->bp_sums.reserve(bp_scan_sums(ba.nb_class)));
+        HIPCHK(ctx->bp_ck.reserve(bp_chunks_max(ba.nb_class, chunk, ctx->Pf)));
         ia.val = ctx->bi_val.p;
         ia.wgt = ctx->bi_wgt.p;
         ia.task_img = ctx->bi_task.p;
@@ -3500,6 +3506,8 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
         ba.off = ctx->bp_off.p;
         ba.coff = ctx->bp_coff.p;
         ba.cursor = ctx->bp_cursor.p;
+        ba.ck_brick = ctx->bp_ck.p;
+        ba.sums = ctx->bp_sums.p;
         ba.rec = ctx->bi_rec.p;
         ba.bp_data = gd;
         ba.bp_weight = gw;

@@ -276,10 +276,11 @@ struct PostArgs {
 };
 
 // Binned 3D backprojection (backproject.hip)
+constexpr int kBrickX = 16, kBrickY = 8, kBrickZ = 4;  // base voxels of a brick
 struct BpArgs {
     int K, Pf, NOR, R, pad, padF, c, r_max;
     size_t grid_stride;
-    int nbx, nby, nbz, nb_class;  // bricks of 8 base voxels per axis (x over padF, y/z over pad)
+    int nbx, nby, nbz, nb_class;  // bricks per axis (x over padF, y/z over pad)
     const int* task_img;
     const int* task_m;
     const double* Ai_fine;        // [R][NOR][6]
@@ -291,6 +292,8 @@ struct BpArgs {
     unsigned* off;                // [nb + 1]
     unsigned* coff;               // [nb + 1] chunks of the brick kernel per brick, prefix sums
     unsigned* cursor;             // [nb]
+    unsigned* ck_brick;           // [bp_chunks_max] brick of every chunk
+    unsigned* sums;               // [bp_scan_sums] totals of blocks of bricks
     unsigned long long* rec;      // [records] slice << 32 | pixel
     float* bp_data;
     float* bp_weight;
@@ -525,6 +528,8 @@ hipError_t launch_bp_add2d(hipStream_t s, const double* acc, size_t n, float* bp
 hipError_t launch_store_sums(hipStream_t s, const StoreArgs& a);
 // With a.ntask_dev (device-driven pools) S is read on the device and persist_blocks blocks stride over
 // the slices (one pixel block per grid row) and over the brick chunks.
+inline size_t bp_scan_sums(size_t nb) { return 2 * ((nb + 1023) / 1024); }
+size_t bp_chunks_max(size_t nb, long long S, int Pf);  // chunks S slices of Pf pixels can make over nb bricks
 hipError_t launch_backproject_binned(hipStream_t s, long long S, const BpArgs& a, int persist_blocks = 0);
 // 2D: bands of grid rows accumulated in LDS, the slices of a class split over parts blocks per band
 struct BandPlan {

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dim,ori,cur,n,ctf", [(3, 16, 16, 1, True), (3, 24, 18, 70, True), (3, 16, 16, 1100, False),
-                                               (2, 16, 16, 1, True), (2, 24, 18, 70, False), (2, 20, 20, 1100, True)])
+                                               (3, 56, 56, 40, True), (2, 16, 16, 1, True), (2, 24, 18, 70, False), (2, 20, 20, 1100, True)])
 def test_backproject_images(engine, dim, ori, cur, n, ctf):
     print(f"[bp images dim={dim} ori={ori} cur={cur} n={n} ctf={ctf}]", flush=True)
     engine.configure(ref_dim=dim, ori_size=ori, current_size=cur, coarse_size=cur, nr_classes=2, nr_groups=1,
