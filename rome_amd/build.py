@@ -25,11 +25,13 @@ FLAGS = [
     "-Xarch_host", "-ffp-contract=off",
     "-Wall", "-Wno-unused-function",
 ]
+# vectors of equal scalars (8 registers each) made ahead of k_gemm_pq_cols' loop spilled 1.5 KB a lane
+FILE_FLAGS = {"gemm_lowp.hip": ["-fno-slp-vectorize"]}
 
 
 def _compile(src):
     obj = os.path.join(OBJ, src + ".o")
-    cmd = [HIPCC] + FLAGS + ["-c", os.path.join(CSRC, src), "-o", obj]
+    cmd = [HIPCC] + FLAGS + FILE_FLAGS.get(src, []) + ["-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     err = "\n".join(l for l in r.stderr.splitlines() if "packed-fp32-ops" not in l)
     if r.returncode != 0:

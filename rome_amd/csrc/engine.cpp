@@ -329,6 +329,7 @@ struct rome_ctx {
     // mixed-precision arm: scaled BF16/FP16 copies of the coarse table and of the image operand
     DevBuf<int> fct_absmax;
     DevBuf<uint16_t> A16, W16;  // A16: every rotation, or the half table of the paired cross term
+    DevBuf<uint16_t> A16f;          // the half table in MFMA fragment order (paired cross term)
     DevBuf<uint16_t> A16lo, W16lo;  // rounding remainders (split three-product recompute of marked samples)
     DevBuf<double> D2c, c_dmin1;    // recomputed diff2 of the marked coarse samples; first pass's minimum
     long long last_marked = 0;      // last pool: marked coarse samples recomputed (mixed arms)
@@ -647,6 +648,10 @@ int ensure_ready(rome_ctx* ctx) {
             HIPCHK(launch_fct_to_lowp(ctx->stream, ctx->cfg.precision, ctx->FcT.p, ctx->Pc_pad, ctx->Mpad, ctx->Mtot,
                                       rows, ctx->pq ? ctx->PSI / 2 : 0, ctx->fct_absmax.p, ctx->A16.p, ctx->A16lo.p,
                                       K16));
+            if (ctx->pq) {
+                HIPCHK(ctx->A16f.reserve(pq_fragments_len(rows, K16)));
+                HIPCHK(launch_pq_fragments(ctx->stream, ctx->A16.p, rows, K16, ctx->A16f.p));
+            }
         }
         ctx->fct_dirty = false;
     }
@@ -1214,14 +1219,15 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
         } else {
             LowpGemmArgs la{ctx->A16.p, ctx->W16.p, ctx->At.p, ctx->inv_scale.p, Ep, ctx->valid.p,
                             ctx->emin_key.p, K16, ctx->Mpad, Npad, M, Ncols, T,
-                            gemm_sub_band(ctx->Mpad / 256, (size_t)256 * K16 * 2, (size_t)5 << 19), L, 0, 0};
+                            gemm_sub_band(ctx->Mpad / 256, (size_t)256 * K16 * 2, (size_t)5 << 19), L, 0, 0, nullptr};
             if (ctx->pq) {  // the paired cross term over the half table (list or E output)
                 la.Mh = M / 2;
                 la.psih = ctx->PSI / 2;
+                la.Af = ctx->A16f.p;
                 la.sband = gemm_sub_band(la.Mh / 128, (size_t)128 * K16 * 2, (size_t)5 << 19);
                 if (!list) la.list.lpd = ctx->lpd_row.p;
             }
-            HIPCHK(launch_gemm_lowp(s, prec, la));
+            HIPCHK(launch_gemm_lowp(s, prec, la, ctx->n_cu));
         }
         stage_end(ctx, 2);
         return finish(list ? &L : nullptr);
@@ -1281,7 +1287,7 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
                 la.sband = gemm_sub_band(la.Mh / 128, (size_t)128 * K16 * 2, (size_t)5 << 19);
                 la.list.lpd = ctx->lpd_row.p;
             }
-            HIPCHK(launch_gemm_lowp(s, prec, la));
+            HIPCHK(launch_gemm_lowp(s, prec, la, ctx->n_cu));
             AuditArgs aa{P.E_audit.p, a0, T, M, P.nbins, P.gwords, P.gmask.p, wp, P.audit_mass.p};
             HIPCHK(audit_mass(s, na, aa));
         }
@@ -3483,7 +3489,8 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
         ba.r_max = ctx->r_max;
         ba.grid_stride = gn;
         ba.nbx = (ctx->padF + kBrickX - 1) / kBrickX;
-        ba.nby = ba.nbz = (ctx->pad + kBrickZ - 1) / kBrickZ;
+        ba.nby = (ctx->pad + kBrickY - 1) / kBrickY;
+        ba.nbz = (ctx->pad + kBrickZ - 1) / kBrickZ;
         ba.nb_class = ba.nbx * ba.nby * ba.nbz;
         HIPCHK(ctx->bp_count.reserve(ba.nb_class));
         HIPCHK(ctx->bp_off.reserve(ba.nb_class + 1));

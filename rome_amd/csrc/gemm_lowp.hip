@@ -14,6 +14,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "device_util.h"
 #include "gemm_common.h"
 #include "kernels.h"
@@ -453,6 +455,324 @@ __global__ __launch_bounds__(256, kPqBlocksPerCU) void k_gemm_lowp_pq(LowpGemmAr
                                    a.Mtot, a.Mpad, a.Ncols, a.T, slot_min);
 }
 
+// Paired cross term with list output, columns resident: a block of 8 waves holds 32 TJ columns (all of K16, Re and Im)
+// of the image operand in LDS and its waves take 32-row blocks of the half table in turn, with P and Q accumulators for
+// 32 rows x 32 TJ columns.  The rows stream from L2 in the order the MFMA reads them (one 1 KB load a fragment, four
+// steps of 16 k in flight); nothing is shared but the columns, so there is no barrier after the fill, and one wave's
+// epilogue runs beside the other waves' MFMAs.  An XCD keeps to one band of rows that fits its L2.  Same MFMAs over the
+// same ascending k per element as k_gemm_lowp_pq, whose 128-row tiles waited for their operands at two barriers every
+// 32 k and spent half their time so: 18432 rotations x 162000 columns x 512 k in FP16: 3548 ->
+// 2134 us, of which the matrix cores are busy 27 %; the epilogue's vector instructions bound it now.
+// The epilogue is that of gemm_epilogue_list per wave and row block: the bound of an image lives in LDS for the block,
+// starts from the global one and is exchanged with it once a row block; columns whose minimum of E less the largest
+// ln pdf_direction of the rows is past the limit have no entry and are left at that.  Every load in the loop is
+// unconditional: behind a branch each wait would be for all of them (6.2 ms), as behind a register spill.
+constexpr int kPqSlots = 5;  // images a column tile may touch
+// K16 / 2 in whole sets of four steps of 16 (zeros behind)
+__host__ __device__ __forceinline__ int pq_half(int K16) { return (K16 / 2 + 63) / 64 * 64; }
+template <typename T, int TJ>
+__global__ __launch_bounds__(512, 2) void k_gemm_pq_cols(LowpGemmArgs a, int bands, int nct) {
+    constexpr int BN = 32 * TJ, NW = 8;
+    typedef typename Lowp<T>::v8 v8;
+    extern __shared__ __attribute__((aligned(16))) char dyn[];
+    T* Bs = reinterpret_cast<T*>(dyn);  // [BN][K16 + 8]: rows 4 banks apart
+    __shared__ __attribute__((aligned(16))) float s_at[NW][kPqSlots][64], s_lp[NW][64];
+    __shared__ int s_cnt[NW][kPqSlots], s_vb[kPqSlots], s_min[kPqSlots], s_next;
+    __shared__ float s_reach[kPqSlots];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5;
+    const int x = blockIdx.x & 7, bi = blockIdx.x >> 3;  // XCD (blocks reach them round-robin), block within it
+    const int band = x % bands;
+    int ct = bi * (8 / bands) + x / bands;
+    if (ct >= nct) return;
+    // the bands start at different columns: the later ones find an image's bound set by the earlier ones
+    ct = (ct + band * ((nct + bands - 1) / bands)) % nct;
+    const int nrb = a.Mh / 32, rb_end = (int)((long long)nrb * (band + 1) / bands);
+    const int n0 = ct * BN, KH = a.K16 / 2, KHp = pq_half(a.K16), LDW = 2 * KHp + 8, nkk = KHp / 16;  // nkk % 4 == 0
+    const int img0 = n0 / a.T, nsl = (min(n0 + BN, a.Ncols) - 1) / a.T - img0 + 1;
+    {
+        const T* B = reinterpret_cast<const T*>(a.B);
+        const int ph = KHp / 8, pr = 2 * ph, np = BN * pr;  // 16-byte pieces of a half row, a row, the tile
+        for (int v0 = tid; v0 < np; v0 += 4 * 512) {
+            uint4 r[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {  // columns past the last repeat it (dropped below); padding k: zero
+                const int v = min(v0 + u * 512, np - 1), row = v / pr, c = v - row * pr, k = (c % ph) * 8;
+                const uint4 x = *reinterpret_cast<const uint4*>(B + (size_t)min(n0 + row, a.Ncols - 1) * a.K16 +
+                                                                (c / ph) * KH + min(k, KH - 8));
+                r[u] = k < KH ? x : make_uint4(0u, 0u, 0u, 0u);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int v = v0 + u * 512, row = v / pr;
+                if (v < np) *reinterpret_cast<uint4*>(Bs + (size_t)row * LDW + 8 * (v - row * pr)) = r[u];
+            }
+        }
+    }
+    if (tid < nsl) {
+        s_vb[tid] = __hip_atomic_load(&a.list.vbound[img0 + tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_min[tid] = INT_MAX;
+        s_reach[tid] = a.list.reach[img0 + tid];
+    }
+    if (tid == 0) s_next = (int)((long long)nrb * band / bands);
+    __syncthreads();
+    int sl_j[TJ];
+    float s_j[TJ], emin_j[TJ];
+    bool ok_j[TJ];
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) {
+        const int col = n0 + j * 32 + (lane & 31);
+        ok_j[j] = col < a.Ncols;
+        const int img = (int)((unsigned)min(col, a.Ncols - 1) / (unsigned)a.T);
+        sl_j[j] = img - img0;
+        s_j[j] = a.inv_scale[img];
+        emin_j[j] = INFINITY;
+    }
+    auto next_rb = [&]() {
+        int v = 0;
+        if (lane == 0) v = atomicAdd(&s_next, 1);
+        return __builtin_amdgcn_readfirstlane(v);
+    };
+    const T* const Af = reinterpret_cast<const T*>(a.Af);
+    const size_t rb_len = (size_t)nkk * 1024;
+    v8 ar[4], ai[4];  // rows of four steps (Re, Im)
+    auto load_a = [&](int q, const T* A, int kk) {
+        ar[q] = *reinterpret_cast<const v8*>(A + (size_t)kk * 1024);
+        ai[q] = *reinterpret_cast<const v8*>(A + (size_t)kk * 1024 + 512);
+    };
+    const unsigned up = (unsigned)a.psih;
+    auto rot = [&](unsigned hh) { return (int)((hh / up) * 2 * up + hh % up); };  // rotation of a half-table row
+    int rb = next_rb();
+    if (rb < rb_end) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) load_a(q, Af + rb * rb_len + lane * 8, q);
+    }
+    while (rb < rb_end) {
+        // the lane's number through an opaque copy: what is derived from it would otherwise be computed ahead of the
+        // loop, and spilled
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const int eh = ln >> 5;
+        const int rb_next = next_rb();
+        const T *A = Af + rb * rb_len + ln * 8, *An = Af + min(rb_next, rb_end - 1) * rb_len + ln * 8;
+        // what the epilogue reads of global memory, one row a lane: P + Q rotations in the first half of the wave
+        const int m_l = rot((unsigned)(rb * 32 + (ln & 31))) + eh * a.psih;
+        const float lp_l = a.list.lpd[m_l];
+        float at_l[kPqSlots];
+#pragma unroll
+        for (int q = 0; q < kPqSlots; ++q) at_l[q] = a.At[(size_t)(img0 + min(q, nsl - 1)) * a.Mpad + m_l];
+        const int vb_g = __hip_atomic_load(&a.list.vbound[img0 + min(ln, nsl - 1)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        f16v acc[2][TJ];  // P, Q
+        const T* const bl = Bs + (ln & 31) * LDW + 8 * eh;
+        v8 bre[TJ], bim[TJ];
+        auto load_b = [&](int j, int kk) {
+            bre[j] = *reinterpret_cast<const v8*>(bl + j * 32 * LDW + kk * 16);
+            bim[j] = *reinterpret_cast<const v8*>(bl + j * 32 * LDW + kk * 16 + KHp);
+        };
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) load_b(j, 0);
+        auto steps = [&](int k0, auto first) {
+            // four steps on, past the end the next row block's first: no branch, so that each wait counts the loads behind
+            const T* Ak = k0 + 4 < nkk ? A + (size_t)(k0 + 4) * 1024 : An;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int kn = min(k0 + q + 1, nkk - 1);
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) {
+                    const bool zero = first.value && q == 0;
+                    acc[0][j] = Lowp<T>::mfma(ar[q], bre[j], zero ? f16v{} : acc[0][j]);
+                    acc[1][j] = Lowp<T>::mfma(ai[q], bim[j], zero ? f16v{} : acc[1][j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    load_b(j, kn);
+                }
+                load_a(q, Ak, q);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        steps(0, std::true_type{});
+        for (int k0 = 4; k0 < nkk; k0 += 4) steps(k0, std::false_type{});
+        const float pen = lp_l > -INFINITY ? 0.f : INFINITY;  // rows without a prior: E = +inf
+#pragma unroll
+        for (int q = 0; q < kPqSlots; ++q) s_at[w][q][ln] = at_l[q] + pen;
+        s_lp[w][ln] = lp_l;
+        if (ln < nsl) {
+            s_cnt[w][ln] = 0;
+            if (vb_g < s_vb[ln]) atomicMin(&s_vb[ln], vb_g);
+        }
+        float lp_max = lp_l;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) lp_max = fmaxf(lp_max, __shfl_xor(lp_max, o, 64));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        // E in place of P, Q, and its minimum
+        float em[TJ];
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) em[j] = INFINITY;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r0 = 8 * q + 4 * eh;
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) {
+                const float4 a0 = *reinterpret_cast<const float4*>(&s_at[w][sl_j[j]][r0]);
+                const float4 a1 = *reinterpret_cast<const float4*>(&s_at[w][sl_j[j]][32 + r0]);
+                const float at0[4] = {a0.x, a0.y, a0.z, a0.w}, at1[4] = {a1.x, a1.y, a1.z, a1.w};
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const float P = acc[0][j][4 * q + u], Q = acc[1][j][4 * q + u];
+                    const float e0 = e_value<true>(at0[u], P + Q, s_j[j]), e1 = e_value<true>(at1[u], P - Q, s_j[j]);
+                    acc[0][j][4 * q + u] = e0;
+                    acc[1][j][4 * q + u] = e1;
+                    em[j] = fminf(fminf(em[j], e0), e1);
+                }
+                __builtin_amdgcn_sched_barrier(0);  // registers: one column block's rows at a time
+            }
+        }
+        unsigned bits[TJ];  // entries among the lane's rows of the column: bit 16 i + register
+        int off[TJ];
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            emin_j[j] = fminf(emin_j[j], em[j]);
+            bits[j] = 0u;
+            int sl = sl_j[j];
+            asm volatile("" : "+v"(sl));
+            int b = *(volatile int*)&s_vb[sl];
+            const float r = s_reach[sl];
+            auto limit = [&](int key) {
+                const float bv = float_from_order_key(key);
+                return ok_j[j] && key != INT_MAX ? bv + r + 1e-6f * (fabsf(bv) + r) + 1e-3f : -INFINITY;
+            };
+            // no v = E - ln pdf_direction of the column's rows lies below em - lp_max (to FP32 rounding, which rounds
+            // monotonely): neither an entry nor a better bound where that is past the limit
+            const float v_low = em[j] - lp_max;
+            float lim = limit(b);
+            if (!__ballot(ok_j[j] && (v_low < lim || (b == INT_MAX && v_low < INFINITY)))) continue;
+            // f(i, q, v): the four values v of block i, quad q
+            auto quads = [&](auto f) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const float4 l = *reinterpret_cast<const float4*>(&s_lp[w][32 * i + 8 * q + 4 * eh]);
+                        const float v[4] = {acc[i][j][4 * q] - l.x, acc[i][j][4 * q + 1] - l.y, acc[i][j][4 * q + 2] - l.z,
+                                            acc[i][j][4 * q + 3] - l.w};
+                        f(i, q, v);
+                        if (q & 1) __builtin_amdgcn_sched_barrier(0);
+                    }
+            };
+            if (__ballot(ok_j[j] && (b == INT_MAX || v_low < float_from_order_key(b)))) {
+                float v = INFINITY;
+                quads([&](int, int, const float(&x)[4]) { v = fminf(fminf(fminf(v, x[0]), x[1]), fminf(x[2], x[3])); });
+                const int key = ok_j[j] && v < INFINITY ? float_order_key(v + 1e-6f * fabsf(v) + 1e-4f) : INT_MAX;
+                const bool better = key < b;
+                if (better) atomicMin(&s_vb[sl], key);
+                if (__ballot(better)) {
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    b = *(volatile int*)&s_vb[sl];
+                    lim = limit(b);
+                    if (ln < nsl) atomicMin(&a.list.vbound[img0 + ln], *(volatile int*)&s_vb[ln]);
+                }
+            }
+            quads([&](int i, int q, const float(&x)[4]) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) bits[j] |= x[u] < lim ? 1u << (16 * i + 4 * q + u) : 0u;
+            });
+            if (bits[j]) off[j] = atomicAdd(&s_cnt[w][sl], __popc(bits[j]));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        unsigned all = bits[0];
+#pragma unroll
+        for (int j = 1; j < TJ; ++j) all |= bits[j];
+        if (__ballot(all != 0u)) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (ln < nsl) {
+                const int c = s_cnt[w][ln];
+                s_cnt[w][ln] = c ? atomicAdd(&a.list.count[img0 + ln], c) : 0;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            int mq[4];  // rotations of the lane's four quads of rows
+#pragma unroll
+            for (int q = 0; q < 4; ++q) mq[q] = rot((unsigned)(rb * 32 + 8 * q + 4 * eh));
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) {
+                if (!__ballot(bits[j] != 0u)) continue;
+                int sl = sl_j[j];
+                asm volatile("" : "+v"(sl));
+                const int img = img0 + sl;
+                const unsigned tm = (unsigned)(n0 + j * 32 + (ln & 31) - img * a.T) * (unsigned)a.Mtot;
+                int pos = bits[j] ? s_cnt[w][sl] + off[j] : 0;
+                unsigned* const ent = a.list.ent + (size_t)img * a.list.cap;
+                float* const val = a.list.val + (size_t)img * a.list.cap;
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const unsigned nib = bits[j] >> (16 * i + 4 * q) & 15u;
+                        if (!__ballot(nib != 0u)) continue;
+                        const unsigned m = tm + (unsigned)(mq[q] + i * a.psih);
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            if (!(nib >> u & 1u)) continue;
+                            if (pos < a.list.cap) {
+                                ent[pos] = m + u;
+                                val[pos] = acc[i][j][4 * q + u];
+                            }
+                            ++pos;
+                        }
+                    }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        rb = rb_next;
+    }
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+        if (ok_j[j] && emin_j[j] < INFINITY) atomicMin(&s_min[sl_j[j]], float_order_key(emin_j[j]));
+    __syncthreads();
+    if (tid < nsl && s_min[tid] != INT_MAX) atomicMin(&a.emin_key[img0 + tid], s_min[tid]);
+}
+
+// The half table in the order k_gemm_pq_cols streams it: [row block of 32][step of 16 k][Re | Im][lane][8].
+__global__ __launch_bounds__(256) void k_pq_fragments(const uint4* __restrict__ A16, int Mh, int K16,
+                                                      uint4* __restrict__ Af) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;  // 16-byte piece of the output
+    const int KHp = pq_half(K16), nkk = KHp / 16;
+    if (i >= (size_t)Mh * KHp / 4) return;
+    const int lane = (int)(i & 63), half = (int)(i >> 6) & 1;
+    const size_t f = i >> 7;
+    const int k = (int)(f % nkk) * 16 + 8 * (lane >> 5), row = (int)(f / nkk) * 32 + (lane & 31);
+    Af[i] = k < K16 / 2 ? A16[((size_t)row * K16 + half * (K16 / 2) + k) / 8] : make_uint4(0u, 0u, 0u, 0u);
+}
+
+// row bands of k_gemm_pq_cols (a power of two up to the 8 XCDs): as few as fit 2.5 MB of an XCD's 4 MB L2 each
+int pq_bands(const LowpGemmArgs& a) {
+    int bands = 1;
+    while (bands < 8 && (size_t)a.Mh * pq_half(a.K16) * 4 / bands > ((size_t)5 << 19)) bands *= 2;
+    return bands;
+}
+
+template <typename T, int TJ>
+hipError_t go_pq_cols(hipStream_t s, const LowpGemmArgs& a) {
+    const int nct = (a.Ncols + 32 * TJ - 1) / (32 * TJ), bands = pq_bands(a);
+    const unsigned blocks = 8u * (unsigned)((nct + 8 / bands - 1) / (8 / bands));
+    const size_t lds = (size_t)32 * TJ * (2 * pq_half(a.K16) + 8) * 2;
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm_pq_cols<T, TJ>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    k_gemm_pq_cols<T, TJ><<<blocks, 512, lds, s>>>(a, bands, nct);
+    return hipGetLastError();
+}
+
+// Columns of 32 a tile of k_gemm_pq_cols holds: three (96; four spill registers) where they fit in LDS beside its 13 KB,
+// else two.  0, the tiled kernel: tiles of more images than there are slots for, and fewer than four blocks a CU, whose
+// unequal rounds and fills cost what the loop gains (6912 half rows x 9657 columns x 320 k, 1.6 blocks a CU: 236 us both,
+// and longer lists; 9216 x 162000 x 512 k, 26 a CU: 3548 -> 2134 us).
+int pq_cols_tj(const LowpGemmArgs& a, int n_cu) {
+    for (int tj = 3; tj >= 2; --tj) {
+        if (32 * tj * (2 * pq_half(a.K16) + 8) * 2 + (13 << 10) > (160 << 10)) continue;
+        if ((32 * tj - 1) / a.T + 2 > kPqSlots || (long long)(a.Ncols / (32 * tj)) * pq_bands(a) < 4LL * n_cu) return 0;
+        return tj;
+    }
+    return 0;
+}
+
 // sF: power of two that brings max |FcT| into [0.5, 1) (exact rescaling)
 DEV float table_scale(const int* absmax_bits) {
     const float mx = __int_as_float(*absmax_bits);
@@ -630,13 +950,19 @@ __global__ __launch_bounds__(256) void k_recompute_split(RecomputeArgs a) {
 
 }  // namespace
 
-hipError_t launch_gemm_lowp(hipStream_t s, int precision, const LowpGemmArgs& a) {
+hipError_t launch_gemm_lowp(hipStream_t s, int precision, const LowpGemmArgs& a, int n_cu) {
+    if (precision != 1 && precision != 2) return hipErrorInvalidValue;
     if (a.Mpad % 256 || a.Npad % 256 || a.K16 % 64 || a.K16 <= 0) return hipErrorInvalidValue;
     if (a.psih > 0) {  // paired cross term
         if (a.psih % 4 || a.Mh % 128 || 2 * a.Mh != a.Mtot || a.Mtot % 4 || a.T < 8 || !a.list.lpd)
             return hipErrorInvalidValue;
         const bool lst = a.list.count != nullptr;
         if (!lst && (!a.E || !a.list.lpd)) return hipErrorInvalidValue;
+        if (lst && a.Af) {
+            const int tj = pq_cols_tj(a, n_cu);
+            if (tj == 3) return precision == 1 ? go_pq_cols<__bf16, 3>(s, a) : go_pq_cols<_Float16, 3>(s, a);
+            if (tj == 2) return precision == 1 ? go_pq_cols<__bf16, 2>(s, a) : go_pq_cols<_Float16, 2>(s, a);
+        }
         const unsigned tiles = gemm_grouped_blocks(a.Mh / 128, a.Npad / kPqBN, a.sband);
         if (precision == 1) {
             if (lst) k_gemm_lowp_pq<__bf16, true><<<tiles, 256, 0, s>>>(a);
@@ -677,6 +1003,15 @@ hipError_t launch_fct_to_lowp(hipStream_t s, int precision, const float* FcT, in
         k_fct_to_lowp<_Float16><<<blocks, 256, 0, s>>>(FcT, Pc_pad, Mpad, Mtot, rows, psih, fct_absmax, (_Float16*)A16,
                                                         (_Float16*)A16lo, K16);
     else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+size_t pq_fragments_len(int Mh, int K16) { return (size_t)Mh * 2 * pq_half(K16); }
+
+hipError_t launch_pq_fragments(hipStream_t s, const void* A16, int Mh, int K16, void* Af) {
+    if (Mh % 32 || K16 % 32) return hipErrorInvalidValue;
+    k_pq_fragments<<<(unsigned)(((size_t)Mh * pq_half(K16) / 4 + 255) / 256), 256, 0, s>>>(
+        static_cast<const uint4*>(A16), Mh, K16, static_cast<uint4*>(Af));
     return hipGetLastError();
 }
 

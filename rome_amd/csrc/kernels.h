@@ -121,6 +121,7 @@ struct LowpGemmArgs {
     // rotation m + psih (psi + 180 deg) has the conjugate projection, so with P = sum Re*Re and
     // Q = sum Im*Im over the K16/2 halves, C(m) = P + Q and C(m + psih) = P - Q: half the MFMA work
     int Mh, psih;
+    const void* Af;  // the half table in MFMA fragment order (launch_pq_fragments), or null
 };
 
 struct PrepLowpArgs {
@@ -585,6 +586,8 @@ hipError_t launch_fct_to_lowp(hipStream_t s, int precision, const float* FcT, in
                               int rows, int psih, const int* fct_absmax, void* A16, void* A16lo, int K16);
 hipError_t launch_recompute_split(hipStream_t s, int precision, int n, const RecomputeArgs& a);
 hipError_t launch_prep_lowp(hipStream_t s, int precision, int n, const PrepLowpArgs& a);
-hipError_t launch_gemm_lowp(hipStream_t s, int precision, const LowpGemmArgs& a);
+hipError_t launch_gemm_lowp(hipStream_t s, int precision, const LowpGemmArgs& a, int n_cu);
+size_t pq_fragments_len(int Mh, int K16);  // values of that table
+hipError_t launch_pq_fragments(hipStream_t s, const void* A16, int Mh, int K16, void* Af);
 
 }  // namespace rome
