@@ -2273,15 +2273,11 @@ int rome_reset_sums(rome_ctx* ctx) {
     if (!ctx->configured) return fail(ctx, ROME_ERR_ARG, "rome_configure has not been called");
     HIPCHK(hipSetDevice(ctx->device));
     hipStream_t s = ctx->stream;
-    HIPCHK(hipMemsetAsync(ctx->bp_data.p, 0, 2 * ctx->grid_n * ctx->K * sizeof(float), s));
-    HIPCHK(hipMemsetAsync(ctx->bp_weight.p, 0, ctx->grid_n * ctx->K * sizeof(float), s));
-    HIPCHK(hipMemsetAsync(ctx->wsum_sigma2.p, 0, (size_t)ctx->cfg.nr_groups * ctx->oriF * sizeof(double), s));
-    HIPCHK(hipMemsetAsync(ctx->wsum_pdf_class.p, 0, ctx->K * sizeof(double), s));
-    HIPCHK(hipMemsetAsync(ctx->wsum_pdf_dir.p, 0, (size_t)ctx->K * ctx->D * sizeof(double), s));
-    HIPCHK(hipMemsetAsync(ctx->wsum_sumw_group.p, 0, ctx->cfg.nr_groups * sizeof(double), s));
-    HIPCHK(hipMemsetAsync(ctx->wsum_prior_x.p, 0, ctx->K * sizeof(double), s));
-    HIPCHK(hipMemsetAsync(ctx->wsum_prior_y.p, 0, ctx->K * sizeof(double), s));
-    HIPCHK(hipMemsetAsync(ctx->wsum_scalars.p, 0, 4 * sizeof(double), s));
+    const size_t f = sizeof(float), d = sizeof(double), K = ctx->K, G = ctx->cfg.nr_groups;
+    HIPCHK(launch_zero(s, {{ctx->bp_data.p, 2 * ctx->grid_n * K * f}, {ctx->bp_weight.p, ctx->grid_n * K * f},
+                           {ctx->wsum_sigma2.p, G * ctx->oriF * d}, {ctx->wsum_pdf_class.p, K * d},
+                           {ctx->wsum_pdf_dir.p, K * ctx->D * d}, {ctx->wsum_sumw_group.p, G * d},
+                           {ctx->wsum_prior_x.p, K * d}, {ctx->wsum_prior_y.p, K * d}, {ctx->wsum_scalars.p, 4 * d}}));
     HIPCHK(hipStreamSynchronize(s));
     return ROME_OK;
 }
@@ -2370,20 +2366,14 @@ int rome_get_sums(rome_ctx* ctx, rome_sums* o) {
     if (!ctx || !o) return ROME_ERR_ARG;
     if (!ctx->configured) return fail(ctx, ROME_ERR_ARG, "rome_configure has not been called");
     HIPCHK(hipSetDevice(ctx->device));
-    hipStream_t s = ctx->stream;
-    auto cp = [&](double* h, const double* d, size_t n) -> hipError_t {
-        return h ? hipMemcpyAsync(h, d, n * sizeof(double), hipMemcpyDeviceToHost, s) : hipSuccess;
-    };
-    const int G = ctx->cfg.nr_groups;
-    HIPCHK(cp(o->wsum_sigma2_noise, ctx->wsum_sigma2.p, (size_t)G * ctx->oriF));
-    HIPCHK(cp(o->wsum_sumw_group, ctx->wsum_sumw_group.p, G));
-    HIPCHK(cp(o->wsum_pdf_class, ctx->wsum_pdf_class.p, ctx->K));
-    HIPCHK(cp(o->wsum_pdf_direction, ctx->wsum_pdf_dir.p, (size_t)ctx->K * ctx->D));
-    HIPCHK(cp(o->wsum_prior_offx, ctx->wsum_prior_x.p, ctx->K));
-    HIPCHK(cp(o->wsum_prior_offy, ctx->wsum_prior_y.p, ctx->K));
-    HIPCHK(cp(o->wsum_scalars, ctx->wsum_scalars.p, 4));
-    HIPCHK(hipStreamSynchronize(s));
-    return ROME_OK;
+    const size_t d = sizeof(double), K = ctx->K, G = ctx->cfg.nr_groups;
+    return readback(ctx, {{ctx->wsum_sigma2.p, o->wsum_sigma2_noise, G * ctx->oriF * d},
+                          {ctx->wsum_sumw_group.p, o->wsum_sumw_group, G * d},
+                          {ctx->wsum_pdf_class.p, o->wsum_pdf_class, K * d},
+                          {ctx->wsum_pdf_dir.p, o->wsum_pdf_direction, K * ctx->D * d},
+                          {ctx->wsum_prior_x.p, o->wsum_prior_offx, K * d},
+                          {ctx->wsum_prior_y.p, o->wsum_prior_offy, K * d},
+                          {ctx->wsum_scalars.p, o->wsum_scalars, 4 * d}});
 }
 
 int rome_get_backprojector(rome_ctx* ctx, int iclass, double* data, double* weight) {
@@ -2860,7 +2850,7 @@ int rome_reconstruct(rome_ctx* ctx, int iclass, const rome_recon_params* prm, co
     HIPCHK(ctx->rc_Ft.reserve(std::max(nFt, nT)));
     HIPCHK(ctx->rc_Mout.reserve(nMo));
     HIPCHK(ctx->rc_vol.reserve(nv));
-    HIPCHK(ctx->rc_sums.reserve(4 * (size_t)std::max(oriF, ori)));
+    HIPCHK(ctx->rc_sums.reserve(4 * (size_t)oriF + 2 + 2 * (size_t)ori));
     HIPCHK(ctx->rc_tau2.reserve(oriF));
     HIPCHK(ctx->rc_bad.reserve(1));
     if (data_in) {
@@ -2875,20 +2865,25 @@ int rome_reconstruct(rome_ctx* ctx, int iclass, const rome_recon_params* prm, co
     HIPCHK(rc_fold(s, ctx->rc_data.p, ctx->rc_weight.p, Dz, P, PF));
     HIPCHK(rc_decenter_real(s, ctx->rc_weight.p, ctx->rc_Fw.p, Dz, P, PF, max_r2));
     // radial average of the inverse noise power (:2019-2060)
-    double* s0 = ctx->rc_sums.p;
-    double* s1 = s0 + oriF;
-    HIPCHK(hipMemsetAsync(s0, 0, 2 * oriF * sizeof(double), s));
+    // shell sums of the spectrum (two arrays) and of the MAP weights (two), the background's two, the new map's spectrum
+    // (two): read back once at the end, so that nothing waits for the host in between (unless tau2 comes from the FSC,
+    // which needs sigma2 first).  A read-back after each and its wait left the GPU idle for a quarter of a 2D class.
+    double *s0 = ctx->rc_sums.p, *s1 = s0 + oriF, *s2 = s1 + oriF, *s3 = s2 + oriF, *bg = s3 + oriF, *sp = bg + 2;
+    HIPCHK(launch_zero(s, {{s0, (4 * (size_t)oriF + 2 + 2 * (size_t)ori) * sizeof(double)}, {ctx->rc_bad.p, sizeof(int)}}));
     HIPCHK(rc_spectrum(s, ctx->rc_Fw.p, Dz, P, PF, max_r2, pf, osc, oriF, s0, s1));
-    std::vector<double> h0(oriF), h1(oriF);
-    HIPCHK(hipMemcpyAsync(h0.data(), s0, oriF * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(h1.data(), s1, oriF * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    for (int i = 0; i < oriF; ++i) {
-        if (h0[i] > 1e-10) sigma2[i] = h1[i] / h0[i];
-        else if (h0[i] == 0.) sigma2[i] = 0.;
-        else return fail(ctx, ROME_ERR_NUMERIC, "unexpectedly small, yet non-zero sigma2 value (shell %d)", i);
-    }
+    std::vector<double> h(4 * (size_t)oriF), hsp(2 * (size_t)ori);
+    auto take_sigma2 = [&]() -> int {
+        for (int i = 0; i < oriF; ++i) {
+            if (h[i] > 1e-10) sigma2[i] = h[oriF + i] / h[i];
+            else if (h[i] == 0.) sigma2[i] = 0.;
+            else return fail(ctx, ROME_ERR_NUMERIC, "unexpectedly small, yet non-zero sigma2 value (shell %d)", i);
+        }
+        return ROME_OK;
+    };
     if (prm->update_tau2_with_fsc) {  // tau2 from the FSC (:2062-2080)
+        rc = readback(ctx, {{s0, h.data(), 2 * oriF * sizeof(double)}});
+        if (!rc) rc = take_sigma2();
+        if (rc) return rc;
         for (int i = 0; i < oriF; ++i) {
             double myfsc = std::max(0.001, fsc[i]);
             if (prm->is_whole_instead_of_half) myfsc = std::sqrt(2. * myfsc / (myfsc + 1.));
@@ -2900,19 +2895,8 @@ int rome_reconstruct(rome_ctx* ctx, int iclass, const rome_recon_params* prm, co
     }
     if (prm->do_map) {
         HIPCHK(hipMemcpyAsync(ctx->rc_tau2.p, tau2, oriF * sizeof(double), hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemsetAsync(s0, 0, 2 * oriF * sizeof(double), s));
-        HIPCHK(hipMemsetAsync(ctx->rc_bad.p, 0, sizeof(int), s));
         HIPCHK(rc_map(s, ctx->rc_Fw.p, Dz, P, PF, max_r2, pf, osc, prm->tau2_fudge, ctx->rc_tau2.p, prm->minres_map,
-                      oriF, s0, s1, ctx->rc_bad.p));
-        int bad = 0;
-        HIPCHK(hipMemcpyAsync(h0.data(), s0, oriF * sizeof(double), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipMemcpyAsync(h1.data(), s1, oriF * sizeof(double), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipMemcpyAsync(&bad, ctx->rc_bad.p, sizeof(int), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        if (bad) return fail(ctx, ROME_ERR_NUMERIC, "negative values in the tau2 spectrum");
-        if (!prm->update_tau2_with_fsc)
-            for (int i = 0; i < oriF; ++i)
-                data_vs_prior[i] = i > r_max ? 0. : (h1[i] < 0.001 ? 999. : h0[i] / h1[i]);
+                      oriF, s2, s3, ctx->rc_bad.p));
     }
     HIPCHK(rc_normalise(s, ctx->rc_Fw.p, ctx->rc_data.p, ng, prm->normalise));
     // iterative gridding weights (Pipe & Menon), :2196-2274
@@ -2952,9 +2936,8 @@ int rome_reconstruct(rome_ctx* ctx, int iclass, const rome_recon_params* prm, co
         return fail(ctx, ROME_ERR_HIP, "hipfftExecZ2D failed");
     const double normfft = ctx->is3d ? (double)(pf * pf * pf * ori) : (double)(pf * pf);
     HIPCHK(rc_center_window(s, ctx->rc_Mout.p, ctx->rc_vol.p, NZ, N, OZ, ori, normfft));
-    HIPCHK(hipMemsetAsync(s0, 0, 2 * sizeof(double), s));
-    HIPCHK(rc_bgsum(s, ctx->rc_vol.p, OZ, ori, (double)ori / 2., 3., s0));
-    HIPCHK(rc_mask_grid(s, ctx->rc_vol.p, OZ, ori, pf, (double)ori / 2., 3., s0));
+    HIPCHK(rc_bgsum(s, ctx->rc_vol.p, OZ, ori, (double)ori / 2., 3., bg));
+    HIPCHK(rc_mask_grid(s, ctx->rc_vol.p, OZ, ori, pf, (double)ori / 2., 3., bg));
     if (prm->update_tau2_with_fsc) {  // new tau2 = power spectrum of the new map (:2473-2510)
         hipfftHandle planO;
         rc = fft_plan(ctx, HIPFFT_D2Z, rank, ori, &planO);
@@ -2964,15 +2947,31 @@ int rome_reconstruct(rome_ctx* ctx, int iclass, const rome_recon_params* prm, co
         HIPCHK(hipMemcpyAsync(ctx->rc_M.p, ctx->rc_vol.p, nv * sizeof(double), hipMemcpyDeviceToDevice, s));
         if (hipfftExecD2Z(planO, ctx->rc_M.p, Z(ctx->rc_Fc.p)) != HIPFFT_SUCCESS)
             return fail(ctx, ROME_ERR_HIP, "hipfftExecD2Z failed");
-        HIPCHK(hipMemsetAsync(s0, 0, 2 * ori * sizeof(double), s));
-        HIPCHK(rc_map_spectrum(s, ctx->rc_Fc.p, OZ, ori, (double)nv, s0, s0 + ori));
-        std::vector<double> sp(2 * ori);
-        HIPCHK(hipMemcpyAsync(sp.data(), s0, 2 * ori * sizeof(double), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        const double nf = ctx->is3d ? (double)ori * ori : 1.;
-        for (int i = 0; i < oriF; ++i) tau2[i] = prm->tau2_fudge * (sp[i] / sp[ori + i] * nf / 2.);
+        HIPCHK(rc_map_spectrum(s, ctx->rc_Fc.p, OZ, ori, (double)nv, sp, sp + ori));
     }
-    HIPCHK(ctx->copy_out.run(s, {{vol_out, ctx->rc_vol.p, nv * sizeof(double)}}));
+    // the sums and, if it is small, the map in one read-back
+    const bool small = nv * sizeof(double) <= ((size_t)1 << 20);
+    std::vector<double> vol(small ? nv : 0);
+    int bad = 0;
+    rc = readback(ctx, {{s0, h.data(), h.size() * sizeof(double)},
+                        {ctx->rc_bad.p, &bad, sizeof(int)},
+                        {sp, prm->update_tau2_with_fsc ? hsp.data() : nullptr, hsp.size() * sizeof(double)},
+                        {ctx->rc_vol.p, small ? vol.data() : nullptr, nv * sizeof(double)}});
+    if (!rc && !prm->update_tau2_with_fsc) rc = take_sigma2();
+    if (rc) return rc;
+    if (prm->do_map) {
+        if (bad) return fail(ctx, ROME_ERR_NUMERIC, "negative values in the tau2 spectrum");
+        const double *h0 = h.data() + 2 * oriF, *h1 = h0 + oriF;
+        if (!prm->update_tau2_with_fsc)
+            for (int i = 0; i < oriF; ++i)
+                data_vs_prior[i] = i > r_max ? 0. : (h1[i] < 0.001 ? 999. : h0[i] / h1[i]);
+    }
+    if (prm->update_tau2_with_fsc) {
+        const double nf = ctx->is3d ? (double)ori * ori : 1.;
+        for (int i = 0; i < oriF; ++i) tau2[i] = prm->tau2_fudge * (hsp[i] / hsp[ori + i] * nf / 2.);
+    }
+    if (small) std::memcpy(vol_out, vol.data(), nv * sizeof(double));
+    else HIPCHK(ctx->copy_out.run(s, {{vol_out, ctx->rc_vol.p, nv * sizeof(double)}}));
     return ROME_OK;
 }
 

@@ -3,6 +3,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <utility>
+#include <vector>
+
 #include "rome_common.h"
 
 namespace rome {
@@ -483,6 +486,9 @@ struct PackArgs {
     void* dst;
 };
 hipError_t launch_pack(hipStream_t s, const PackArgs& a);
+// up to kZeroSegs arrays (4-byte multiples) cleared by one kernel
+constexpr int kZeroSegs = 12;
+hipError_t launch_zero(hipStream_t s, const std::vector<std::pair<void*, size_t>>& arrays);
 
 // Per-image metadata of the last pass (the max-posterior sample): meta columns 0-6 (PMAX, CLASS,
 // ROT, TILT, PSI, XOFF, YOFF; 7 and 8 zero, filled by the sums kernel) and argmax = (class, dir, psi,

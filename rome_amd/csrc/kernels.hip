@@ -1645,6 +1645,48 @@ hipError_t launch_pack(hipStream_t s, const PackArgs& a) {
     return hipGetLastError();
 }
 
+struct ZeroArgs {
+    unsigned* p[kZeroSegs];
+    unsigned long long first[kZeroSegs + 1];  // block that starts on array q; first[n] = blocks in all
+    unsigned long long words[kZeroSegs];
+    int n;
+};
+constexpr int kZeroWords = 4096;  // a block's share of an array
+
+// The sums of a pass: two class grids and seven arrays of a few KB, each a launch of its own as a memset.
+__global__ __launch_bounds__(256) void k_zero(ZeroArgs a) {
+    int q = 0;
+    while (q + 1 < a.n && a.first[q + 1] <= blockIdx.x) ++q;
+    const unsigned long long w0 = (blockIdx.x - a.first[q]) * kZeroWords, w1 = min(w0 + kZeroWords, a.words[q]);
+    unsigned* p = a.p[q];
+    if (w1 - w0 == kZeroWords && (reinterpret_cast<uintptr_t>(p) & 15) == 0) {
+#pragma unroll
+        for (int i = 0; i < kZeroWords / 1024; ++i)
+            reinterpret_cast<uint4*>(p + w0)[threadIdx.x + 256 * i] = make_uint4(0u, 0u, 0u, 0u);
+    } else {
+        for (unsigned long long w = w0 + threadIdx.x; w < w1; w += 256) p[w] = 0u;
+    }
+}
+
+hipError_t launch_zero(hipStream_t s, const std::vector<std::pair<void*, size_t>>& arrays) {
+    if (arrays.size() > (size_t)kZeroSegs) return hipErrorInvalidValue;
+    ZeroArgs a{};
+    unsigned long long blocks = 0;
+    for (const auto& x : arrays) {
+        if (x.second % 4) return hipErrorInvalidValue;
+        if (x.second == 0) continue;
+        a.p[a.n] = static_cast<unsigned*>(x.first);
+        a.words[a.n] = x.second / 4;
+        a.first[a.n++] = blocks;
+        blocks += (x.second / 4 + kZeroWords - 1) / kZeroWords;
+    }
+    a.first[a.n] = blocks;
+    if (blocks == 0) return hipSuccess;
+    if (blocks > 0x7fffffffULL) return hipErrorInvalidValue;
+    k_zero<<<(unsigned)blocks, 256, 0, s>>>(a);
+    return hipGetLastError();
+}
+
 hipError_t launch_fct_norm(hipStream_t s, const float* FcT, int Pc, int Pc_pad, int Mpad, int Kq, float* Qc) {
     const size_t tot = (size_t)Kq * Mpad;
     k_fct_norm<<<(unsigned)((tot + 255) / 256), 256, 0, s>>>(FcT, Pc, Pc_pad, Mpad, Kq, Qc);
