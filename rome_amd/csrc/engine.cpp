@@ -3482,6 +3482,7 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
         ba.Pf = Pf;
         ba.NOR = 1;
         ba.R = chunk;  // slice = image: its "rotation" is its own index
+        ba.whole_bricks = 1;
         ba.pad = ctx->pad;
         ba.padF = ctx->padF;
         ba.c = ctx->cgrid;

@@ -298,6 +298,9 @@ struct BpArgs {
     unsigned* cursor;             // [nb]
     unsigned* ck_brick;           // [bp_chunks_max] brick of every chunk
     unsigned* sums;               // [bp_scan_sums] totals of blocks of bricks
+    // a brick's records by one block, each voxel's in one running FP32 sum (whole images: hundreds of equal values meet
+    // in the voxels around the origin, and split sums of those round differently); else in chunks, hot bricks in parallel
+    int whole_bricks = 0;
     unsigned long long* rec;      // [records] slice << 32 | pixel
     float* bp_data;
     float* bp_weight;
