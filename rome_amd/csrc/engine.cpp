@@ -379,7 +379,7 @@ struct rome_ctx {
     DevBuf<unsigned> bp_count, bp_off, bp_coff, bp_cursor, bp_ck, bp_sums;
     DevBuf<unsigned long long> bp_rec;
     // whole images at given poses (rome_backproject_images), at most 1024 at a time
-    DevBuf<double> bi_in, bi_one, bi_acc;
+    DevBuf<double> bi_in, bi_one;
     DevBuf<float2> bi_val;
     DevBuf<float> bi_wgt;
     DevBuf<int> bi_task;
@@ -3472,22 +3472,36 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
     ia.r_max = ctx->r_max;
     float *gd = ctx->bp_data.p + 2 * gn * iclass, *gw = ctx->bp_weight.p + gn * iclass;
     BpArgs ba{};
+    HIPCHK(ctx->bi_val.reserve((size_t)chunk * Pf));
+    HIPCHK(ctx->bi_wgt.reserve((size_t)chunk * Pf));
+    HIPCHK(ctx->bi_task.reserve(2 * (size_t)chunk));
+    HIPCHK(ctx->bi_one.reserve(chunk));
+    ba.K = 1;
+    ba.Pf = Pf;
+    ba.NOR = 1;
+    ba.R = chunk;  // slice = image: its "rotation" is its own index
+    ba.whole_bricks = 1;
+    ba.pad = ctx->pad;
+    ba.padF = ctx->padF;
+    ba.c = ctx->cgrid;
+    ba.r_max = ctx->r_max;
+    ba.grid_stride = gn;
+    ia.val = ctx->bi_val.p;
+    ia.wgt = ctx->bi_wgt.p;
+    ia.task_img = ctx->bi_task.p;
+    ia.task_m = ctx->bi_task.p + chunk;
+    ia.slice_w = ctx->bi_one.p;
+    ba.task_img = ia.task_img;
+    ba.task_m = ia.task_m;
+    ba.f_xy = ctx->f_xy.p;
+    ba.MC2bp = ctx->bi_wgt.p;
+    ba.slice_w = ctx->bi_one.p;
+    ba.slice_val = ctx->bi_val.p;
+    ba.bp_data = gd;
+    ba.bp_weight = gw;
+    BandPlan plan{};
     if (ctx->is3d) {
-        HIPCHK(ctx->bi_val.reserve((size_t)chunk * Pf));
-        HIPCHK(ctx->bi_wgt.reserve((size_t)chunk * Pf));
         HIPCHK(ctx->bi_rec.reserve((size_t)chunk * Pf));
-        HIPCHK(ctx->bi_task.reserve(2 * (size_t)chunk));
-        HIPCHK(ctx->bi_one.reserve(chunk));
-        ba.K = 1;
-        ba.Pf = Pf;
-        ba.NOR = 1;
-        ba.R = chunk;  // slice = image: its "rotation" is its own index
-        ba.whole_bricks = 1;
-        ba.pad = ctx->pad;
-        ba.padF = ctx->padF;
-        ba.c = ctx->cgrid;
-        ba.r_max = ctx->r_max;
-        ba.grid_stride = gn;
         ba.nbx = (ctx->padF + kBrickX - 1) / kBrickX;
         ba.nby = (ctx->pad + kBrickY - 1) / kBrickY;
         ba.nbz = (ctx->pad + kBrickZ - 1) / kBrickZ;
@@ -3498,17 +3512,6 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
         HIPCHK(ctx->bp_cursor.reserve(ba.nb_class));
         HIPCHK(ctx->bp_sums.reserve(bp_scan_sums(ba.nb_class)));
         HIPCHK(ctx->bp_ck.reserve(bp_chunks_max(ba.nb_class, chunk, ctx->Pf)));
-        ia.val = ctx->bi_val.p;
-        ia.wgt = ctx->bi_wgt.p;
-        ia.task_img = ctx->bi_task.p;
-        ia.task_m = ctx->bi_task.p + chunk;
-        ia.slice_w = ctx->bi_one.p;
-        ba.task_img = ia.task_img;
-        ba.task_m = ia.task_m;
-        ba.f_xy = ctx->f_xy.p;
-        ba.MC2bp = ctx->bi_wgt.p;
-        ba.slice_w = ctx->bi_one.p;
-        ba.slice_val = ctx->bi_val.p;
         ba.count = ctx->bp_count.p;
         ba.off = ctx->bp_off.p;
         ba.coff = ctx->bp_coff.p;
@@ -3516,12 +3519,8 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
         ba.ck_brick = ctx->bp_ck.p;
         ba.sums = ctx->bp_sums.p;
         ba.rec = ctx->bi_rec.p;
-        ba.bp_data = gd;
-        ba.bp_weight = gw;
-    } else {
-        HIPCHK(ctx->bi_acc.reserve(3 * gn * kBpCopies));
-        HIPCHK(launch_fill32(s, ctx->bi_acc.p, 0u, 2 * 3 * gn * kBpCopies));
-        ia.acc = ctx->bi_acc.p;
+    } else {  // one part: a grid point is one running FP32 sum, as in 3D
+        plan = bp_band_plan(1, 1, ctx->pad, ctx->padF, ctx->n_cu);
     }
     for (int i0 = 0; i0 < n; i0 += chunk) {
         const int m = std::min(chunk, n - i0);
@@ -3547,17 +3546,10 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
         ia.Ai = ba.Ai_fine = dm;
         ia.sx = dm + 6 * (size_t)m;
         ia.sy = dm + 7 * (size_t)m;
-        if (ctx->is3d) {
-            HIPCHK(launch_bp_image_values(s, m, ia));
-            HIPCHK(launch_backproject_binned(s, m, ba));
-        } else {
-            HIPCHK(launch_bp_images2d(s, m, ia));
-        }
+        HIPCHK(launch_bp_image_values(s, m, ia));
+        if (ctx->is3d) HIPCHK(launch_backproject_binned(s, m, ba));
+        else HIPCHK(launch_backproject_bands(s, m, ba, plan, nullptr));
         HIPCHK(hipStreamSynchronize(s));  // the staging buffers are reused by the next chunk
-    }
-    if (!ctx->is3d) {
-        HIPCHK(launch_bp_add2d(s, ctx->bi_acc.p, gn, gd, gw));
-        HIPCHK(hipStreamSynchronize(s));
     }
     return ROME_OK;
 }

@@ -462,7 +462,7 @@ __global__ __launch_bounds__(256, kPqBlocksPerCU) void k_gemm_lowp_pq(LowpGemmAr
 // epilogue runs beside the other waves' MFMAs.  An XCD keeps to one band of rows that fits its L2.  Same MFMAs over the
 // same ascending k per element as k_gemm_lowp_pq, whose 128-row tiles waited for their operands at two barriers every
 // 32 k and spent half their time so: 18432 rotations x 162000 columns x 512 k in FP16: 3548 ->
-// 2134 us, of which the matrix cores are busy 27 %; the epilogue's vector instructions bound it now.
+// 2134 us, of which the matrix cores are busy 32 %; the epilogue's vector instructions bound it now.
 // The epilogue is that of gemm_epilogue_list per wave and row block: the bound of an image lives in LDS for the block,
 // starts from the global one and is exchanged with it once a row block; columns whose minimum of E less the largest
 // ln pdf_direction of the rows is past the limit have no entry and are left at that.  Every load in the loop is

@@ -526,15 +526,10 @@ struct BpImageArgs {
     int pad, padF, c, r_max;
     float2* val;              // [n][Pf] shifted transform times the CTF
     float* wgt;               // [n][Pf] CTF^2
-    int *task_img, *task_m;   // [n] 0, 1, ..: every image its own slice (binned scatter)
+    int *task_img, *task_m;   // [n] 0, 1, ..: every image its own slice (binned scatter, bands)
     double* slice_w;          // [n] 1
-    double* acc;              // 2D: [kBpCopies][3][pad * padF] sums (re, im, weight), zero at the start
 };
-constexpr int kBpCopies = 8;
 hipError_t launch_bp_image_values(hipStream_t s, int n, const BpImageArgs& a);
-hipError_t launch_bp_images2d(hipStream_t s, int n, const BpImageArgs& a);
-// 2D sums added to the class grid (n = pad * padF elements)
-hipError_t launch_bp_add2d(hipStream_t s, const double* acc, size_t n, float* bp_data, float* bp_weight);
 hipError_t launch_store_sums(hipStream_t s, const StoreArgs& a);
 // With a.ntask_dev (device-driven pools) S is read on the device and persist_blocks blocks stride over
 // the slices (one pixel block per grid row) and over the brick chunks.

@@ -1455,7 +1455,7 @@ __global__ void k_meta(MetaArgs a) {
 // MyBackProjector::backproject of images at their own poses (apps/rome_reconstruct.cpp:104-330): the transform
 // (current_size half-plane) shifted by the image's tabulated phase, times the CTF, and the weight CTF^2; the
 // pixel set is the fine one (x = 0 column for y >= 0 only, as the reference's first_x rule), radius r_max.
-// 3D: these values are the slices of the binned scatter (backproject.hip), one slice per image; a direct
+// These values are the slices of the binned (3D) or banded (2D) scatter (backproject.hip), one slice per image; a direct
 // scatter's 24 float atomics a pixel took 1.82 ms for 400 images of 100^2, this pass and the binned one 0.2.
 DEV void bp_image_value(const BpImageArgs& a, int img, int p, float2& v, float& w) {
     const size_t nf = (size_t)img * a.F2 + a.f_nfine[p];
@@ -1478,48 +1478,6 @@ __global__ __launch_bounds__(256) void k_bp_image_values(BpImageArgs a) {
     bp_image_value(a, img, p, v, w);
     a.val[(size_t)img * a.Pf + p] = v;
     a.wgt[(size_t)img * a.Pf + p] = w;
-}
-
-// 2D: direct scatter into FP64 sums, a copy per XCD (blocks reach the XCDs round-robin) so that the images'
-// few thousand shared grid points are contended an eighth as much; the sums do not depend on the order to
-// FP32 rounding.
-__global__ __launch_bounds__(256) void k_bp_images2d(BpImageArgs a) {
-    const int img = blockIdx.x;
-    const size_t gn = (size_t)a.pad * a.padF;
-    double* acc = a.acc + 3 * gn * (blockIdx.x % kBpCopies);
-    for (int p = threadIdx.x; p < a.Pf; p += blockDim.x) {
-        const int xy = a.f_xy[p];
-        const int x = px_x(xy), y = px_y(xy);
-        if (x * x + y * y > a.r_max * a.r_max) continue;
-        float2 v;
-        float wgt;
-        bp_image_value(a, img, p, v, wgt);
-        if (!(wgt > 0.f)) continue;
-        const Coords c = map_coords(a.Ai + 6 * (size_t)img, x, y, a.c, false);
-        const float vr = v.x, vi = c.neg ? -v.y : v.y;
-        const float mfx = 1.f - c.fx, mfy = 1.f - c.fy;
-        const float dd[4] = {mfy * mfx, mfy * c.fx, c.fy * mfx, c.fy * c.fx};
-#pragma unroll
-        for (int cc = 0; cc < 4; ++cc) {
-            const size_t idx = (size_t)(c.y0 + (cc >> 1)) * a.padF + (c.x0 + (cc & 1));
-            atomicAdd(&acc[idx], (double)(dd[cc] * vr));
-            atomicAdd(&acc[gn + idx], (double)(dd[cc] * vi));
-            atomicAdd(&acc[2 * gn + idx], (double)(dd[cc] * wgt));
-        }
-    }
-}
-
-__global__ __launch_bounds__(256) void k_bp_add2d(const double* __restrict__ acc, size_t n, float* __restrict__ bp_data,
-                                                  float* __restrict__ bp_weight) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    double s[3] = {0., 0., 0.};
-    for (int k = 0; k < kBpCopies; ++k)
-#pragma unroll
-        for (int q = 0; q < 3; ++q) s[q] += acc[(3 * (size_t)k + q) * n + i];
-    bp_data[2 * i] = (float)((double)bp_data[2 * i] + s[0]);
-    bp_data[2 * i + 1] = (float)((double)bp_data[2 * i + 1] + s[1]);
-    bp_weight[i] = (float)((double)bp_weight[i] + s[2]);
 }
 
 // ------------------------------------------------------------------ launch wrappers
@@ -1939,19 +1897,6 @@ hipError_t launch_store_sums(hipStream_t s, const StoreArgs& a) {
 hipError_t launch_bp_image_values(hipStream_t s, int n, const BpImageArgs& a) {
     if (n <= 0) return hipSuccess;
     k_bp_image_values<<<dim3((a.Pf + 255) / 256, n), 256, 0, s>>>(a);
-    LAUNCH_CHECK();
-    return hipSuccess;
-}
-
-hipError_t launch_bp_images2d(hipStream_t s, int n, const BpImageArgs& a) {
-    if (n <= 0) return hipSuccess;
-    k_bp_images2d<<<n, 256, 0, s>>>(a);
-    LAUNCH_CHECK();
-    return hipSuccess;
-}
-
-hipError_t launch_bp_add2d(hipStream_t s, const double* acc, size_t n, float* bp_data, float* bp_weight) {
-    k_bp_add2d<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(acc, n, bp_data, bp_weight);
     LAUNCH_CHECK();
     return hipSuccess;
 }

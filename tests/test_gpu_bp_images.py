@@ -1,4 +1,4 @@
-"""rome_backproject_images (binned scatter in 3D, FP64 sums in 2D) against the FP64 oracle's backprojection: one
+"""rome_backproject_images (binned scatter in 3D, bands in 2D) against the FP64 oracle's backprojection: one
 image, a pool past the 1024 images of one device pass, with and without CTF images, into the second of two classes
 and on top of an earlier call.  Corner weights and values are FP32 products of a few terms (a few 2^-24 each) and a
 voxel's sum takes at most a few thousand of them: 1e-5 relative L2, as for the E-step's grids."""
@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dim,ori,cur,n,ctf", [(3, 16, 16, 1, True), (3, 24, 18, 70, True), (3, 16, 16, 1100, False),
-                                               (3, 56, 56, 40, True), (2, 16, 16, 1, True), (2, 24, 18, 70, False), (2, 20, 20, 1100, True)])
+                                               (3, 56, 56, 40, True), (2, 16, 16, 1, True), (2, 24, 18, 70, False), (2, 20, 20, 1100, True), (2, 100, 100, 9, True)])
 def test_backproject_images(engine, dim, ori, cur, n, ctf):
     print(f"[bp images dim={dim} ori={ori} cur={cur} n={n} ctf={ctf}]", flush=True)
     engine.configure(ref_dim=dim, ori_size=ori, current_size=cur, coarse_size=cur, nr_classes=2, nr_groups=1,
