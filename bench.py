@@ -525,12 +525,15 @@ def main():
     # psi and psi + 180 deg share one half-table row in the mixed arm when the in-plane sampling pairs them
     # (an even count of psi steps per half turn, the half table a multiple of 128 rows, >= 8 shifts)
     paired = head_prec != "fp32" and prob["nr_psi"] % 8 == 0 and (M // 2) % 128 == 0 and T >= 8
-    lowp = ("k_gemm_lowp_pq<%s, " + ("list>" if listed else "E>")) if paired else \
+    # pools of at least four blocks a CU hold the columns in LDS (96 a block, the half table in bands of 2.5 MB)
+    cols = paired and listed and B * T // 96 * 4 >= 4 * 256
+    lowp = "k_gemm_pq_cols<%s>" if cols else ("k_gemm_lowp_pq<%s, " + ("list>" if listed else "E>")) if paired else \
         ("k_gemm_lowp_list<%s>" if listed else "k_gemm_lowp<%s>")
     kname = "k_coarse_gemm (coarse cross term, FP32 MFMA)" if head_prec == "fp32" else \
         (lowp % head_prec) + " (coarse cross term, %s MFMA%s)" % (head_prec.upper(),
                                                                   ", psi/psi+180 paired" if paired else "")
-    row = ("k_gemm_lowp_pq<_Float16, true>" if paired else "k_gemm_lowp_list<_Float16>")
+    row = "k_gemm_pq_cols<_Float16, 3>" if cols else \
+        ("k_gemm_lowp_pq<_Float16, true>" if paired else "k_gemm_lowp_list<_Float16>")
     traffic = measured_traffic(row) if head_prec == "fp16" and listed else None
     roofline = {"kernel": kname, "bound": "mfma",
                 "achieved": round(gemm_tflops, 2), "peak": peak, "unit": "TFLOP/s",
