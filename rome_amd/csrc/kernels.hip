@@ -587,7 +587,9 @@ __global__ __launch_bounds__(1024) void k_task_count_keys(int* __restrict__ keys
     }
 }
 
-// Emission from the sorted keys: block q of the image is key q; a task starts at each new rotation.
+// Emission from the sorted keys: block q of the image is key q; a task starts at each new rotation.  An image with more
+// samples than its row of keys (cnt > cap: a device-driven pool, which is aborted) was counted as none and emits none: the
+// task and block buffers hold cap entries an image.
 __global__ __launch_bounds__(1024) void k_task_emit_keys(const int* __restrict__ keys, const int* __restrict__ cnt,
                                                          int cap, int T, const long long* __restrict__ task_off,
                                                          const long long* __restrict__ blk_off,
@@ -598,6 +600,7 @@ __global__ __launch_bounds__(1024) void k_task_emit_keys(const int* __restrict__
     __shared__ int base;
     const int img = blockIdx.x, tid = threadIdx.x;
     const int c = cnt[img];
+    if (c > cap) return;
     const int* k = keys + (size_t)img * cap;
     const long long bt = task_off[img], bb = blk_off[img];
     if (tid == 0) base = 0;
