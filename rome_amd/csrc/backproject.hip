@@ -385,23 +385,64 @@ __global__ __launch_bounds__(256, WHOLE ? 4 : 5) void k_bp_brick(BpArgs a, int n
     }
 }
 
-// 2D: block (band, class, part) adds the bilinear corners that fall on its rows [y0, y0 + rows) of the class grid,
-// over the slices of its share of the tasks, in LDS; one part adds its band to the grids, several leave partial
-// sums for k_bp_band_add.  Per tile of slices the block lists those of its class, then works through them one after
-// the other, a corner of all pixels at a time: the pixels of a slice are two voxels apart, so no two of them have
-// the same base voxel and the additions need no atomics (LDS float atomics take about a lane per two cycles: 298
+// 2D: block (band, slot) adds the bilinear corners that fall on its rows [y0, y0 + rows) of a class grid, over the
+// slices of the slot's share of the class, in LDS; a class of one slot adds its band to the grids, the slots of
+// several leave partial sums for k_bp_band_add.  Per tile of slices the block lists those of its class, then works through
+// them one after the other, a corner of all pixels at a time: the pixels of a slice are two voxels apart, so no two of
+// them have the same base voxel and the additions need no atomics (LDS float atomics take about a lane per two cycles: 298
 // us).  A band is as many rows as fit in LDS (all 131 for 64^2 images at full resolution); with several, each works
 // out every pixel's coordinates for the corners it keeps.  1000 images of 64^2 in ten classes: 54 us (direct
 // scatter: 1.04 ms with the slices' own sums, 24 M float atomics to L2).
+// The slots follow the classes' slices (slice_cnt, counted by k_post): the same number for every class left one
+// that takes all of 200 images among 20 classes to two blocks of a slice a 1.15 us (6400 slices of 64^2: 7.3 ms, 0.53 now).
 constexpr int kBandThreads = 1024;
+constexpr int kBandParts = 32;  // most slots of a class: k_bp_band_add reads them all
+struct BandSlots {
+    int first, parts;  // of a class
+};
+// By the first wave: lane k has class k's share of the slots.  A slot each, the others by the number of slices, and
+// at least four slices for each (a block clears and writes its whole band); classes without a slice have none.
+DEV BandSlots band_slots(const unsigned* cnt, int K, int slots) {
+    const int lane = threadIdx.x & 63;
+    const unsigned c = lane < K ? cnt[lane] : 0u;
+    unsigned long long all = c;
+    for (int o = 32; o > 0; o >>= 1) all += __shfl_xor(all, o, 64);
+    int p = 0;
+    if (c) p = min(min(1 + (int)((unsigned long long)(slots - K) * c / all), kBandParts), (int)((c + 3u) / 4u));
+    int in = p;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(in, o, 64);
+        if (lane >= o) in += v;
+    }
+    return {in - p, p};
+}
+
 __global__ __launch_bounds__(kBandThreads) void k_bp_band(BpArgs a, long long S_host, int rows_max, float* work) {
     extern __shared__ float box[];  // [3][rows * padF]
     __shared__ int l_s[kBandThreads], l_img[kBandThreads], l_r[kBandThreads];  // the tile's slices of this class:
     __shared__ double l_w[kBandThreads];                                       // slice, image, rotation, weight
-    __shared__ int cnt;
+    __shared__ int cnt, s_slot[3];
     const long long ntask = bp_slices(a, S_host) / a.NOR;
     if (ntask == 0) return;
-    const int tid = threadIdx.x, k = blockIdx.y, part = blockIdx.z, parts = gridDim.z;
+    const int tid = threadIdx.x, slot = blockIdx.y;
+    int k = 0, part = 0, parts = 1;
+    if (a.slice_cnt) {
+        if (tid == 0) s_slot[2] = 0;
+        __syncthreads();
+        if (tid < 64) {
+            const BandSlots b = band_slots(a.slice_cnt, a.K, gridDim.y);
+            if (slot >= b.first && slot < b.first + b.parts) {
+                s_slot[0] = tid;
+                s_slot[1] = slot - b.first;
+                s_slot[2] = b.parts;
+            }
+        }
+        __syncthreads();
+        k = s_slot[0];
+        part = s_slot[1];
+        parts = s_slot[2];
+        if (parts == 0) return;
+    }
     const int y0 = blockIdx.x * rows_max, rows = min(rows_max, a.pad - y0), nb = rows * a.padF;
     float *br = box, *bi = box + nb, *bw = box + 2 * nb;
     for (int i = tid; i < 3 * nb; i += kBandThreads) box[i] = 0.f;
@@ -478,7 +519,7 @@ __global__ __launch_bounds__(kBandThreads) void k_bp_band(BpArgs a, long long S_
             gw[i] += bw[i];
         }
     } else {
-        float* o = work + 3 * gn * ((size_t)part * a.K + k) + g0;
+        float* o = work + 3 * gn * (size_t)slot + g0;
         for (int i = tid; i < nb; i += kBandThreads) {
             o[i] = br[i];
             o[gn + i] = bi[i];
@@ -487,16 +528,24 @@ __global__ __launch_bounds__(kBandThreads) void k_bp_band(BpArgs a, long long S_
     }
 }
 
-// The parts' sums of a class (blockIdx.y) added to its grids.
-__global__ __launch_bounds__(256) void k_bp_band_add(BpArgs a, long long S_host, int parts,
+// The slots' sums of a class of several (blockIdx.y) added to its grids.
+__global__ __launch_bounds__(256) void k_bp_band_add(BpArgs a, long long S_host, int slots,
                                                      const float* __restrict__ work) {
+    __shared__ BandSlots s_b;
+    if (bp_slices(a, S_host) == 0) return;
     const size_t gn = a.grid_stride, i = (size_t)blockIdx.x * 256 + threadIdx.x;
     const int k = blockIdx.y;
-    if (i >= gn || bp_slices(a, S_host) == 0) return;
+    if (threadIdx.x < 64) {
+        const BandSlots b = band_slots(a.slice_cnt, a.K, slots);
+        if ((int)threadIdx.x == k) s_b = b;
+    }
+    __syncthreads();
+    if (i >= gn || s_b.parts < 2) return;
+    const float* w = work + 3 * gn * (size_t)s_b.first + i;
     float s[3] = {0.f, 0.f, 0.f};
-    for (int part = 0; part < parts; ++part)
+    for (int part = 0; part < s_b.parts; ++part)
 #pragma unroll
-        for (int q = 0; q < 3; ++q) s[q] += work[(3 * ((size_t)part * a.K + k) + q) * gn + i];
+        for (int q = 0; q < 3; ++q) s[q] += w[(3 * (size_t)part + q) * gn];
     a.bp_data[2 * (gn * k + i)] += s[0];
     a.bp_data[2 * (gn * k + i) + 1] += s[1];
     a.bp_weight[gn * k + i] += s[2];
@@ -511,29 +560,28 @@ void bp_scan(hipStream_t s, const BpArgs& a, int nb) {
 
 }  // namespace
 
-BandPlan bp_band_plan(int n, int K, int pad, int padF, int n_cu) {
+BandPlan bp_band_plan(int K, int pad, int padF, int n_cu) {
     BandPlan b;
     const int fit = std::max(1, (138 << 10) / (12 * padF));  // rows in LDS beside the block's list
     b.bands = (pad + fit - 1) / fit;
     b.rows = (pad + b.bands - 1) / b.bands;
-    // parts: a block per CU, but at least four images for each (a block clears and writes its whole band)
-    b.parts = std::max(1, std::min({n_cu / (K * b.bands), n / (4 * K), 32}));
-    b.work = b.parts > 1 ? (size_t)3 * b.parts * K * pad * padF : 0;
+    b.slots = std::max(K, std::min(n_cu / b.bands, kBandParts * K));  // a block per CU
+    b.work = b.slots > K ? (size_t)3 * b.slots * pad * padF : 0;
     return b;
 }
 
 hipError_t launch_backproject_bands(hipStream_t s, long long S, const BpArgs& a, const BandPlan& b, float* work) {
     if (!a.ntask_dev && S <= 0) return hipSuccess;
     const size_t lds = (size_t)12 * b.rows * a.padF;
-    if (lds + 20 * kBandThreads + 16 > ((size_t)160 << 10) || b.bands < 1 || b.parts < 1 || (b.parts > 1 && !work) ||
-        a.grid_stride != (size_t)a.pad * a.padF)
+    if (lds + 20 * kBandThreads + 16 > ((size_t)160 << 10) || b.bands < 1 || a.K > 64 || b.slots < a.K ||
+        (a.slice_cnt ? b.slots > a.K && !work : b.slots != 1) || a.grid_stride != (size_t)a.pad * a.padF)
         return hipErrorInvalidValue;
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_bp_band),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    k_bp_band<<<dim3((unsigned)b.bands, (unsigned)a.K, (unsigned)b.parts), kBandThreads, lds, s>>>(a, S, b.rows, work);
-    if (b.parts > 1)
-        k_bp_band_add<<<dim3((unsigned)((a.grid_stride + 255) / 256), (unsigned)a.K), 256, 0, s>>>(a, S, b.parts, work);
+    k_bp_band<<<dim3((unsigned)b.bands, (unsigned)b.slots), kBandThreads, lds, s>>>(a, S, b.rows, work);
+    if (b.slots > a.K)
+        k_bp_band_add<<<dim3((unsigned)((a.grid_stride + 255) / 256), (unsigned)a.K), 256, 0, s>>>(a, S, b.slots, work);
     return hipGetLastError();
 }
 

@@ -374,7 +374,8 @@ struct rome_ctx {
     // binned backprojection
     static constexpr size_t kBinnedBytes = (size_t)40 << 30;  // slice values + records per batch
     DevBuf<float2> slice_val;
-    DevBuf<float> bp_work;  // partial bands of 2D grids
+    DevBuf<float> bp_work;       // partial bands of 2D grids
+    DevBuf<unsigned> slice_cnt;  // slices of every 2D class
     DevBuf<double> slice_w;
     DevBuf<unsigned> bp_count, bp_off, bp_coff, bp_cursor, bp_ck, bp_sums;
     DevBuf<unsigned long long> bp_rec;
@@ -1596,11 +1597,17 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
             HIPCHK(sized(ctx->slice_w, (size_t)S));
             pp.slice_val = ctx->slice_val.p;
             pp.slice_w = ctx->slice_w.p;
+            if (!ctx->is3d) {
+                HIPCHK(ctx->slice_cnt.reserve(ctx->K));
+                pp.slice_cnt = ctx->slice_cnt.p;
+            }
         }
         stage_begin(ctx, 8);
         hipError_t pe = hipErrorNotSupported;
+        if (dd || binned)
+            HIPCHK(launch_zero(s, {{ctx->wnorm.p, n * sizeof(double)},
+                                   {pp.slice_cnt, pp.slice_cnt ? ctx->K * sizeof(unsigned) : 0}}));
         if (dd) {
-            HIPCHK(launch_fill32(s, ctx->wnorm.p, 0u, 2 * (size_t)n));
             if (binned && by_slice)
                 HIPCHK(launch_post_slices(s, ntasks, NOR, NOT, pp, ctx->persist_blocks(2), ctx->guess_tasks(n, ntasks)));
             else if (binned)
@@ -1610,10 +1617,7 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
             pd.slice_w = nullptr;
             pe = launch_post(s, n, NOR, NOT, pd);
         } else {
-            if (binned) {
-                HIPCHK(launch_fill32(s, ctx->wnorm.p, 0u, 2 * (size_t)n));
-                pe = launch_post_slices(s, ntasks, NOR, NOT, pp);
-            }
+            if (binned) pe = launch_post_slices(s, ntasks, NOR, NOT, pp);
             if (pe == hipErrorNotSupported) pe = launch_post(s, n, NOR, NOT, pp);
         }
         HIPCHK(pe);
@@ -1668,8 +1672,9 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
             if (ctx->is3d) {
                 HIPCHK(launch_backproject_binned(s, S, ba, ctx->persist_blocks(3)));
             } else {
-                const BandPlan plan = bp_band_plan(n, ctx->K, ctx->pad, ctx->padF, ctx->n_cu);
+                const BandPlan plan = bp_band_plan(ctx->K, ctx->pad, ctx->padF, ctx->n_cu);
                 HIPCHK(ctx->bp_work.reserve(plan.work));
+                ba.slice_cnt = ctx->slice_cnt.p;
                 HIPCHK(launch_backproject_bands(s, S, ba, plan, ctx->bp_work.p));
             }
             stage_end(ctx, 10);
@@ -3519,8 +3524,9 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
         ba.ck_brick = ctx->bp_ck.p;
         ba.sums = ctx->bp_sums.p;
         ba.rec = ctx->bi_rec.p;
-    } else {  // one part: a grid point is one running FP32 sum, as in 3D
-        plan = bp_band_plan(1, 1, ctx->pad, ctx->padF, ctx->n_cu);
+    } else {  // one slot: a grid point is one running FP32 sum, as in 3D
+        plan = bp_band_plan(1, ctx->pad, ctx->padF, ctx->n_cu);
+        plan.slots = 1;
     }
     for (int i0 = 0; i0 < n; i0 += chunk) {
         const int m = std::min(chunk, n - i0);

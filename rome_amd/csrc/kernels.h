@@ -271,6 +271,7 @@ struct PostArgs {
     // binned / banded backprojection: slices go to HBM instead of the grids (null: direct scatter)
     float2* slice_val;          // [ntask * NOR][Pf]
     double* slice_w;            // [ntask * NOR]
+    unsigned* slice_cnt = nullptr;  // [K] 2D: slices with weight of every class (zeroed by the caller)
     // device-driven pools (null otherwise): the task total on the device, the slice buffer's capacity
     // (pools with more slices take the direct scatter) and the pool abort flag
     const long long* ntask_dev = nullptr;
@@ -292,6 +293,7 @@ struct BpArgs {
     const float* MC2bp;           // [n][Pf]
     const double* slice_w;        // [S] sum of the slice's normalised significant weights (0: none)
     const float2* slice_val;      // [S][Pf]
+    const unsigned* slice_cnt = nullptr;  // [K] bands: slices with weight of every class; null: one class, one slot
     unsigned* count;              // [nb]
     unsigned* off;                // [nb + 1]
     unsigned* coff;               // [nb + 1] chunks of the brick kernel per brick, prefix sums
@@ -536,12 +538,12 @@ hipError_t launch_store_sums(hipStream_t s, const StoreArgs& a);
 inline size_t bp_scan_sums(size_t nb) { return 2 * ((nb + 1023) / 1024); }
 size_t bp_chunks_max(size_t nb, long long S, int Pf);  // chunks S slices of Pf pixels can make over nb bricks
 hipError_t launch_backproject_binned(hipStream_t s, long long S, const BpArgs& a, int persist_blocks = 0);
-// 2D: bands of grid rows accumulated in LDS, the slices of a class split over parts blocks per band
+// 2D: bands of grid rows accumulated in LDS, blocks (slots) of a band given to the classes by their slices
 struct BandPlan {
-    int rows, bands, parts;
-    size_t work;  // floats of partial sums (0: one part, added to the grids directly)
+    int rows, bands, slots;
+    size_t work;  // floats of partial sums (0: a slot a class, added to the grids directly)
 };
-BandPlan bp_band_plan(int n, int K, int pad, int padF, int n_cu);
+BandPlan bp_band_plan(int K, int pad, int padF, int n_cu);
 hipError_t launch_backproject_bands(hipStream_t s, long long S, const BpArgs& a, const BandPlan& plan, float* work);
 // M-step reconstruction (reconstruct.hip)
 hipError_t rc_fold(hipStream_t s, double2* data, double* weight, int Dz, int P, int PF);

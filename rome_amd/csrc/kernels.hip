@@ -1049,6 +1049,7 @@ __global__ __launch_bounds__(NT) void k_post(PostArgs a) {
     __shared__ double red[NT / 64];
     __shared__ double shell[kMaxShell];
     __shared__ double s_pdfk[kMaxK], s_px[kMaxK], s_py[kMaxK];
+    __shared__ unsigned s_cnt[kMaxK];
     // device-driven: aborted, or the other form's (slices that fit the buffer are binned)
     if (a.ntask_dev && (*a.abort || (*a.ntask_dev * NOR <= a.slice_cap) != BINNED)) return;
     const int img = blockIdx.x, tid = threadIdx.x;
@@ -1059,7 +1060,10 @@ __global__ __launch_bounds__(NT) void k_post(PostArgs a) {
 #pragma unroll
     for (int j = 0; j < PPT; ++j) wsig[j] = 0.;
     for (int s = tid; s < a.oriF; s += NT) shell[s] = 0.;
-    for (int k = tid; k < a.K; k += NT) s_pdfk[k] = s_px[k] = s_py[k] = 0.;
+    for (int k = tid; k < a.K; k += NT) {
+        s_pdfk[k] = s_px[k] = s_py[k] = 0.;
+        s_cnt[k] = 0u;
+    }
     double t_sumw = 0., t_off = 0.;  // thread 0 accumulators
     __syncthreads();
     const float2* X = a.Xf + (size_t)img * a.Pf;
@@ -1156,7 +1160,10 @@ __global__ __launch_bounds__(NT) void k_post(PostArgs a) {
                         if (p < a.Pf) V[p] = acc[j];
                     }
                 }
-                if (tid == 0) a.slice_w[sl] = wslice;
+                if (tid == 0) {
+                    a.slice_w[sl] = wslice;
+                    s_cnt[k] += wslice > 0.;
+                }
             } else if (wslice > 0.) {
                 // trilinear scatter of the slice (MyBackProjector::backproject, src/reconstruct.cpp:977-1164)
                 float* gd = a.bp_data + a.grid_stride * 2 * k;
@@ -1219,6 +1226,7 @@ __global__ __launch_bounds__(NT) void k_post(PostArgs a) {
         if (s_pdfk[kk] != 0.) atomicAdd(&a.wsum_pdf_class[kk], s_pdfk[kk]);
         if (s_px[kk] != 0.) atomicAdd(&a.wsum_prior_x[kk], s_px[kk]);
         if (s_py[kk] != 0.) atomicAdd(&a.wsum_prior_y[kk], s_py[kk]);
+        if (BINNED && a.slice_cnt && s_cnt[kk]) atomicAdd(&a.slice_cnt[kk], s_cnt[kk]);
     }
     if (tid == 0) {
         a.wnorm[img] = tot;
