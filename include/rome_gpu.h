@@ -288,7 +288,7 @@ int rome_get_execution_stats(rome_ctx* ctx, long long* out6);
  * keeps the fastest grid of each kernel for the context.  chosen [4] receives the grids (blocks),
  * stage_ms [4][4] the measured stage times per candidate.  The runs add to the E-step sums: call
  * rome_reset_sums afterwards.  rome_set_persistent_grids sets the four grids directly (0: the default,
- * 2, 8, 2 and 32 blocks per CU) and forgets the task and rotation totals of earlier pools, from which
+ * 2, 8, 2 and 32 blocks per CU; those of the post slices stand for the work of 1024 threads) and forgets the task and rotation totals of earlier pools, from which
  * the first launches of the fine diff2, the projection and the post slices are sized (the next pool's
  * are then sized from 4 per image, and what exceeds them goes through the work queue / the tails). */
 int rome_autotune(rome_ctx* ctx, const rome_device_images* images, const int* sig_keys, const int* sig_cnt, int cap,

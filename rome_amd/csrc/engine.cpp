@@ -455,11 +455,9 @@ struct rome_ctx {
     double last_launch_ms = 0., last_wait_ms = 0.;  // host time issuing the last device-driven pool / waiting
     static constexpr size_t kPfineBytes = (size_t)32 << 30;  // fine projections of a device-driven pool
     // pool_flags: [0] abort, [1] fine diff2 queue head, [2] invalid given keys, [3] unused, then 64-bit
-    // work counters from word 4: 8 per-XCD of the fine projection's tail, 8 of the post slices' tail
-    static constexpr int kPoolFlagWords = 4 + 2 * 16;
-    unsigned long long* work_counters(int first) const {
-        return reinterpret_cast<unsigned long long*>(pool_flags.p + 4) + first;
-    }
+    // work counters from word 4: 8 per-XCD of the fine projection's tail
+    static constexpr int kPoolFlagWords = 4 + 2 * 8;
+    unsigned long long* work_counters() const { return reinterpret_cast<unsigned long long*>(pool_flags.p + 4); }
     // Device-driven launches: the first launch of the fine diff2, the projection and the post slices
     // covers the counts of the pools before (10 % above the largest of them, decaying; the blocks past a
     // pool's own count return at once), a tail kernel or the work queue the rest.  Without history: 4
@@ -1470,7 +1468,7 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
     stage_begin(ctx, 5);
     HIPCHK(launch_project_fine(s, ctx->grids.p, ctx->is3d ? ctx->cube.p : nullptr, ctx->grid_n, ctx->pad, ctx->padF,
                                ctx->cgrid, ctx->is3d, ctx->Ai_f.p, ctx->R, NOR, ctx->ulist.p, U,
-                               dd ? ctx->ucount.p : nullptr, ctx->work_counters(0), ctx->persist_blocks(1),
+                               dd ? ctx->ucount.p : nullptr, ctx->work_counters(), ctx->persist_blocks(1),
                                ctx->guess_U(n, U), ctx->f_xy.p, ctx->Pf, ctx->r_max, ctx->Pfine.p));
     stage_end(ctx, 5);
     FineArgs fa;
@@ -1588,7 +1586,6 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
             pp.ntask_dev = ctx->task_off.p + n;
             pp.abort = ctx->pool_flags.p;
             pp.slice_cap = binned ? slice_cap : -1;  // -1: the direct scatter takes every pool
-            pp.xq = ctx->work_counters(8);
         }
         pp.slice_val = nullptr;
         pp.slice_w = nullptr;

@@ -277,7 +277,6 @@ struct PostArgs {
     const long long* ntask_dev = nullptr;
     long long slice_cap = 0;
     const int* abort = nullptr;
-    unsigned long long* xq = nullptr;  // 8 per-XCD work counters of the per-slice kernel (zero at launch)
 };
 
 // Binned 3D backprojection (backproject.hip)
