@@ -1140,7 +1140,8 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
             HIPCHK(launch_weights_fine(s, n, wp_exact, ctx->D2c.p, ctx->blk_task.p, ctx->blk_t.p, ctx->task_m.p,
                                        ctx->blk_off.p, 1, wc_exact, cand, TailArgs{ctx->c_tail.p, ctx->c_dmin1.p}, sg));
         else if (L)
-            HIPCHK(launch_weights_list(s, n, wp, *L, ctx->C2c.p, ctx->emin_key.p, wc, sg, cand, ctx->list_scan()));
+            HIPCHK(launch_weights_list(s, n, wp, *L, ctx->C2c.p, ctx->emin_key.p, wc, sg, cand, ctx->list_scan(),
+                                       ctx->n_cu));
         else
             HIPCHK(launch_weights_coarse(s, n, wp, ctx->E.p, ctx->C2c.p, ctx->emin_key.p, wc, sg, cand));
         stage_end(ctx, 3);

@@ -433,7 +433,7 @@ struct ListScanArgs {
 };
 hipError_t launch_weights_list(hipStream_t s, int n, const WeightParams& wp, const ListArgs& list, const double* C2c,
                                const int* emin_key, const WeightOutArgs& wo, const SigArgs& sig,
-                               const CandArgs& cand, const ListScanArgs& scan);
+                               const CandArgs& cand, const ListScanArgs& scan, int n_cu);
 // reach[img] = kWeightWindow + (max - min of ln pdf_offset over (class, translation)) + slack,
 // +inf when a pdf_offset is zero; clears the images' histograms of the list scan
 hipError_t launch_list_reach(hipStream_t s, int n, const WeightParams& wp, float* reach, const ListScanArgs& scan);

@@ -18,7 +18,8 @@
 //   mark   : (coarse) the samples with w >= threshold: their keys m*T + t per image, or bits of
 //            the significance mask.
 // When an image has more candidates than the list holds, the entries down to the crossing bucket (and the mark
-// margin) are collected in one more pass; if those do not fit either, select / mark rescan the entries.
+// margin) are collected in one more pass, unless the buckets already tell that those do not fit either; then select /
+// mark rescan the entries.
 //
 // A coarse list longer than kSplitList is scanned by kListParts blocks (k_list_scan) ahead of its image's
 // block: a broad posterior leaves hundreds of thousands of entries inside the window, each an FP64 exponential.
@@ -77,6 +78,7 @@ struct WShared {
     int nmark;
     int done;
     int bstar, blast;
+    long long least;  // entries down to the crossing bucket's end
     double lo, width, mbefore;
     long long cbefore;
     double thr;
@@ -350,6 +352,7 @@ __device__ void weight_pass(int img, size_t count, double cimg, const WeightPara
                 }
                 sh.mbefore = m;
                 sh.cbefore = c;
+                sh.least = c + sh.hcnt[bs];
                 sh.lo = sh.lo + bs * sh.width;
                 sh.done = (sh.hcnt[bs] <= (unsigned)kSortCap || level >= 2) ? 1 : 0;
                 sh.width = sh.width / (double)kBinCount;
@@ -364,10 +367,11 @@ __device__ void weight_pass(int img, size_t count, double cimg, const WeightPara
         if (!listed && level == 0) {
             // everything select and mark can still ask for: w >= thr_mark >= the bucket's least weight exp(-margin)
             const double need = hi + wp.mark_margin + 1e-6;
+            const bool fits = need < kWin && sh.least <= cand.cap;  // as far as the buckets tell
             __syncthreads();
             if (tid == 0) sh.ncand = 0;
             __syncthreads();
-            if (need < kWin)
+            if (fits)
                 for_window(pre_bound(u0, need), [&](size_t e) {
                     double d;
                     int m, t;
@@ -386,7 +390,7 @@ __device__ void weight_pass(int img, size_t count, double cimg, const WeightPara
                 });
             __syncthreads();
             ncand = sh.ncand;
-            listed = need < kWin && ncand <= cand.cap;
+            listed = fits && ncand <= cand.cap;
         }
         if (sh.done == 1) {
             visit(lo, hi, [&](double w, double, long long e) {
@@ -692,11 +696,14 @@ __global__ __launch_bounds__(256) void k_list_scan(WeightParams wp, ListArgs L, 
 
 // Coarse weights from the list the cross-term GEMM kept (every entry within kWin of the minimum
 // u, and more): entries i = 0 .. count-1 of the image's list, argmax keys in the reference's order.
-// 512 threads, two blocks per CU without spills (1024 at 64 VGPRs spilled 44 registers).
-constexpr int kListThreads = 512;
-__global__ __launch_bounds__(kListThreads, 4) void k_weights_list(WeightParams wp, ListArgs L, const double* __restrict__ C2c,
-                                                               const int* __restrict__ emin_key, WeightOut wo,
-                                                               SigArgs sig, Cand cand, ListScanArgs scan) {
+// 1024 threads an image for pools of no more images than CUs; else 512, two blocks per CU without spills (1024 at 64
+// VGPRs spilled 44 registers).  Either way a CU's 16 waves: 50 images with lists of 746 thousand entries 9.5 ms with 512
+// threads, 4.6 with 1024; lists past 65536 by 1024 threads in a launch of their own cost 2000 images with 9 thousand
+// on average 0.45 ms against 0.36, one launch waiting for the other.
+template <int NT>
+__global__ __launch_bounds__(NT, 4) void k_weights_list(WeightParams wp, ListArgs L, const double* __restrict__ C2c,
+                                                        const int* __restrict__ emin_key, WeightOut wo, SigArgs sig,
+                                                        Cand cand, ListScanArgs scan) {
     __shared__ WShared sh;
     const int img = blockIdx.x;
     const int cnt = L.count[img];
@@ -722,10 +729,10 @@ __global__ __launch_bounds__(kListThreads, 4) void k_weights_list(WeightParams w
     auto key = [&](size_t, int m, int t) { return (long long)m * T + t; };
     const bool split = cnt > kSplitList;
     if (!split) scan.part = nullptr;
-    weight_pass<kListThreads>(img, (size_t)cnt, C2c[img], wp, get, pre, key, wo, sh, sig, cand, emin_key,
-                              TailArgs{nullptr, nullptr}, scan);
+    weight_pass<NT>(img, (size_t)cnt, C2c[img], wp, get, pre, key, wo, sh, sig, cand, emin_key,
+                    TailArgs{nullptr, nullptr}, scan);
     if (split)  // the scan of a rerun of this pool's weights starts from zero again
-        for (int b = threadIdx.x; b < kBinCount; b += kListThreads) {
+        for (int b = threadIdx.x; b < kBinCount; b += NT) {
             scan.hsum[(size_t)img * kBinCount + b] = 0.;
             scan.hcnt[(size_t)img * kBinCount + b] = 0u;
         }
@@ -795,13 +802,15 @@ hipError_t launch_weights_coarse(hipStream_t s, int n, const WeightParams& wp, c
 
 hipError_t launch_weights_list(hipStream_t s, int n, const WeightParams& wp, const ListArgs& list, const double* C2c,
                                const int* emin_key, const WeightOutArgs& wo, const SigArgs& sig,
-                               const CandArgs& c, const ListScanArgs& scan) {
+                               const CandArgs& c, const ListScanArgs& scan, int n_cu) {
     if (wp.K * wp.T > kMaxKT) return hipErrorInvalidValue;
     if (sig.keys && ((long long)wp.Mtot * wp.T > 0x7fffffffLL || sig.cap > kSigCap)) return hipErrorInvalidValue;
     WeightOut o{wo.dmin, wo.sumw, wo.maxw, wo.amax, wo.thr, wo.nsig, wo.status, wo.tail};
+    const Cand cd{c.w, c.du, c.e, c.cap};
     if (list.cap > kSplitList)
         k_list_scan<<<dim3(n, kListParts), 256, off_bytes(wp), s>>>(wp, list, C2c, emin_key, scan);
-    k_weights_list<<<n, kListThreads, off_bytes(wp), s>>>(wp, list, C2c, emin_key, o, sig, Cand{c.w, c.du, c.e, c.cap}, scan);
+    if (n <= n_cu) k_weights_list<1024><<<n, 1024, off_bytes(wp), s>>>(wp, list, C2c, emin_key, o, sig, cd, scan);
+    else k_weights_list<512><<<n, 512, off_bytes(wp), s>>>(wp, list, C2c, emin_key, o, sig, cd, scan);
     return hipGetLastError();
 }
 
