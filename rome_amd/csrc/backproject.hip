@@ -425,24 +425,19 @@ __global__ __launch_bounds__(kBandThreads) void k_bp_band(BpArgs a, long long S_
     const long long ntask = bp_slices(a, S_host) / a.NOR;
     if (ntask == 0) return;
     const int tid = threadIdx.x, slot = blockIdx.y;
-    int k = 0, part = 0, parts = 1;
-    if (a.slice_cnt) {
-        if (tid == 0) s_slot[2] = 0;
-        __syncthreads();
-        if (tid < 64) {
-            const BandSlots b = band_slots(a.slice_cnt, a.K, gridDim.y);
-            if (slot >= b.first && slot < b.first + b.parts) {
-                s_slot[0] = tid;
-                s_slot[1] = slot - b.first;
-                s_slot[2] = b.parts;
-            }
+    if (tid == 0) s_slot[2] = 0;
+    __syncthreads();
+    if (tid < 64) {
+        const BandSlots b = band_slots(a.slice_cnt, a.K, gridDim.y);
+        if (slot >= b.first && slot < b.first + b.parts) {
+            s_slot[0] = tid;
+            s_slot[1] = slot - b.first;
+            s_slot[2] = b.parts;
         }
-        __syncthreads();
-        k = s_slot[0];
-        part = s_slot[1];
-        parts = s_slot[2];
-        if (parts == 0) return;
     }
+    __syncthreads();
+    const int k = s_slot[0], part = s_slot[1], parts = s_slot[2];
+    if (parts == 0) return;
     const int y0 = blockIdx.x * rows_max, rows = min(rows_max, a.pad - y0), nb = rows * a.padF;
     float *br = box, *bi = box + nb, *bw = box + 2 * nb;
     for (int i = tid; i < 3 * nb; i += kBandThreads) box[i] = 0.f;
@@ -574,7 +569,7 @@ hipError_t launch_backproject_bands(hipStream_t s, long long S, const BpArgs& a,
     if (!a.ntask_dev && S <= 0) return hipSuccess;
     const size_t lds = (size_t)12 * b.rows * a.padF;
     if (lds + 20 * kBandThreads + 16 > ((size_t)160 << 10) || b.bands < 1 || a.K > 64 || b.slots < a.K ||
-        (a.slice_cnt ? b.slots > a.K && !work : b.slots != 1) || a.grid_stride != (size_t)a.pad * a.padF)
+        !a.slice_cnt || (b.slots > a.K && !work) || a.grid_stride != (size_t)a.pad * a.padF)
         return hipErrorInvalidValue;
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_bp_band),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

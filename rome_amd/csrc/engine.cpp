@@ -3469,42 +3469,41 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
     ia.f_xy = ctx->f_xy.p;
     ia.sintab = ctx->sintab.p;
     ia.costab = ctx->costab.p;
-    ia.pad = ctx->pad;
     ia.padF = ctx->padF;
     ia.c = ctx->cgrid;
     ia.r_max = ctx->r_max;
-    float *gd = ctx->bp_data.p + 2 * gn * iclass, *gw = ctx->bp_weight.p + gn * iclass;
+    ia.bp_data = ctx->bp_data.p + 2 * gn * iclass;
+    ia.bp_weight = ctx->bp_weight.p + gn * iclass;
     BpArgs ba{};
-    HIPCHK(ctx->bi_val.reserve((size_t)chunk * Pf));
-    HIPCHK(ctx->bi_wgt.reserve((size_t)chunk * Pf));
-    HIPCHK(ctx->bi_task.reserve(2 * (size_t)chunk));
-    HIPCHK(ctx->bi_one.reserve(chunk));
-    ba.K = 1;
-    ba.Pf = Pf;
-    ba.NOR = 1;
-    ba.R = chunk;  // slice = image: its "rotation" is its own index
-    ba.whole_bricks = 1;
-    ba.pad = ctx->pad;
-    ba.padF = ctx->padF;
-    ba.c = ctx->cgrid;
-    ba.r_max = ctx->r_max;
-    ba.grid_stride = gn;
-    ia.val = ctx->bi_val.p;
-    ia.wgt = ctx->bi_wgt.p;
-    ia.task_img = ctx->bi_task.p;
-    ia.task_m = ctx->bi_task.p + chunk;
-    ia.slice_w = ctx->bi_one.p;
-    ba.task_img = ia.task_img;
-    ba.task_m = ia.task_m;
-    ba.f_xy = ctx->f_xy.p;
-    ba.MC2bp = ctx->bi_wgt.p;
-    ba.slice_w = ctx->bi_one.p;
-    ba.slice_val = ctx->bi_val.p;
-    ba.bp_data = gd;
-    ba.bp_weight = gw;
-    BandPlan plan{};
     if (ctx->is3d) {
+        HIPCHK(ctx->bi_val.reserve((size_t)chunk * Pf));
+        HIPCHK(ctx->bi_wgt.reserve((size_t)chunk * Pf));
+        HIPCHK(ctx->bi_task.reserve(2 * (size_t)chunk));
+        HIPCHK(ctx->bi_one.reserve(chunk));
         HIPCHK(ctx->bi_rec.reserve((size_t)chunk * Pf));
+        ia.val = ctx->bi_val.p;
+        ia.wgt = ctx->bi_wgt.p;
+        ia.task_img = ctx->bi_task.p;
+        ia.task_m = ctx->bi_task.p + chunk;
+        ia.slice_w = ctx->bi_one.p;
+        ba.K = 1;
+        ba.Pf = Pf;
+        ba.NOR = 1;
+        ba.R = chunk;  // slice = image: its "rotation" is its own index
+        ba.whole_bricks = 1;
+        ba.pad = ctx->pad;
+        ba.padF = ctx->padF;
+        ba.c = ctx->cgrid;
+        ba.r_max = ctx->r_max;
+        ba.grid_stride = gn;
+        ba.task_img = ia.task_img;
+        ba.task_m = ia.task_m;
+        ba.f_xy = ctx->f_xy.p;
+        ba.MC2bp = ctx->bi_wgt.p;
+        ba.slice_w = ctx->bi_one.p;
+        ba.slice_val = ctx->bi_val.p;
+        ba.bp_data = ia.bp_data;
+        ba.bp_weight = ia.bp_weight;
         ba.nbx = (ctx->padF + kBrickX - 1) / kBrickX;
         ba.nby = (ctx->pad + kBrickY - 1) / kBrickY;
         ba.nbz = (ctx->pad + kBrickZ - 1) / kBrickZ;
@@ -3522,9 +3521,6 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
         ba.ck_brick = ctx->bp_ck.p;
         ba.sums = ctx->bp_sums.p;
         ba.rec = ctx->bi_rec.p;
-    } else {  // one slot: a grid point is one running FP32 sum, as in 3D
-        plan = bp_band_plan(1, ctx->pad, ctx->padF, ctx->n_cu);
-        plan.slots = 1;
     }
     for (int i0 = 0; i0 < n; i0 += chunk) {
         const int m = std::min(chunk, n - i0);
@@ -3550,9 +3546,12 @@ int rome_backproject_images(rome_ctx* ctx, int iclass, int n, const double* fre,
         ia.Ai = ba.Ai_fine = dm;
         ia.sx = dm + 6 * (size_t)m;
         ia.sy = dm + 7 * (size_t)m;
-        HIPCHK(launch_bp_image_values(s, m, ia));
-        if (ctx->is3d) HIPCHK(launch_backproject_binned(s, m, ba));
-        else HIPCHK(launch_backproject_bands(s, m, ba, plan, nullptr));
+        if (ctx->is3d) {
+            HIPCHK(launch_bp_image_values(s, m, ia));
+            HIPCHK(launch_backproject_binned(s, m, ba));
+        } else {
+            HIPCHK(launch_bp_images_2d(s, m, ia));
+        }
         HIPCHK(hipStreamSynchronize(s));  // the staging buffers are reused by the next chunk
     }
     return ROME_OK;

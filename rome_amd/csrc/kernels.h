@@ -292,7 +292,7 @@ struct BpArgs {
     const float* MC2bp;           // [n][Pf]
     const double* slice_w;        // [S] sum of the slice's normalised significant weights (0: none)
     const float2* slice_val;      // [S][Pf]
-    const unsigned* slice_cnt = nullptr;  // [K] bands: slices with weight of every class; null: one class, one slot
+    const unsigned* slice_cnt = nullptr;  // [K] bands: slices with weight of every class
     unsigned* count;              // [nb]
     unsigned* off;                // [nb + 1]
     unsigned* coff;               // [nb + 1] chunks of the brick kernel per brick, prefix sums
@@ -514,7 +514,7 @@ struct MetaArgs {
 };
 hipError_t launch_meta(hipStream_t s, const MetaArgs& a);
 // Whole images at their own poses into one class grid (the offline reconstruction): the pixel values and
-// weights as slices for the binned scatter (3D), or scattered (2D).
+// weights as slices for the binned scatter (3D), or scattered (2D: data and weight grids).
 struct BpImageArgs {
     const double *fre, *fim;  // [n][F2] transforms (current_size half-plane)
     const double* ctf;        // [n][F2], or null: ones
@@ -524,13 +524,16 @@ struct BpImageArgs {
     const int* f_nfine;
     const int* f_xy;
     const double *sintab, *costab;
-    int pad, padF, c, r_max;
+    int padF, c, r_max;
     float2* val;              // [n][Pf] shifted transform times the CTF
     float* wgt;               // [n][Pf] CTF^2
-    int *task_img, *task_m;   // [n] 0, 1, ..: every image its own slice (binned scatter, bands)
+    int *task_img, *task_m;   // [n] 0, 1, ..: every image its own slice (binned scatter)
     double* slice_w;          // [n] 1
+    float* bp_data;           // 2D: the class's grid [pad][padF], interleaved
+    float* bp_weight;
 };
 hipError_t launch_bp_image_values(hipStream_t s, int n, const BpImageArgs& a);
+hipError_t launch_bp_images_2d(hipStream_t s, int n, const BpImageArgs& a);
 hipError_t launch_store_sums(hipStream_t s, const StoreArgs& a);
 // With a.ntask_dev (device-driven pools) S is read on the device and persist_blocks blocks stride over
 // the slices (one pixel block per grid row) and over the brick chunks.

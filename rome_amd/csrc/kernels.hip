@@ -1460,8 +1460,10 @@ __global__ void k_meta(MetaArgs a) {
 // MyBackProjector::backproject of images at their own poses (apps/rome_reconstruct.cpp:104-330): the transform
 // (current_size half-plane) shifted by the image's tabulated phase, times the CTF, and the weight CTF^2; the
 // pixel set is the fine one (x = 0 column for y >= 0 only, as the reference's first_x rule), radius r_max.
-// These values are the slices of the binned (3D) or banded (2D) scatter (backproject.hip), one slice per image; a direct
-// scatter's 24 float atomics a pixel took 1.82 ms for 400 images of 100^2, this pass and the binned one 0.2.
+// 3D: these values are the slices of the binned scatter (backproject.hip), one slice per image; a direct scatter's 24
+// float atomics a pixel took 1.82 ms for 400 images of 100^2, this pass and the binned one 0.2.  2D: scattered
+// right here, a grid point being one running FP32 sum as in 3D (the bands would need all images of a grid point in
+// one block: 20000 images of 32^2 50 ms with their uploads, 15.5 scattered; 10000 of 64^2 48 and 25).
 DEV void bp_image_value(const BpImageArgs& a, int img, int p, float2& v, float& w) {
     const size_t nf = (size_t)img * a.F2 + a.f_nfine[p];
     const float cv = a.ctf ? (float)a.ctf[nf] : 1.f;
@@ -1483,6 +1485,29 @@ __global__ __launch_bounds__(256) void k_bp_image_values(BpImageArgs a) {
     bp_image_value(a, img, p, v, w);
     a.val[(size_t)img * a.Pf + p] = v;
     a.wgt[(size_t)img * a.Pf + p] = w;
+}
+
+__global__ __launch_bounds__(256) void k_bp_images_2d(BpImageArgs a) {
+    const int img = blockIdx.y, p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= a.Pf) return;
+    const int xy = a.f_xy[p];
+    const int x = px_x(xy), y = px_y(xy);
+    if (x * x + y * y > a.r_max * a.r_max) return;
+    float2 v;
+    float w;
+    bp_image_value(a, img, p, v, w);
+    if (!(w > 0.f)) return;
+    const Coords c = map_coords(a.Ai + 6 * (size_t)img, x, y, a.c, false);
+    if (c.neg) v.y = -v.y;
+    const float mfx = 1.f - c.fx, mfy = 1.f - c.fy;
+    const float dd[4] = {mfy * mfx, mfy * c.fx, c.fy * mfx, c.fy * c.fx};
+#pragma unroll
+    for (int cc = 0; cc < 4; ++cc) {
+        const size_t idx = (size_t)(c.y0 + (cc >> 1)) * a.padF + c.x0 + (cc & 1);
+        atomicAdd(&a.bp_data[2 * idx], dd[cc] * v.x);
+        atomicAdd(&a.bp_data[2 * idx + 1], dd[cc] * v.y);
+        atomicAdd(&a.bp_weight[idx], dd[cc] * w);
+    }
 }
 
 // ------------------------------------------------------------------ launch wrappers
@@ -1906,6 +1931,14 @@ hipError_t launch_store_sums(hipStream_t s, const StoreArgs& a) {
 hipError_t launch_bp_image_values(hipStream_t s, int n, const BpImageArgs& a) {
     if (n <= 0) return hipSuccess;
     k_bp_image_values<<<dim3((a.Pf + 255) / 256, n), 256, 0, s>>>(a);
+    LAUNCH_CHECK();
+    return hipSuccess;
+}
+
+hipError_t launch_bp_images_2d(hipStream_t s, int n, const BpImageArgs& a) {
+    if (n <= 0) return hipSuccess;
+    if (n > 65535) return hipErrorInvalidValue;
+    k_bp_images_2d<<<dim3((a.Pf + 255) / 256, n), 256, 0, s>>>(a);
     LAUNCH_CHECK();
     return hipSuccess;
 }
