@@ -376,6 +376,7 @@ struct rome_ctx {
     DevBuf<float2> slice_val;
     DevBuf<float> bp_work;       // partial bands of 2D grids
     DevBuf<unsigned> slice_cnt;  // slices of every 2D class
+    bool bands = true;           // 2D: false once the slice buffer could not be had (until rome_configure)
     DevBuf<double> slice_w;
     DevBuf<unsigned> bp_count, bp_off, bp_coff, bp_cursor, bp_ck, bp_sums;
     DevBuf<unsigned long long> bp_rec;
@@ -484,8 +485,12 @@ struct rome_ctx {
         const long long by_mem = (long long)(kPfineBytes / ((size_t)NORf * Pf * sizeof(float2)));
         return (int)std::max<long long>(1, std::min<long long>({(long long)Mtot, (long long)n * sig_cap, by_mem}));
     }
-    // slices of the binned / banded backprojection a device-driven pool can hold.  2D classes have few samples
-    // an image: 32 tasks each, or 512 MB, and the direct scatter for more
+    // slices of the banded backprojection of a host-synchronised 2D pool: 32 tasks an image, or 4 GB
+    long long host_slice_cap(int n) const {
+        return std::max<long long>(((long long)4 << 30) / (8 * Pf), (long long)n * 32 * NORf);
+    }
+    // slices of the binned / banded backprojection a device-driven pool can hold (reserved whatever it needs).  2D classes
+    // have few samples an image: 32 tasks each, or 512 MB, whichever is more, and the direct scatter past that
     long long dd_slice_cap(int n) const {
         if (!is3d)
             return std::min((long long)n * sig_cap * NORf,
@@ -1581,18 +1586,28 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
         const long long slice_cap = ctx->dd_slice_cap(n);
         const bool by_slice = post_slices_supported(NOR, NOT, ctx->Pf, ctx->is3d);
         if (dd) S = by_slice || !ctx->is3d ? slice_cap : 0;
-        const bool binned = S > 0 && (!ctx->is3d || (unsigned long long)S * ctx->Pf < (1ULL << 32)) &&
-                            (size_t)S * ctx->Pf * 16 <= rome_ctx::kBinnedBytes;
+        // 2D, whose direct scatter needs no buffer: a bounded one, and none where the memory cannot be had
+        bool binned = S > 0 && (ctx->is3d ? (unsigned long long)S * ctx->Pf < (1ULL << 32)
+                                          : ctx->bands && (dd || S <= ctx->host_slice_cap(n))) &&
+                      (size_t)S * ctx->Pf * 16 <= rome_ctx::kBinnedBytes;
+        pp.slice_val = nullptr;
+        pp.slice_w = nullptr;
+        if (binned) {
+            hipError_t e = sized(ctx->slice_val, (size_t)S * ctx->Pf);
+            if (e == hipSuccess) e = sized(ctx->slice_w, (size_t)S);
+            if (e == hipErrorOutOfMemory && !ctx->is3d) {
+                (void)hipGetLastError();
+                binned = ctx->bands = false;
+            } else {
+                HIPCHK(e);
+            }
+        }
         if (dd) {
             pp.ntask_dev = ctx->task_off.p + n;
             pp.abort = ctx->pool_flags.p;
             pp.slice_cap = binned ? slice_cap : -1;  // -1: the direct scatter takes every pool
         }
-        pp.slice_val = nullptr;
-        pp.slice_w = nullptr;
         if (binned) {
-            HIPCHK(sized(ctx->slice_val, (size_t)S * ctx->Pf));
-            HIPCHK(sized(ctx->slice_w, (size_t)S));
             pp.slice_val = ctx->slice_val.p;
             pp.slice_w = ctx->slice_w.p;
             if (!ctx->is3d) {
@@ -2106,6 +2121,7 @@ int rome_configure(rome_ctx* ctx, const rome_config* cfg) {
     HIPCHK(ctx->wsum_scalars.reserve(4));
     ctx->have_ref.assign(ctx->K, 0);
     ctx->configured = true;
+    ctx->bands = true;
     ctx->have_sampling = ctx->have_model = false;
     ctx->fct_dirty = true;
     HIPCHK(hipStreamSynchronize(s));
