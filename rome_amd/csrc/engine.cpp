@@ -605,12 +605,12 @@ int upload_poses(rome_ctx* ctx) {
 
 int build_phase_tables(rome_ctx* ctx) {
     const rome_config& c = ctx->cfg;
-    HIPCHK(ctx->Sc.reserve((size_t)ctx->T * ctx->Pc));
+    // of the coarse operands: by pixel in the FP32 arm, by shift in the mixed ones
+    const bool by_pixel = c.precision == ROME_PREC_FP32;
+    DevBuf<float2>& coarse = by_pixel ? ctx->ScT : ctx->Sc;
+    HIPCHK(coarse.reserve((size_t)ctx->T * ctx->Pc));
     HIPCHK(launch_phase_table(ctx->stream, ctx->d_sxc.p, ctx->d_syc.p, ctx->T, ctx->c_xy.p, ctx->Pc, c.ori_size,
-                              ctx->sintab.p, ctx->costab.p, ctx->Sc.p));
-    HIPCHK(ctx->ScT.reserve((size_t)ctx->T * ctx->Pc));
-    HIPCHK(launch_phase_table(ctx->stream, ctx->d_sxc.p, ctx->d_syc.p, ctx->T, ctx->c_xy.p, ctx->Pc, c.ori_size,
-                              ctx->sintab.p, ctx->costab.p, ctx->ScT.p, true));
+                              ctx->sintab.p, ctx->costab.p, coarse.p, by_pixel));
     const int nsf = ctx->T * ctx->NOTf;
     HIPCHK(ctx->Sf.reserve((size_t)nsf * ctx->Pf));
     const double* sx = ctx->two_pass ? ctx->d_sxf.p : ctx->d_sxc.p;
