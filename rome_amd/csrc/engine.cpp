@@ -403,6 +403,7 @@ struct rome_ctx {
     DevBuf<double2> rc_data, rc_Fc, rc_Ft;
     DevBuf<double> rc_weight, rc_Fw, rc_Fnw, rc_M, rc_Mout, rc_vol, rc_tab, rc_sums, rc_tau2;
     DevBuf<int> rc_bad;
+    DevBuf<double> rc_mid;            // between the halves of the gridding iterations' transforms (large 2D)
     DevBuf<double> dft_cos, dft_sin;  // of the gridding iterations, for dft_P points
     int dft_P = 0;
     std::vector<double> rc_tab_h;
@@ -2941,6 +2942,10 @@ int rome_reconstruct(rome_ctx* ctx, int iclass, const rome_recon_params* prm, co
     ga.Fnw = ctx->rc_Fnw.p;
     ga.T0 = ctx->rc_Fc.p;
     ga.T1 = ctx->rc_Ft.p;
+    if (const size_t mid = gridding_mid_len(PF, ctx->is3d, sym)) {
+        HIPCHK(ctx->rc_mid.reserve(mid));
+        ga.mid = ctx->rc_mid.p;
+    }
     ga.tab = ctx->rc_tab.p;
     ga.ntab = 10000;
     ga.npad = ori * pf;

@@ -85,12 +85,14 @@ DEV int below_root(int m) {
 }
 
 // z lines of one (y, 16 x) tile.  BACK: G(+-z) from T, the weight update; FWD: the transform of
-// Fnewweight * Fweight into out.  First iteration: FWD only; last: BACK only.
-template <int TPW, bool BACK, bool FWD, bool SYM>
-__global__ __launch_bounds__(max_threads(TPW)) void k_grid_z(GriddingArgs a, const double2* __restrict__ T,
-                                                             double2* __restrict__ out) {
+// Fnewweight * Fweight into out.  First iteration: FWD only; last: BACK only.  SPLIT: a block is one wave, blockIdx.z
+// its row tile, and what the two halves hand over goes through a.mid instead of LDS, in a launch each.
+template <int TPW, bool BACK, bool FWD, bool SYM, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 64 : max_threads(TPW)) void k_grid_z(GriddingArgs a, const double2* __restrict__ T,
+                                                                          double2* __restrict__ out) {
+    static_assert(!SPLIT || BACK != FWD, "one half a launch");
     extern __shared__ double lds[];  // [2][nt * 256]: e, o of the next transform
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, W = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, wave = SPLIT ? blockIdx.z : threadIdx.x >> 6, W = SPLIT ? gridDim.z : blockDim.x >> 6;
     const int kr = lane >> 4, x = blockIdx.x * 16 + (lane & 15), iy = blockIdx.y;
     const int y = iy < a.H ? iy : iy - a.P;
     const int zlim = below_root(a.max_r2 - y * y - (int)(blockIdx.x * 16) * (int)(blockIdx.x * 16));
@@ -101,8 +103,8 @@ __global__ __launch_bounds__(max_threads(TPW)) void k_grid_z(GriddingArgs a, con
     const size_t zs = (size_t)a.Py * a.H;  // real arrays [z][y][H]
     const size_t xy = (size_t)iy * a.H + min(x, a.H - 1);
     const size_t ts = (size_t)a.Py * a.ldx, tx = (size_t)iy * a.ldx + x;  // T [z'][y][ldx]
-    double* le = lds;
-    double* lo = lds + a.nt * 256;
+    double* le = SPLIT ? a.mid + (size_t)blockIdx.x * a.nt * 512 : lds;
+    double* lo = le + a.nt * 256;
     if constexpr (BACK) {
         d4 ce[TPW], so[TPW], ci[TPW], sr[TPW];
 #pragma unroll
@@ -168,7 +170,7 @@ __global__ __launch_bounds__(max_threads(TPW)) void k_grid_z(GriddingArgs a, con
                     e = fp + fm;
                     o = fp - fm;
                 }
-                if constexpr (FWD) {
+                if constexpr (FWD || SPLIT) {
                     le[t * 256 + r * 64 + lane] = e;
                     lo[t * 256 + r * 64 + lane] = o;
                 }
@@ -184,7 +186,7 @@ __global__ __launch_bounds__(max_threads(TPW)) void k_grid_z(GriddingArgs a, con
             constexpr int NQ = decltype(n)::value;
             for (int k0 = 0; k0 < 4 * ntz; k0 += kU) {
                 double e[kU], o[kU];
-                if constexpr (BACK) {
+                if constexpr (BACK || SPLIT) {
 #pragma unroll
                     for (int u = 0; u < kU; ++u) {
                         e[u] = le[(k0 + u) * 64 + lane];
@@ -295,12 +297,14 @@ DEV double blob_at(const GriddingArgs& a, int r2) {
     return idx < a.ntab ? a.tab[idx] / a.tab0 : 0.;
 }
 
-// 16 x lines (y', z' >= 0; lines in memory order): forward to M, times the blob, back.
-template <int TPW, bool SYM>
-__global__ __launch_bounds__(max_threads(TPW)) void k_grid_x(GriddingArgs a, const double2* __restrict__ in,
-                                                             double2* __restrict__ out) {
-    extern __shared__ double lds[];  // SYM: [2][nt * 256]; else [4][nt * 256]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, W = blockDim.x >> 6;
+// 16 x lines (y', z' >= 0; lines in memory order): forward to M, times the blob, back.  PART 1, 2: one of the halves, a
+// block being one wave, blockIdx.y its row tile, and what they hand over in a.mid; 0: both, through LDS.
+template <int TPW, bool SYM, int PART>
+__global__ __launch_bounds__(PART ? 64 : max_threads(TPW)) void k_grid_x(GriddingArgs a, const double2* __restrict__ in,
+                                                                         double2* __restrict__ out) {
+    extern __shared__ double dyn[];  // SYM: [2][nt * 256]; else [4][nt * 256]
+    double* lds = PART ? a.mid + (size_t)blockIdx.x * (SYM ? 2 : 4) * a.nt * 256 : dyn;
+    const int lane = threadIdx.x & 63, wave = PART ? blockIdx.y : threadIdx.x >> 6, W = PART ? gridDim.y : blockDim.x >> 6;
     const int line = blockIdx.x * 16 + (lane & 15);
     const bool yin = line < a.H * a.Py;
     const int kr = lane >> 4, iz = (yin ? line : 0) / a.Py, iy = (yin ? line : 0) - iz * a.Py;
@@ -308,7 +312,7 @@ __global__ __launch_bounds__(max_threads(TPW)) void k_grid_x(GriddingArgs a, con
     const size_t row = (size_t)(yin ? line : 0) * a.ldx;
     const int n1 = a.nt * 256;
     const int ntx = (a.xlim >> 4) + 1;  // 16-column groups with a point inside the ball
-    {
+    if constexpr (PART != 2) {
         d4 tc[TPW], ts[TPW];
 #pragma unroll
         for (int q = 0; q < TPW; ++q) tc[q] = ts[q] = d4{0., 0., 0., 0.};
@@ -360,7 +364,8 @@ __global__ __launch_bounds__(max_threads(TPW)) void k_grid_x(GriddingArgs a, con
             }
         }
     }
-    __syncthreads();
+    if constexpr (PART == 1) return;
+    if constexpr (PART == 0) __syncthreads();
     d4 g[SYM ? 2 : 4][TPW];
 #pragma unroll
     for (int p = 0; p < (SYM ? 2 : 4); ++p)
@@ -414,45 +419,72 @@ __global__ __launch_bounds__(max_threads(TPW)) void k_grid_x(GriddingArgs a, con
 template <int TPW>
 static hipError_t iterate(hipStream_t s, const GriddingArgs& a, bool sym, int iters) {
     const int W = (a.nt + TPW - 1) / TPW, xt = (a.xlim >> 4) + 1, nth = 64 * W;
-    const dim3 gz(xt, a.Py), gx((a.H * a.Py + 15) / 16), gyf((xt * a.H + 3) / 4, W);
-    const int nzb = sym ? a.H : a.P;
-    const dim3 gyb((xt * nzb + 3) / 4, W);
+    const dim3 gz(xt, a.Py), gx((a.H * a.Py + 15) / 16);
     const size_t l1 = (size_t)a.nt * 256 * sizeof(double);
     // above 64 KB a launch needs the kernel's leave (without SYM from H = 129 on)
     if (!sym && 4 * l1 > 65536) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_grid_x<TPW, false>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_grid_x<TPW, false, 0>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)(4 * l1));
         if (e != hipSuccess) return e;
     }
-    k_grid_z<TPW, false, true, true><<<gz, nth, 0, s>>>(a, nullptr, a.T0);
+    k_grid_z<TPW, false, true, true, false><<<gz, nth, 0, s>>>(a, nullptr, a.T0);
     double2 *p = a.T0, *q = a.T1;
     for (int it = 0; it < iters; ++it) {
-        if (a.Py > 1) {
-            k_grid_y<TPW, false><<<gyf, 256, 0, s>>>(a, a.H, p, q);
+        const int nzb = sym ? a.H : a.P;
+        if constexpr (TPW > 1) {  // (2D has no y)
+            k_grid_y<TPW, false><<<dim3((xt * a.H + 3) / 4, W), 256, 0, s>>>(a, a.H, p, q);
             std::swap(p, q);
         }
-        if (sym) k_grid_x<TPW, true><<<gx, nth, 2 * l1, s>>>(a, p, q);
-        else k_grid_x<TPW, false><<<gx, nth, 4 * l1, s>>>(a, p, q);
+        if (sym) k_grid_x<TPW, true, 0><<<gx, nth, 2 * l1, s>>>(a, p, q);
+        else k_grid_x<TPW, false, 0><<<gx, nth, 4 * l1, s>>>(a, p, q);
         std::swap(p, q);
-        if (a.Py > 1) {
-            k_grid_y<TPW, true><<<gyb, 256, 0, s>>>(a, nzb, p, q);
+        if constexpr (TPW > 1) {
+            k_grid_y<TPW, true><<<dim3((xt * nzb + 3) / 4, W), 256, 0, s>>>(a, nzb, p, q);
             std::swap(p, q);
         }
         const bool last = it + 1 == iters;
-        if (sym && last) k_grid_z<TPW, true, false, true><<<gz, nth, 0, s>>>(a, p, q);
-        else if (sym) k_grid_z<TPW, true, true, true><<<gz, nth, 2 * l1, s>>>(a, p, q);
-        else if (last) k_grid_z<TPW, true, false, false><<<gz, nth, 0, s>>>(a, p, q);
-        else k_grid_z<TPW, true, true, false><<<gz, nth, 2 * l1, s>>>(a, p, q);
+        if (sym && last) k_grid_z<TPW, true, false, true, false><<<gz, nth, 0, s>>>(a, p, q);
+        else if (sym) k_grid_z<TPW, true, true, true, false><<<gz, nth, 2 * l1, s>>>(a, p, q);
+        else if (last) k_grid_z<TPW, true, false, false, false><<<gz, nth, 0, s>>>(a, p, q);
+        else k_grid_z<TPW, true, true, false, false><<<gz, nth, 2 * l1, s>>>(a, p, q);
         std::swap(p, q);
     }
     return hipGetLastError();
+}
+
+// 2D, large: every half transform a launch of one-wave blocks, a 16 x 16 tile each
+template <bool SYM>
+static hipError_t iterate_split(hipStream_t s, const GriddingArgs& a, int iters) {
+    const int xt = (a.xlim >> 4) + 1;
+    const unsigned nl = (unsigned)(a.H + 15) / 16;
+    k_grid_z<1, false, true, true, false><<<dim3(xt, 1), 64 * a.nt, 0, s>>>(a, nullptr, a.T0);
+    for (int it = 0; it < iters; ++it) {
+        k_grid_x<1, SYM, 1><<<dim3(nl, a.nt), 64, 0, s>>>(a, a.T0, a.T1);
+        k_grid_x<1, SYM, 2><<<dim3(nl, xt), 64, 0, s>>>(a, a.T0, a.T1);
+        k_grid_z<1, true, false, SYM, true><<<dim3(xt, 1, a.nt), 64, 0, s>>>(a, a.T1, a.T0);
+        if (it + 1 < iters) k_grid_z<1, false, true, SYM, true><<<dim3(xt, 1, a.nt), 64, 0, s>>>(a, a.T1, a.T0);
+    }
+    return hipGetLastError();
+}
+
+// 2D, from 7 row tiles on, or 5 without SYM: a block's matrix cores are the bound then, and a tile of 16 columns is one
+// block.  Ten iterations of a class, whole against split: H = 88 0.385 and 0.396 ms, 98 0.394 and 0.378, 172 0.730
+// and 0.534; without SYM H = 68 0.469 and 0.472, 74 0.465 and 0.453, 172 0.981 and 0.682.
+static bool gridding_split(int nt, bool is3d, bool sym) { return !is3d && nt >= (sym ? 7 : 5); }
+
+size_t gridding_mid_len(int H, bool is3d, bool sym) {
+    const int nt = (H + 15) / 16;
+    return gridding_split(nt, is3d, sym) ? (size_t)nt * nt * 1024 : 0;
 }
 
 hipError_t gridding_iterations(hipStream_t s, const GriddingArgs& a, bool sym, int iters) {
     if (iters <= 0) return hipSuccess;
     if (a.nt < 1 || a.nt > kMaxTiles || a.nk != 4 * a.nt || a.ldx < 16 * a.nt || a.xlim < 0 || a.xlim >= a.H || a.P != 2 * a.H - 1 || (a.Py != 1 && a.Py != a.P))
         return hipErrorInvalidValue;
-    return a.Py > 1 ? iterate<3>(s, a, sym, iters) : iterate<1>(s, a, sym, iters);
+    if (a.Py > 1) return iterate<3>(s, a, sym, iters);
+    if (!gridding_split(a.nt, false, sym)) return iterate<1>(s, a, sym, iters);
+    if (!a.mid) return hipErrorInvalidValue;
+    return sym ? iterate_split<true>(s, a, iters) : iterate_split<false>(s, a, iters);
 }
 
 }  // namespace rome

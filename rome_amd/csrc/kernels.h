@@ -565,10 +565,12 @@ struct GriddingArgs {
     const double* Fw;
     double* Fnw;
     double2 *T0, *T1;
+    double* mid;                // [gridding_mid_len], null if that is 0
     const double* tab;          // blob transform, ntab samples `sampling` apart in units of 1 / npad
     int ntab, npad;
     double sampling, tab0, size;
 };
+size_t gridding_mid_len(int H, bool is3d, bool sym);
 hipError_t gridding_iterations(hipStream_t s, const GriddingArgs& a, bool sym, int iters);
 hipError_t rc_final_fconv(hipStream_t s, const double2* data, const double* Fnw, double2* Fc, int Dz, int P, int PF,
                           int max_r2);
