@@ -739,6 +739,20 @@ int readback(rome_ctx* ctx, const std::vector<Seg>& segs) {
     return r ? r : readback_end(ctx, segs, L);
 }
 
+// Results to a caller's arrays: up to 1 MB packed into one copy (a copy each costs 10-20 us: nine of one image of 32^2
+// 0.25 ms a call, 0.13 now), else through the ring.  On the host when it returns.
+int copy_out(rome_ctx* ctx, const std::vector<CopyOut::Part>& parts) {
+    size_t total = 0;
+    for (const auto& p : parts) total += p.dst ? p.bytes : 0;
+    if (total > ((size_t)1 << 20)) {
+        HIPCHK(ctx->copy_out.run(ctx->stream, parts));
+        return ROME_OK;
+    }
+    std::vector<Seg> segs;
+    for (const auto& p : parts) segs.push_back({p.src, p.dst, p.bytes});
+    return readback(ctx, segs);
+}
+
 WeightParams weight_params(rome_ctx* ctx) {
     WeightParams wp;
     wp.K = ctx->K;
@@ -2767,10 +2781,11 @@ int rome_fourier_map(rome_ctx* ctx, int iclass, const double* vol, int do_griddi
     HIPCHK(launch_fm_window(s, ctx->fm_F.p, padori, dim3, pf, ctx->r_max, ctx->pad, oriF, normfft,
                             grid_out ? ctx->fm_grid64.p : nullptr, g32, ctx->fm_pw.p, ctx->fm_cnt.p));
     std::vector<double> pw(oriF), cnt(oriF);
-    HIPCHK(hipMemcpyAsync(pw.data(), ctx->fm_pw.p, oriF * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(cnt.data(), ctx->fm_cnt.p, oriF * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIPCHK(ctx->copy_out.run(s, {{corrected_map, ctx->fm_corr.p, nvol * sizeof(double)},
-                                 {grid_out, ctx->fm_grid64.p, ctx->grid_n * sizeof(double2)}}));
+    rc = copy_out(ctx, {{pw.data(), ctx->fm_pw.p, oriF * sizeof(double)},
+                        {cnt.data(), ctx->fm_cnt.p, oriF * sizeof(double)},
+                        {corrected_map, ctx->fm_corr.p, nvol * sizeof(double)},
+                        {grid_out, ctx->fm_grid64.p, ctx->grid_n * sizeof(double2)}});
+    if (rc) return rc;
     if (power_spectrum)  // radial average (src/reconstruct.cpp:213-221)
         for (int i = 0; i < oriF; ++i) power_spectrum[i] = cnt[i] < 1. ? 0. : pw[i] / cnt[i];
     ctx->have_ref[iclass] = 1;
@@ -3099,11 +3114,12 @@ int rome_prepare_images(rome_ctx* ctx, const rome_raw_images* in, const rome_pre
             auto part = [&](double* dst, const double* src, size_t per) {
                 return CopyOut::Part{dst ? dst + (size_t)i0 * per : nullptr, src, n * per * sizeof(double)};
             };
-            HIPCHK(ctx->copy_out.run(s, {part(ho->fmask_re, a.fmask_re, cF), part(ho->fmask_im, a.fmask_im, cF),
-                                         part(ho->fnomask_re, a.fnomask_re, cF), part(ho->fnomask_im, a.fnomask_im, cF),
-                                         part(ho->fctf, a.fctf, cF), part(ho->power_img, a.power, oriF),
-                                         part(ho->highres_Xi2, a.hxi2, 1), part(ho->old_offx, a.old_offx, 1),
-                                         part(ho->old_offy, a.old_offy, 1)}));
+            rc = copy_out(ctx, {part(ho->fmask_re, a.fmask_re, cF), part(ho->fmask_im, a.fmask_im, cF),
+                                part(ho->fnomask_re, a.fnomask_re, cF), part(ho->fnomask_im, a.fnomask_im, cF),
+                                part(ho->fctf, a.fctf, cF), part(ho->power_img, a.power, oriF),
+                                part(ho->highres_Xi2, a.hxi2, 1), part(ho->old_offx, a.old_offx, 1),
+                                part(ho->old_offy, a.old_offy, 1)});
+            if (rc) return rc;
         }
         HIPCHK(hipStreamSynchronize(s));  // the staging buffers are reused by the next chunk
     }
@@ -3324,8 +3340,7 @@ int rome_proposal_get_params(rome_ctx* ctx, rome_proposal_params* o) {
             parts.push_back({dst[q], P.w[q].p, (size_t)P.rows[l] * P.cols[l] * sizeof(float)});
         }
     }
-    HIPCHK(ctx->copy_out.run(ctx->stream, parts));
-    return ROME_OK;
+    return copy_out(ctx, parts);
 }
 
 int rome_proposal_set_params(rome_ctx* ctx, const rome_proposal_params* in) {
