@@ -472,7 +472,8 @@ def main():
         if learned:
             pstats = eng.proposal_stats()
             eng.proposal_mode("off")
-        return dict(value=args.steps * B / dt, dt=dt, prof=prof, stats={**eng.batch_stats(), **eng.coarse_stats()},
+        return dict(value=args.steps * B / dt, dt=dt, prof=prof, stats={**eng.batch_stats(), **eng.coarse_stats(),
+                                                                    "cross": eng.cross_term()},
                     amax=amax, meta=meta, truth_agree=float(np.mean(agree)), full_batches=full_batches,
                     proposal=pstats, execution={"mode": args.execution, "last_per_step": execs,
                                                 "step_ms": [round(x, 2) for x in step_ms],
@@ -522,17 +523,16 @@ def main():
     peak = MFMA_PEAK_TFLOPS[head_prec]
     # coarse list output (the product path) in every timed batch, rather than the full pose term
     listed = stats.get("mode") == 0 and rl["full_batches"] == 0
-    # psi and psi + 180 deg share one half-table row in the mixed arm when the in-plane sampling pairs them
-    # (an even count of psi steps per half turn, the half table a multiple of 128 rows, >= 8 shifts)
-    paired = head_prec != "fp32" and prob["nr_psi"] % 8 == 0 and (M // 2) % 128 == 0 and T >= 8
-    # pools of at least four blocks a CU hold the columns in LDS (96 a block, the half table in bands of 2.5 MB)
-    cols = paired and listed and B * T // 96 * 4 >= 4 * 256
+    # the kernel the library took: psi and psi + 180 deg share one half-table row where the in-plane sampling pairs
+    # them, and large pools hold the columns in LDS
+    cross = stats["cross"]
+    paired, cols = cross["kernel"].startswith("paired"), cross["columns"] // 32
     lowp = "k_gemm_pq_cols<%s>" if cols else ("k_gemm_lowp_pq<%s, " + ("list>" if listed else "E>")) if paired else \
         ("k_gemm_lowp_list<%s>" if listed else "k_gemm_lowp<%s>")
     kname = "k_coarse_gemm (coarse cross term, FP32 MFMA)" if head_prec == "fp32" else \
         (lowp % head_prec) + " (coarse cross term, %s MFMA%s)" % (head_prec.upper(),
                                                                   ", psi/psi+180 paired" if paired else "")
-    row = "k_gemm_pq_cols<_Float16, 3>" if cols else \
+    row = "k_gemm_pq_cols<_Float16, %d>" % cols if cols else \
         ("k_gemm_lowp_pq<_Float16, true>" if paired else "k_gemm_lowp_list<_Float16>")
     traffic = measured_traffic(row) if head_prec == "fp16" and listed else None
     roofline = {"kernel": kname, "bound": "mfma",

@@ -323,6 +323,9 @@ int rome_set_coarse_mode(rome_ctx* ctx, int mode, int list_cap);
 /* Last pool: out3 = {0 list / 1 full / 2 list overflowed and the pool ran full, largest list,
  * total list entries}. */
 int rome_get_coarse_stats(rome_ctx* ctx, long long* out3);
+/* Last pool: out2 = {kernel of the coarse cross term: 0 FP32, 1 BF16 / FP16 by rotations, 2 by pairs of rotations in
+ * tiles, 3 by pairs with the columns resident in LDS; the columns a block then holds, else 0}. */
+int rome_get_cross_term(rome_ctx* ctx, int* out2);
 
 /* Form of the coarse significance the fine pass is built from (no counterpart in the reference, whose
  * Exp_Mweight stores it per sample): by default the keys of each image's significant samples, up to

@@ -32,6 +32,7 @@ EXPORTED = (
     "rome_proposal_forward", "rome_proposal_gradients", "rome_proposal_training_rows", "rome_backproject_images",
     "rome_project_device_noalloc", "rome_set_execution", "rome_get_execution_stats", "rome_expectation_fine_device",
     "rome_autotune", "rome_set_persistent_grids", "rome_proposal_set_thresholds", "rome_set_class_range",
+    "rome_get_cross_term",
 )
 
 EXEC_HOST, EXEC_DEVICE, EXEC_GRAPH = 0, 1, 2
@@ -557,6 +558,12 @@ class Engine:
         out = np.zeros(3, np.int64)
         self._check(lib().rome_get_coarse_stats(self._h, _p(out, C.c_longlong)), "rome_get_coarse_stats")
         return dict(zip(("mode", "list_max", "list_total"), out.tolist()))
+
+    def cross_term(self):
+        """Kernel of the last pool's coarse cross term and the columns its blocks hold in LDS (0: none)."""
+        out = np.zeros(2, np.int32)
+        self._check(lib().rome_get_cross_term(self._h, _p(out, C.c_int)), "rome_get_cross_term")
+        return {"kernel": ("fp32", "rotations", "paired", "paired_columns")[out[0]], "columns": int(out[1])}
 
     def set_class_range(self, iclass_min=-1, iclass_max=-1):
         """Classes the next pools run (the seeding iteration's single class per pool); (-1, -1): all."""

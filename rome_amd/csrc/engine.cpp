@@ -2621,6 +2621,23 @@ int rome_get_coarse_stats(rome_ctx* ctx, long long* out) {
     return ROME_OK;
 }
 
+int rome_get_cross_term(rome_ctx* ctx, int* out) {
+    if (!ctx || !out) return ROME_ERR_ARG;
+    if (!ctx->configured || ctx->last_n == 0) return fail(ctx, ROME_ERR_ARG, "no E-step has run");
+    out[0] = out[1] = 0;
+    if (ctx->cfg.precision == ROME_PREC_FP32) return ROME_OK;
+    out[0] = ctx->pq ? 2 : 1;
+    if (!ctx->pq || ctx->last_coarse_full != 0) return ROME_OK;
+    LowpGemmArgs la{};
+    la.K16 = ctx->K16();
+    la.T = ctx->T;
+    la.Ncols = ctx->last_n * ctx->T;
+    la.Mh = ctx->Mtot / 2;
+    out[1] = pq_resident_columns(la, ctx->n_cu);
+    if (out[1]) out[0] = 3;
+    return ROME_OK;
+}
+
 int rome_get_batch_stats(rome_ctx* ctx, long long* out) {
     if (!ctx || !out) return ROME_ERR_ARG;
     out[0] = ctx->last_n;

@@ -1006,6 +1006,8 @@ hipError_t launch_fct_to_lowp(hipStream_t s, int precision, const float* FcT, in
     return hipGetLastError();
 }
 
+int pq_resident_columns(const LowpGemmArgs& a, int n_cu) { return 32 * pq_cols_tj(a, n_cu); }
+
 size_t pq_fragments_len(int Mh, int K16) { return (size_t)Mh * 2 * pq_half(K16); }
 
 hipError_t launch_pq_fragments(hipStream_t s, const void* A16, int Mh, int K16, void* Af) {

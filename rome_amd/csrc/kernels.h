@@ -597,6 +597,7 @@ hipError_t launch_fct_to_lowp(hipStream_t s, int precision, const float* FcT, in
 hipError_t launch_recompute_split(hipStream_t s, int precision, int n, const RecomputeArgs& a);
 hipError_t launch_prep_lowp(hipStream_t s, int precision, int n, const PrepLowpArgs& a);
 hipError_t launch_gemm_lowp(hipStream_t s, int precision, const LowpGemmArgs& a, int n_cu);
+int pq_resident_columns(const LowpGemmArgs& a, int n_cu);  // a block's, 0: the list output's tiled kernel
 size_t pq_fragments_len(int Mh, int K16);  // values of that table
 hipError_t launch_pq_fragments(hipStream_t s, const void* A16, int Mh, int K16, void* Af);
 
