@@ -1136,6 +1136,10 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
     int U = 0;
     std::vector<int> cstatus(n), lcount, scount(n);
     bool sig_dense = false;
+    // the most samples of an image in the present block lists, where the host knows it
+    auto most_blocks = [&]() -> long long {
+        return dd || given || sig_dense ? -1 : *std::max_element(scount.begin(), scount.end());
+    };
     std::vector<Seg> extra_rb;  // further device arrays read back with the significance results
     // weights and significance -> fine-pass task counts and the rotations they need; returns after
     // one host synchronisation.  Sparse: per-image keys of the significant samples; dense: the mask
@@ -1158,7 +1162,8 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
         stage_begin(ctx, 3);
         if (from_d2c)
             HIPCHK(launch_weights_fine(s, n, wp_exact, ctx->D2c.p, ctx->blk_task.p, ctx->blk_t.p, ctx->task_m.p,
-                                       ctx->blk_off.p, 1, wc_exact, cand, TailArgs{ctx->c_tail.p, ctx->c_dmin1.p}, sg));
+                                       ctx->blk_off.p, 1, wc_exact, cand, TailArgs{ctx->c_tail.p, ctx->c_dmin1.p}, sg,
+                                       most_blocks()));
         else if (L)
             HIPCHK(launch_weights_list(s, n, wp, *L, ctx->C2c.p, ctx->emin_key.p, wc, sg, cand, ctx->list_scan(),
                                        ctx->n_cu));
@@ -1528,7 +1533,7 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
     stage_end(ctx, 6);
     stage_begin(ctx, 7);
     HIPCHK(launch_weights_fine(s, n, wp, ctx->D2.p, ctx->blk_task.p, ctx->blk_t.p, ctx->task_m.p, ctx->blk_off.p, NE, wf,
-                               cand, tail));
+                               cand, tail, {nullptr, 1, nullptr, nullptr, 0}, most_blocks()));
     stage_end(ctx, 7);
     if (!given && P.ready && P.mode == ROME_PROPOSAL_COLLECT && ctx->two_pass && ctx->is3d && P.K == ctx->K && P.D == ctx->D &&
         P.PSI == ctx->PSI && P.cur == c.current_size) {

@@ -437,10 +437,12 @@ hipError_t launch_weights_list(hipStream_t s, int n, const WeightParams& wp, con
 // reach[img] = kWeightWindow + (max - min of ln pdf_offset over (class, translation)) + slack,
 // +inf when a pdf_offset is zero; clears the images' histograms of the list scan
 hipError_t launch_list_reach(hipStream_t s, int n, const WeightParams& wp, float* reach, const ListScanArgs& scan);
+// most: the most blocks of an image where the host knows it (else -1)
 hipError_t launch_weights_fine(hipStream_t s, int n, const WeightParams& wp, const double* D2, const int* blk_task,
                                const int* blk_t, const int* task_m, const long long* img_blk, int NE,
                                const WeightOutArgs& wo, const CandArgs& cand, TailArgs tail = TailArgs{nullptr, nullptr},
-                               SigArgs sig = SigArgs{nullptr, 1, nullptr, nullptr, 0});
+                               SigArgs sig = SigArgs{nullptr, 1, nullptr, nullptr, 0},
+                               long long most = -1);
 // Task lists of the fine pass from the significant samples: per image the number of tasks
 // (rotations with any significant translation) and blocks (significant samples), their exclusive
 // scans (task_off, blk_off [n + 1]), used[m] = 1 for every rotation some image needs (zero before)

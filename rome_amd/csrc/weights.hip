@@ -822,7 +822,8 @@ hipError_t launch_list_reach(hipStream_t s, int n, const WeightParams& wp, float
 
 hipError_t launch_weights_fine(hipStream_t s, int n, const WeightParams& wp, const double* D2, const int* blk_task,
                                const int* blk_t, const int* task_m, const long long* img_blk, int NE,
-                               const WeightOutArgs& wo, const CandArgs& c, TailArgs tail, SigArgs sig) {
+                               const WeightOutArgs& wo, const CandArgs& c, TailArgs tail, SigArgs sig,
+                               long long most) {
     int log2NE = 0;
     while ((1 << log2NE) < NE) ++log2NE;
     if ((1 << log2NE) != NE) return hipErrorInvalidValue;
@@ -831,7 +832,7 @@ hipError_t launch_weights_fine(hipStream_t s, int n, const WeightParams& wp, con
     WeightOut o{wo.dmin, wo.sumw, wo.maxw, wo.amax, wo.thr, wo.nsig, wo.status, wo.tail};
     const Cand cd{c.w, c.du, c.e, c.cap};
     k_weights_fine<false><<<n, 256, off_bytes(wp), s>>>(wp, D2, blk_task, blk_t, task_m, img_blk, log2NE, o, cd, tail, sig);
-    if ((long long)wp.Mtot * wp.T * NE > kLongFine)
+    if ((most >= 0 ? most : (long long)wp.Mtot * wp.T) * NE > kLongFine)
         k_weights_fine<true><<<n, 1024, off_bytes(wp), s>>>(wp, D2, blk_task, blk_t, task_m, img_blk, log2NE, o, cd, tail, sig);
     return hipGetLastError();
 }
