@@ -1082,7 +1082,8 @@ int run_pool(rome_ctx* ctx, int n, rome_results* res, int pool_mode, PoolOut* do
     HIPCHK(ctx->At.reserve(given ? 1 : (size_t)n * ctx->Mpad));
     WeightParams wp = weight_params(ctx);
     stage_begin(ctx, 1);
-    if (!given) HIPCHK(launch_coarse_aterm(s, n, ctx->Qc.p, ctx->Kq, M, ctx->Mpad, ctx->MC2c.p, ldn, ctx->At.p));
+    if (!given) HIPCHK(launch_coarse_aterm(s, n, ctx->Qc.p, ctx->Kq, M, ctx->Mpad, ctx->MC2c.p, ldn, ctx->At.p,
+                                           ctx->n_cu));
     if (!given && ctx->coarse_mode == ROME_COARSE_LIST && ctx->two_pass) {
         HIPCHK(ctx->reach.reserve(n));
         HIPCHK(ctx->ls_hsum.reserve((size_t)n * kBinCount));

@@ -763,7 +763,9 @@ hipError_t go_pq_cols(hipStream_t s, const LowpGemmArgs& a) {
 // Columns of 32 a tile of k_gemm_pq_cols holds: three (96; four spill registers) where they fit in LDS beside its 13 KB,
 // else two.  0, the tiled kernel: tiles of more images than there are slots for, and fewer than four blocks a CU, whose
 // unequal rounds and fills cost what the loop gains (6912 half rows x 9657 columns x 320 k, 1.6 blocks a CU: 236 us both,
-// and longer lists; 9216 x 162000 x 512 k, 26 a CU: 3548 -> 2134 us).
+// and longer lists).  With 512 k, tiled and resident: 9216 half rows, 4.1 blocks a CU (310 images of 81 shifts) 577 and
+// 421 us, 7.9 1118 and 767, 26 3548 and 2134; 2304 half rows, 4.1 1456 and 1295, 5.9 1481 and 1522 (the lists' lengths
+// vary by more).
 int pq_cols_tj(const LowpGemmArgs& a, int n_cu) {
     for (int tj = 3; tj >= 2; --tj) {
         if (32 * tj * (2 * pq_half(a.K16) + 8) * 2 + (13 << 10) > (160 << 10)) continue;

@@ -394,7 +394,7 @@ hipError_t launch_prep_images(hipStream_t s, int n, const PrepArgs& a);
 hipError_t launch_fct_norm(hipStream_t s, const float* FcT, int Pc, int Pc_pad, int Mpad, int Kq, float* Qc);
 // At[img][m] = 0.5 * sum_p Qc[p][m] * MC2cT[p][img] (FP32 MFMA); Mpad and ldn multiples of 128
 hipError_t launch_coarse_aterm(hipStream_t s, int n, const float* Qc, int Kq, int Mtot, int Mpad, const float* MC2cT,
-                               int ldn, float* At);
+                               int ldn, float* At, int n_cu);
 hipError_t launch_coarse_gemm(hipStream_t s, const GemmArgs& a);
 struct CandArgs {  // per-image candidate list of the weight pass: [n][cap]
     double* w;

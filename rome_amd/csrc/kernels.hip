@@ -1683,11 +1683,11 @@ hipError_t launch_fct_norm(hipStream_t s, const float* FcT, int Pc, int Pc_pad, 
 }
 
 hipError_t launch_coarse_aterm(hipStream_t s, int n, const float* Qc, int Kq, int Mtot, int Mpad, const float* MC2cT,
-                               int ldn, float* At) {
+                               int ldn, float* At, int n_cu) {
     if (n <= 0) return hipSuccess;
     if (Kq % 16 || Mpad % 128 || ldn % 128 || ldn < n) return hipErrorInvalidValue;
     const dim3 grid(Mpad / 128, ldn / 128);
-    if (grid.x * grid.y < 256)
+    if ((int)(grid.x * grid.y) < n_cu)
         k_coarse_aterm_wave<<<dim3(Mpad / 32, (n + 31) / 32), 64, 0, s>>>(Qc, Kq, Mtot, Mpad, MC2cT, ldn, n, At);
     else
         k_coarse_aterm<<<grid, 256, 0, s>>>(Qc, Kq, Mtot, Mpad, MC2cT, ldn, n, At);

@@ -25,7 +25,7 @@
 // block: a broad posterior leaves hundreds of thousands of entries inside the window, each an FP64 exponential.
 // Measured: 333 images of 13824 rotations x 29 shifts, lists of 50 thousand entries on average and up to 302
 // thousand, one block an image with three exact passes 938 us, now 136 (scan) + 243; 2000 images of 18432 x 81,
-// 10 thousand on average, 547 us, now 132 + 192.
+// 9 thousand on average, 547 us, now 320 with the scan.
 #include <hip/hip_runtime.h>
 #include <limits.h>
 #include <stdint.h>
@@ -603,8 +603,10 @@ __global__ __launch_bounds__(1024) void k_weights_coarse(WeightParams wp, const 
 }
 
 // The scan of weight_pass (the same expressions and anchor) over part blockIdx.y of a list longer than
-// kSplitList, runs of 1024 entries dealt out round-robin.  8192: below it the image's own block is as fast.
-constexpr int kSplitList = 8192;
+// kSplitList, runs of 1024 entries dealt out round-robin.  The line by the whole pass: 2000 images, lists of 9 thousand on
+// average and 210 at most, 0.39, 0.37, 0.32, 0.31 ms with it at 4, 8, 16 and 32 thousand; 200 images of 2.5
+// thousand and 41 at most 0.042, 0.042, 0.044, 0.054.
+constexpr int kSplitList = 16384;
 __global__ __launch_bounds__(256) void k_list_scan(WeightParams wp, ListArgs L, const double* __restrict__ C2c,
                                                    const int* __restrict__ emin_key, ListScanArgs out) {
     __shared__ double hsum[kBinCount];
