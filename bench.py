@@ -546,7 +546,7 @@ def main():
     cpu = None
     parity = None
     if not args.no_cpu_baseline:
-        # the GPU box allots 16 host CPUs to its GPU, whatever nproc reports
+        # 16 host CPUs belong to a GPU, whatever nproc reports
         nproc = os.cpu_count() or 1
         threads = min(nproc, 16)
         ns = args.cpu_sample or 25 * threads

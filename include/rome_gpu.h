@@ -298,8 +298,8 @@ int rome_set_persistent_grids(rome_ctx* ctx, const int* blocks);
 /* Measurement: stage times from HIP events recorded on the engine stream around each kernel
  * group (no counterpart in the reference, whose timers are TIMEPOINT macros, src/time.h:61-75).
  * Stages: 0 prep, 1 coarse norms, 2 coarse cross term, 3 coarse weights, 4 task build,
- * 5 fine projections, 6 fine diff2, 7 fine weights, 8 sigma2/pdf sums and slices (2D: also the
- * backprojection), 9 store sums, 10 binned 3D backprojection, 11 split three-product recompute of the
+ * 5 fine projections, 6 fine diff2, 7 fine weights, 8 sigma2/pdf sums and slices (2D pools past the slice
+ * buffer: also the backprojection), 9 store sums, 10 binned (3D) or banded (2D) backprojection, 11 split three-product recompute of the
  * marked coarse samples (BF16 / FP16 arms; stage 3 then also holds the second weight pass).
  * rome_set_profiling(1) resets the accumulators; rome_get_profile returns the stage count. */
 int rome_set_profiling(rome_ctx* ctx, int on);

@@ -77,7 +77,7 @@ DEV bool bp_sample(const BpArgs& a, long long s, int p, Sample& out) {
     return true;
 }
 
-// brick of the base voxel: class-major, then z, y, x in bricks of 8 (grid coordinates are >= 0)
+// brick of the base voxel: class-major, then z, y, x in bricks of 4, 8 and 16 (grid coordinates are >= 0)
 DEV int brick_of(const BpArgs& a, const Sample& sm) {
     const int bx = sm.c.x0 / kBrickX, by = sm.c.y0 / kBrickY, bz = sm.c.z0 / kBrickZ;
     return sm.k * a.nb_class + (bz * a.nby + by) * a.nbx + bx;

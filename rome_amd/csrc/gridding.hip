@@ -20,7 +20,7 @@
 // from blob(n) on the planes |n| = h unless the table has ended there (it has when current_size = ori_size).
 // SYM = false keeps every z' on the way back and the imaginary part of G: twice the y and z work back.
 //
-// Bound: FP64 MFMA (78.6 TFLOP/s).  Only lines and rows inside the ball r^2 < max_r2 are computed before
+// Bound: FP64 MFMA (66 TFLOP/s in a large product on this card).  Only lines and rows inside the ball r^2 < max_r2 are computed before
 // the first and after the last axis.  A block is one tile of 16 columns; its waves own up to 3 row tiles
 // each, 12 independent accumulators, operands straight from L2 (a k step is 768 matrix cycles for 5 KB).
 #include <hip/hip_runtime.h>
@@ -37,7 +37,7 @@ namespace {
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 constexpr int kU = 4;          // k steps whose operands are loaded together: 16 rows
-constexpr int kMaxTiles = 15;  // row tiles: H <= 240
+constexpr int kMaxTiles = 15;  // row tiles: H <= 240; H = current_size + 2, of at most 202 (rome_configure)
 // Row tiles of 16 per wave: 3 for the many columns of a 3D grid (the fewest operand loads that leave two
 // waves per SIMD); 1 in 2D, where a whole pass is a handful of blocks and its time one wave's chain.
 constexpr int max_threads(int TPW) { return TPW == 1 ? 64 * kMaxTiles : 64 * ((kMaxTiles + TPW - 1) / TPW); }

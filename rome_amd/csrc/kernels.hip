@@ -1363,8 +1363,9 @@ DEV void post_slice_one(const PostArgs& a, long long w, int h) {
 // first jcap = gridDim.x / 8 items of each range.  TAIL = true (device-driven only): a fixed grid strides over
 // the items j >= jcap of each range (usually none: the first launch is sized from the pools before).  A counter per
 // range to take them from costs 53 ns an item (451 k items of 100 images of 192^2: 4.0 ms, 1.4 strided; 1.0
-// without a tail).  Two kernels rather than one with both paths: the loop raises the slice body's register count.  A pool whose slices exceed the slice buffer
-// (slice_cap) goes to the direct scatter instead, and an aborted pool adds nothing.
+// without a tail).  Two kernels rather than one with both paths: the loop raises the slice body's register
+// count.  A pool whose slices exceed the slice buffer (slice_cap) goes to the direct scatter instead, and an aborted
+// pool adds nothing.
 template <int NOR, int NOT, int PPT, int NT, bool TAIL>
 __global__ __launch_bounds__(NT) void k_post_slice(PostArgs a, long long ntask, long long jcap) {
     if (a.ntask_dev) {
