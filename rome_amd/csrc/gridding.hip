@@ -48,12 +48,12 @@ DEV d4 mfma64(double a, double b, d4 c) { return __builtin_amdgcn_mfma_f64_16x16
 // first matrix instruction (masked loads became a round trip each: y 90 us instead of 73, x 184 instead of 150).  The tables are zero past
 // row and column H, a row index is clamped to one of the same column, and cos has 1/2 in column 0, where
 // p(k) + p(-k) counts p(0) twice.
-template <int NQ>
+template <int NQ, int U = kU>
 struct MatOps {
-    double c[kU][NQ], s[kU][NQ];
+    double c[U][NQ], s[U][NQ];
     DEV void load(const GriddingArgs& a, int k0, int wave, int W, int lane) {
 #pragma unroll
-        for (int u = 0; u < kU; ++u)
+        for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int q = 0; q < NQ; ++q) {
                 const size_t o = ((size_t)(wave + q * W) * a.nk + k0 + u) * 64 + lane;
@@ -73,6 +73,15 @@ DEV void for_tiles(int wave, int W, int tiles, F&& body) {
     if (TPW > 2 && wave + 2 * W < tiles) body(Num<TPW>());
     else if (TPW > 1 && wave + W < tiles) body(Num<(TPW < 2 ? TPW : 2)>());
     else if (wave < tiles) body(Num<1>());
+}
+
+// body(Num<n>, k0) over k steps 0 .. n - 1 (a multiple of 4), n at a time: 4, or WIDE 8 and the rest
+template <bool WIDE, typename F>
+DEV void for_steps(int n, F&& body) {
+    int k0 = 0;
+    if constexpr (WIDE)
+        for (; k0 + 2 * kU <= n; k0 += 2 * kU) body(Num<2 * kU>(), k0);
+    for (; k0 < n; k0 += kU) body(Num<kU>(), k0);
 }
 
 // largest k with k^2 < m (m > 0), -1 otherwise
@@ -111,18 +120,19 @@ __global__ __launch_bounds__(SPLIT ? 64 : max_threads(TPW)) void k_grid_z(Griddi
         for (int q = 0; q < TPW; ++q) ce[q] = so[q] = ci[q] = sr[q] = d4{0., 0., 0., 0.};
         for_tiles<TPW>(wave, W, ntz, [&](auto n) {
             constexpr int NQ = decltype(n)::value;
-            for (int k0 = 0; k0 < a.nk; k0 += kU) {
-                double2 p[kU], m[kU];
+            for_steps<SPLIT>(a.nk, [&](auto steps, int k0) {
+                constexpr int U = decltype(steps)::value;
+                double2 p[U], m[U];
 #pragma unroll
-                for (int u = 0; u < kU; ++u) {
+                for (int u = 0; u < U; ++u) {
                     const int z = min(4 * (k0 + u) + kr, a.H - 1);
                     p[u] = T[(size_t)z * ts + tx];
                     if constexpr (!SYM) m[u] = T[(size_t)(z ? a.P - z : 0) * ts + tx];
                 }
-                MatOps<NQ> A;
+                MatOps<NQ, U> A;
                 A.load(a, k0, wave, W, lane);
 #pragma unroll
-                for (int u = 0; u < kU; ++u) {
+                for (int u = 0; u < U; ++u) {
                     double er, oi, ei = 0., orr = 0.;
                     if constexpr (SYM) {
                         er = 2. * p[u].x;
@@ -143,7 +153,7 @@ __global__ __launch_bounds__(SPLIT ? 64 : max_threads(TPW)) void k_grid_z(Griddi
                         }
                     }
                 }
-            }
+            });
         });
 #pragma unroll
         for (int q = 0; q < TPW; ++q) {
@@ -184,17 +194,18 @@ __global__ __launch_bounds__(SPLIT ? 64 : max_threads(TPW)) void k_grid_z(Griddi
         for (int q = 0; q < TPW; ++q) ar[q] = ai[q] = d4{0., 0., 0., 0.};
         for_tiles<TPW>(wave, W, a.nt, [&](auto n) {
             constexpr int NQ = decltype(n)::value;
-            for (int k0 = 0; k0 < 4 * ntz; k0 += kU) {
-                double e[kU], o[kU];
+            for_steps<SPLIT>(4 * ntz, [&](auto steps, int k0) {
+                constexpr int U = decltype(steps)::value;
+                double e[U], o[U];
                 if constexpr (BACK || SPLIT) {
 #pragma unroll
-                    for (int u = 0; u < kU; ++u) {
+                    for (int u = 0; u < U; ++u) {
                         e[u] = le[(k0 + u) * 64 + lane];
                         o[u] = lo[(k0 + u) * 64 + lane];
                     }
                 } else {
 #pragma unroll
-                    for (int u = 0; u < kU; ++u) {
+                    for (int u = 0; u < U; ++u) {
                         const int z = min(4 * (k0 + u) + kr, a.H - 1);
                         const size_t ip = (size_t)z * zs + xy, im = (size_t)(z ? a.P - z : 0) * zs + xy;
                         const double fp = a.Fnw[ip] * a.Fw[ip], fm = a.Fnw[im] * a.Fw[im];
@@ -203,16 +214,16 @@ __global__ __launch_bounds__(SPLIT ? 64 : max_threads(TPW)) void k_grid_z(Griddi
                         o[u] = in * (fp - fm);
                     }
                 }
-                MatOps<NQ> A;
+                MatOps<NQ, U> A;
                 A.load(a, k0, wave, W, lane);
 #pragma unroll
-                for (int u = 0; u < kU; ++u)
+                for (int u = 0; u < U; ++u)
 #pragma unroll
                     for (int q = 0; q < NQ; ++q) {
                         ar[q] = mfma64(A.c[u][q], e[u], ar[q]);
                         ai[q] = mfma64(A.s[u][q], o[u], ai[q]);
                     }
-            }
+            });
         });
 #pragma unroll
         for (int q = 0; q < TPW; ++q) {
@@ -318,20 +329,21 @@ __global__ __launch_bounds__(PART ? 64 : max_threads(TPW)) void k_grid_x(Griddin
         for (int q = 0; q < TPW; ++q) tc[q] = ts[q] = d4{0., 0., 0., 0.};
         for_tiles<TPW>(wave, W, a.nt, [&](auto n) {
             constexpr int NQ = decltype(n)::value;
-            for (int k0 = 0; k0 < 4 * ntx; k0 += kU) {  // columns past the ball are zero
-                double2 b[kU];
+            for_steps<PART != 0>(4 * ntx, [&](auto steps, int k0) {
+                constexpr int U = decltype(steps)::value;  // columns past the ball are zero
+                double2 b[U];
 #pragma unroll
-                for (int u = 0; u < kU; ++u) b[u] = in[row + 4 * (k0 + u) + kr];
-                MatOps<NQ> A;
+                for (int u = 0; u < U; ++u) b[u] = in[row + 4 * (k0 + u) + kr];
+                MatOps<NQ, U> A;
                 A.load(a, k0, wave, W, lane);
 #pragma unroll
-                for (int u = 0; u < kU; ++u)
+                for (int u = 0; u < U; ++u)
 #pragma unroll
                     for (int q = 0; q < NQ; ++q) {
                         tc[q] = mfma64(A.c[u][q], 2. * b[u].x, tc[q]);
                         ts[q] = mfma64(A.s[u][q], 2. * b[u].y, ts[q]);
                     }
-            }
+            });
         });
         // M(+-x') = tc -+ ts; reference radii of +n and -n differ at n = h only
         const int yp = abs(y) + (y == h), ym = abs(y) + (y == -h);
@@ -373,16 +385,17 @@ __global__ __launch_bounds__(PART ? 64 : max_threads(TPW)) void k_grid_x(Griddin
         for (int q = 0; q < TPW; ++q) g[p][q] = d4{0., 0., 0., 0.};
     for_tiles<TPW>(wave, W, ntx, [&](auto n) {
         constexpr int NQ = decltype(n)::value;
-        for (int k0 = 0; k0 < a.nk; k0 += kU) {
-            double b[kU][SYM ? 2 : 4];
+        for_steps<PART != 0>(a.nk, [&](auto steps, int k0) {
+            constexpr int U = decltype(steps)::value;
+            double b[U][SYM ? 2 : 4];
 #pragma unroll
-            for (int u = 0; u < kU; ++u)
+            for (int u = 0; u < U; ++u)
 #pragma unroll
                 for (int p = 0; p < (SYM ? 2 : 4); ++p) b[u][p] = lds[p * n1 + (k0 + u) * 64 + lane];
-            MatOps<NQ> A;
+            MatOps<NQ, U> A;
             A.load(a, k0, wave, W, lane);
 #pragma unroll
-            for (int u = 0; u < kU; ++u)
+            for (int u = 0; u < U; ++u)
 #pragma unroll
                 for (int q = 0; q < NQ; ++q) {
                     g[0][q] = mfma64(A.c[u][q], b[u][0], g[0][q]);
@@ -392,7 +405,7 @@ __global__ __launch_bounds__(PART ? 64 : max_threads(TPW)) void k_grid_x(Griddin
                         g[3][q] = mfma64(A.s[u][q], b[u][3], g[3][q]);
                     }
                 }
-        }
+        });
     });
     if (!yin) return;
     // the line (-y', -z'): another z' > 0 never writes it; at z' = 0 the y' tiles cover every line
@@ -468,8 +481,9 @@ static hipError_t iterate_split(hipStream_t s, const GriddingArgs& a, int iters)
 }
 
 // 2D, from 7 row tiles on, or 5 without SYM: a block's matrix cores are the bound then, and a tile of 16 columns is one
-// block.  Ten iterations of a class, whole against split: H = 88 0.385 and 0.396 ms, 98 0.394 and 0.378, 172 0.730
-// and 0.534; without SYM H = 68 0.469 and 0.472, 74 0.465 and 0.453, 172 0.981 and 0.682.
+// block.  Ten iterations of a class, whole against split: H = 88 0.385 and 0.396 ms, 98 0.394 and 0.359, 172 0.730
+// and 0.489; without SYM H = 68 0.469 and 0.472, 74 0.465 and 0.444, 172 0.981 and 0.651.  One wave a SIMD hides no
+// load by itself, so these blocks take 8 k steps at a time (4: 172 0.534, without SYM 0.682).
 static bool gridding_split(int nt, bool is3d, bool sym) { return !is3d && nt >= (sym ? 7 : 5); }
 
 size_t gridding_mid_len(int H, bool is3d, bool sym) {
